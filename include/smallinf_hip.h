@@ -450,6 +450,63 @@ typedef struct sipa_kchan_write_params {
 
 int32_t sipa_kchan_write_rows(const sipa_kchan_write_params* p, void* stream);
 
+/*
+ * The decoder layer's operations around the paged attention (reference engine/model.py:101-175), bf16 in and out with
+ * fp32 arithmetic. Pointers are device pointers; strides are row strides in elements; the last dimension is contiguous.
+ *
+ * sipa_fused_linear: y = epilogue(norm(x) W^T), one launch, for few tokens (it streams W once per 64 tokens):
+ *   x [T, K], weight [N, K] contiguous, K a multiple of 64; norm_weight [K] or NULL: x is RMS-normalised first,
+ *   x * rsqrt(mean(x^2) + eps) * norm_weight (the row factor applied to the product's fp32 sums).
+ *   SIPA_LINEAR_RESIDUAL: out[t, n] = y + bias[n] + residual[t, n] (each may be NULL);             N % 16 == 0
+ *   SIPA_LINEAR_ROPE:     out = y + bias, then the rotary embedding of the first rot_channels channels (whole heads of
+ *                         head_dim): out[c] = y[c] cos[t, c] + y[c'] sin[t, c] with c' the channel head_dim / 2 away in
+ *                         its head; rot_cos, rot_sin [T, head_dim] contiguous, sin with rotate-half's sign folded in;
+ *                         N % 16 == 0, head_dim % 16 == 0
+ *   SIPA_LINEAR_SILU:     out[t, i] = silu(y[t, i]) * y[t, N / 2 + i];                              N % 16 == 0
+ * x, weight and norm_weight must be 16-byte aligned and x_stride a multiple of 8. out must not overlap the inputs,
+ * except that it may be the residual itself.
+ */
+enum { SIPA_LINEAR_RESIDUAL = 0, SIPA_LINEAR_ROPE = 1, SIPA_LINEAR_SILU = 2 };
+
+typedef struct sipa_linear_params {
+  int32_t struct_size; /* sizeof(sipa_linear_params) */
+  int32_t epilogue;    /* SIPA_LINEAR_* */
+  int32_t num_tokens, in_features, out_features, head_dim, rot_channels;
+  float eps;
+  const void* x;
+  int64_t x_stride;
+  const void* weight;
+  const void* norm_weight;
+  const void* bias;
+  const void* residual;
+  int64_t res_stride;
+  void* out;
+  int64_t out_stride;
+  const void* rot_cos;
+  const void* rot_sin;
+  int32_t num_splits; /* RESIDUAL without norm: workgroups that share a row tile's K (0 or 1: none) */
+  void* part;         /* num_splits > 1: fp32 [N / 16][ceil(T / 16) rounded up to 1, 2 or a multiple of 4][num_splits][256] */
+  void* counters;     /* num_splits > 1: int32 [N / 16][ceil(T / 64)], zero; left at zero */
+} sipa_linear_params;
+
+int32_t sipa_fused_linear(const sipa_linear_params* p, void* stream);
+
+/*
+ * RMSNorm of T rows of K <= 8192 channels (K % 8 == 0): out = bf16(bf16(s * rsqrt(mean(s^2) + eps)) * weight), with
+ * s = x, or s = bf16(x + add) stored to sum when add and sum are given (the residual). Rows 16-byte aligned.
+ */
+int32_t sipa_rms_norm(const void* x, int64_t x_stride, const void* add, int64_t add_stride, const void* weight,
+                      float eps, void* sum, int64_t sum_stride, void* out, int64_t out_stride, int32_t T, int32_t K,
+                      void* stream);
+
+/* Rotary embedding in place on the first H heads of rows x [T, >= H D] (D % 16 == 0), tables as above. */
+int32_t sipa_rope(void* x, int64_t x_stride, const void* cos, const void* sin, int32_t T, int32_t H, int32_t D,
+                  void* stream);
+
+/* out[t, i] = silu(gate_up[t, i]) * gate_up[t, I + i] for i < I (I % 8 == 0). */
+int32_t sipa_silu_mul(const void* gate_up, int64_t gu_stride, void* out, int64_t out_stride, int32_t T, int32_t I,
+                      void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -82,6 +82,17 @@ class KchanWriteParams(ctypes.Structure):
     ]
 
 
+class LinearParams(ctypes.Structure):
+    """Mirror of struct sipa_linear_params."""
+    _fields_ = [
+        ("struct_size", i32), ("epilogue", i32), ("num_tokens", i32), ("in_features", i32), ("out_features", i32),
+        ("head_dim", i32), ("rot_channels", i32), ("eps", f32),
+        ("x", vp), ("x_stride", i64), ("weight", vp), ("norm_weight", vp), ("bias", vp),
+        ("residual", vp), ("res_stride", i64), ("out", vp), ("out_stride", i64), ("rot_cos", vp), ("rot_sin", vp),
+        ("num_splits", i32), ("part", vp), ("counters", vp),
+    ]
+
+
 # name -> (restype, argtypes); every symbol the header declares
 SIGNATURES = {
     "sipa_abi_version": (i32, []),
@@ -112,6 +123,10 @@ SIGNATURES = {
     "sipa_store_tokens": (i32, [vp, vp, i32, i64, i64, i64, i64, vp, i32, i32, i32, vp, vp, vp, vp, i32, i64, i64,
                                 i64, vp]),
     "sipa_kchan_write_rows": (i32, [_c.POINTER(KchanWriteParams), vp]),
+    "sipa_fused_linear": (i32, [_c.POINTER(LinearParams), vp]),
+    "sipa_rms_norm": (i32, [vp, i64, vp, i64, vp, f32, vp, i64, vp, i64, i32, i32, vp]),
+    "sipa_rope": (i32, [vp, i64, vp, vp, i32, i32, i32, vp]),
+    "sipa_silu_mul": (i32, [vp, i64, vp, i64, i32, i32, vp]),
 }
 
 _lib = None

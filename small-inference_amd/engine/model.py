@@ -15,6 +15,7 @@ from dataclasses import dataclass
 import torch
 import torch.nn.functional as F
 
+from . import hip_layer
 from .config import ModelConfig
 
 
@@ -84,6 +85,10 @@ class Qwen2Model:
         """Decoder layer i on hidden states x [T, hidden]; K/V go through the cache."""
         cfg, w = self.cfg, self.layers[i]
         T, Hq, Hkv, d = x.shape[0], cfg.num_q_heads, cfg.num_kv_heads, cfg.head_dim
+        if hip_layer.supported(x, w, rot, Hq + 2 * Hkv, d):
+            qkv = hip_layer.layer_qkv(x, w, cfg.rms_norm_eps, rot, Hq + Hkv, d).view(T, Hq + 2 * Hkv, d)
+            cache.write(i, qkv[:, Hq:Hq + Hkv], qkv[:, Hq + Hkv:])
+            return hip_layer.layer_out(x, cache.attend(i, qkv[:, :Hq], positions, self.scale), w, cfg.rms_norm_eps)
         qkv = F.linear(rms_norm(x, w.input_norm, cfg.rms_norm_eps), w.qkv_w, w.qkv_b)
         qk = rotate(qkv[:, :cfg.q_size + cfg.kv_size].view(T, Hq + Hkv, d), *rot)
         q, k = qk[:, :Hq], qk[:, Hq:]
@@ -102,6 +107,8 @@ class Qwen2Model:
         rot = self.rotary.rows(positions, x.dtype)
         for i in range(self.cfg.num_layers):
             x = self.layer_forward(i, x, positions, cache, rot)
-        if last_only:
+        if last_only and meta.num_tokens != meta.num_seqs:  # one token a sequence: every row is a last one
             x = x[meta.last_token_indices]
+        if hip_layer.rows_ok(x, self.final_norm):
+            return F.linear(hip_layer.rms_norm(x, self.final_norm, self.cfg.rms_norm_eps), self.lm_head)
         return F.linear(rms_norm(x, self.final_norm, self.cfg.rms_norm_eps), self.lm_head)

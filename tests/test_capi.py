@@ -300,3 +300,27 @@ def test_kchan_write_rows_checks_arguments():
     assert lib.sipa_kchan_write_rows(ctypes.byref(params(x_dtype=99)), None) == _hip.EUNSUPPORTED
     assert lib.sipa_kchan_write_rows(ctypes.byref(params(stage=None)), None) == _hip.EINVAL
     assert lib.sipa_kchan_write_rows(ctypes.byref(params(H=0)), None) == _hip.EINVAL
+
+
+def bad_linear(**over):
+    p = _hip.LinearParams()
+    p.struct_size = ctypes.sizeof(_hip.LinearParams)
+    p.num_tokens, p.in_features, p.out_features, p.head_dim = 4, 896, 1152, 64
+    for ptr in ("x", "weight", "out", "rot_cos", "rot_sin"):
+        setattr(p, ptr, 4096)
+    p.x_stride, p.out_stride = 896, 1152
+    for k, v in over.items():
+        setattr(p, k, v)
+    return p
+
+
+@pytest.mark.parametrize("over,code", [
+    (dict(struct_size=8), _hip.EINVAL), (dict(in_features=100), _hip.EUNSUPPORTED), (dict(x=None), _hip.EINVAL),
+    (dict(x=4098), _hip.EUNSUPPORTED), (dict(x_stride=897), _hip.EUNSUPPORTED), (dict(out_features=1144), _hip.EUNSUPPORTED),
+    (dict(epilogue=3), _hip.EINVAL), (dict(epilogue=1, head_dim=24), _hip.EUNSUPPORTED),
+    (dict(epilogue=1, rot_channels=96), _hip.EINVAL), (dict(epilogue=1, rot_channels=64, rot_cos=None), _hip.EINVAL),
+    (dict(epilogue=2, bias=4096), _hip.EINVAL), (dict(num_splits=2), _hip.EWORKSPACE),
+    (dict(num_splits=2, part=4096, counters=4096, epilogue=2), _hip.EINVAL), (dict(num_tokens=-1), _hip.EINVAL)])
+def test_fused_linear_refuses_bad_arguments(over, code):
+    assert _hip.lib().sipa_fused_linear(ctypes.byref(bad_linear(**over)), None) == code
+    assert _hip.lib().sipa_last_error()

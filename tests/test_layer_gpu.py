@@ -1,0 +1,151 @@
+"""The decoder layer's fused operations (csrc/layer.hip through engine/hip_layer.py) against the same operations in
+fp64, and a layer on the kernels against the same layer on torch operations.
+
+Bound, for results of N(0, 1) inputs: the output's own bf16 rounding is at most 2^-9 of each value (2^-9 / sqrt(3) =
+1.1e-3 in the 2-norm at worst); a normalised operand x * w rounded to bf16 adds a relative error of the same size to
+every term of a product, independent from term to term, so again at most 1.1e-3 in the 2-norm, and the gated product
+of SwiGLU carries it twice. Together under 2^-8 = 3.9e-3.
+"""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from cases import fragmented_manager
+from engine import hip_layer
+from engine.config import ModelConfig
+from engine.model import Qwen2Model, rms_norm, rotate
+from engine.paged_cache import PagedKVCache, build_metadata
+
+pytestmark = pytest.mark.gpu
+
+BOUND = 2.0 ** -8
+EPS = 1e-6
+TOKENS = [1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 130]
+
+
+def rel(a, b):
+    return ((a.double() - b).norm() / b.norm()).item()
+
+
+def randn(g, *shape):
+    return torch.randn(*shape, generator=g, device="cuda", dtype=torch.bfloat16)
+
+
+def norm64(x, w):
+    x = x.double()
+    return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + EPS) * w.double()
+
+
+def rotate64(x, cos, sin):
+    h = x.shape[-1] // 2
+    return x * cos.double() + torch.cat([x[..., h:], x[..., :h]], -1) * sin.double()
+
+
+# (hidden, heads, rotated heads, head_dim): the two model shapes, one slice of K, more slices than waves take at once
+SHAPES = [(896, 18, 16, 64), (1536, 16, 14, 128), (64, 3, 2, 16), (4096, 2, 1, 32)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("T", TOKENS)
+def test_projection_with_norm_and_rotary(T, shape):
+    hidden, heads, rotated, d = shape
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x, nw, w, b = randn(g, T, hidden), 1 + 0.1 * randn(g, hidden), randn(g, heads * d, hidden) * 0.05, randn(g, heads * d)
+    rot = randn(g, T, 1, d), randn(g, T, 1, d)
+    print(f"case rotary T {T} {shape}", flush=True)
+    out = hip_layer.fused_linear(x, w, hip_layer.ROPE, norm_weight=nw, eps=EPS, bias=b, rot=rot, head_dim=d,
+                                 rot_channels=rotated * d)
+    y = (norm64(x, nw) @ w.double().t() + b.double()).view(T, heads, d)
+    ref = torch.cat([rotate64(y[:, :rotated], *rot), y[:, rotated:]], 1).view(T, -1)
+    assert rel(out, ref) < BOUND
+
+
+@pytest.mark.parametrize("inter,hidden", [(4864, 896), (8960, 1536), (8, 64)])
+@pytest.mark.parametrize("T", TOKENS)
+def test_gated_projection(T, inter, hidden):
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x, nw, w = randn(g, T, hidden), 1 + 0.1 * randn(g, hidden), randn(g, 2 * inter, hidden) * 0.05
+    print(f"case gated T {T} {inter} x {hidden}", flush=True)
+    out = hip_layer.fused_linear(x, w, hip_layer.SILU, norm_weight=nw, eps=EPS)
+    y = norm64(x, nw) @ w.double().t()
+    assert rel(out, F.silu(y[:, :inter]) * y[:, inter:]) < BOUND
+
+
+@pytest.mark.parametrize("out_f,in_f", [(896, 4864), (1536, 8960), (896, 896), (16, 64), (48, 320)])
+@pytest.mark.parametrize("splits", [1, 2, 4, 7])
+@pytest.mark.parametrize("T", [1, 16, 17, 33, 64, 65])
+def test_projection_with_residual(T, splits, out_f, in_f):
+    """Split K too: more splits than slices of K among them; a second call finds the counters at zero."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x, w, res = randn(g, T, in_f), randn(g, out_f, in_f) * 0.05, randn(g, T, out_f)
+    print(f"case residual T {T} splits {splits} {out_f} x {in_f}", flush=True)
+    ref = x.double() @ w.double().t() + res.double()
+    first = hip_layer.fused_linear(x, w, hip_layer.RESIDUAL, residual=res, num_splits=splits)
+    again = hip_layer.fused_linear(x, w, hip_layer.RESIDUAL, residual=res, num_splits=splits)
+    assert rel(first, ref) < BOUND
+    assert torch.equal(first, again)
+
+
+@pytest.mark.parametrize("K", [8, 896, 1024, 1032, 1536, 2056, 8192])
+@pytest.mark.parametrize("T", [1, 4, 5, 300])
+def test_rms_norm_rows(T, K):
+    """The kernel rounds where the torch operations do: equal but for the order of the sum of squares (a row factor one
+    fp32 step off flips few roundings), the residual sum bit for bit."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x, add, w = randn(g, T, K), randn(g, T, K), 1 + 0.1 * randn(g, K)
+    out, s = hip_layer.rms_norm(x, w, EPS, add=add)
+    assert torch.equal(s, x + add)
+    ref = rms_norm(x + add, w, EPS)
+    assert (out != ref).float().mean() < 0.01 and rel(out, ref.double()) < 2 ** -9
+    assert torch.equal(hip_layer.rms_norm(s, w, EPS), out)
+
+
+@pytest.mark.parametrize("T,heads,extra,d", [(1, 1, 0, 16), (7, 16, 2, 64), (300, 14, 2, 128)])
+def test_rope_and_silu_rows(T, heads, extra, d):
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = randn(g, T, (heads + extra) * d)
+    rot = randn(g, T, 1, d), randn(g, T, 1, d)
+    y = x.clone()
+    hip_layer.rope_(y, rot, heads, d)
+    ref = rotate64(x.view(T, -1, d)[:, :heads].double(), *rot).reshape(T, -1)
+    assert rel(y[:, :heads * d], ref) < 2 ** -9
+    assert torch.equal(y[:, heads * d:], x[:, heads * d:])
+    gu = randn(g, T, 2 * heads * d)
+    half = heads * d
+    assert rel(hip_layer.silu_mul(gu), F.silu(gu[:, :half].double()) * gu[:, half:].double()) < 2 ** -9
+
+
+@pytest.mark.parametrize("T", [1, 16, 33, 130])
+def test_layer_on_kernels_matches_torch_operations(T):
+    """layer_forward under inference_mode (the kernels) against the same call outside it (the torch operations), and
+    what the layer wrote into the cache."""
+    cfg = ModelConfig(vocab_size=64, hidden_size=896, intermediate_size=4864, num_layers=1, num_q_heads=14,
+                      num_kv_heads=2, head_dim=64)
+    model = Qwen2Model(cfg, "cuda", torch.bfloat16, seed=1, max_positions=512, std=0.05)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = randn(g, T, 896)
+    results = []
+    for fused in (True, False):
+        m = fragmented_manager(64, 16, torch.Generator().manual_seed(3))
+        cache = PagedKVCache(cfg, m.num_blocks, 16, "cuda", torch.bfloat16, attn_backend="hip")
+        cache.k.zero_()
+        cache.v.zero_()
+        m.allocate(0, T)
+        meta = build_metadata(m, [(0, 0, T)], "cuda")
+        cache.begin(T, meta)
+        rot = model.rotary.rows(meta.positions, torch.bfloat16)
+        with torch.inference_mode() if fused else torch.no_grad():
+            assert hip_layer.supported(x, model.layers[0], rot, 18, 64) == fused
+            results.append((model.layer_forward(0, x, meta.positions, cache, rot), cache.k, cache.v))
+    for a, b in zip(*results):
+        # the torch side rounds up to 16 times along a chain of operations (norm 2, projection, rotary 3, attention,
+        # projection, sum, norm 2, projection, gate 2, projection, sum), at most 2^-9 of the value each and independent:
+        # sqrt(16) 2^-9 = 2^-7 a side, 2^-6 between two sides
+        assert rel(a, b.double()) < 2.0 ** -6
+
+
+def test_rotate_reference_matches_the_model():
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x, rot = randn(g, 5, 3, 32), (randn(g, 5, 1, 32), randn(g, 5, 1, 32))
+    assert rel(rotate(x, *rot), rotate64(x.double(), *rot)) < BOUND

@@ -54,7 +54,9 @@ namespace sipa {
 constexpr int kHotArgBytes = 3 * 8 + 6 * 4;
 
 // NB: tiles in flight per wave (the register prefetch ring); PHL: P as a bf16 hi + lo pair (else one bf16 term).
-template <int D, int NB, bool PHL>
+// BS: blocks of 16 << BS tokens, addressed as 16-token blocks (fetch_split_ids_flat). 24 x 3000 tokens of 32-token
+// blocks at head_dim 128: 94.4 us on the VALU kernel, which served every block size but 16; 18.5 here.
+template <int D, int NB, bool PHL, int BS>
 __global__ void __launch_bounds__(kThreads) decode_mfma_bf16(const int32_t* __restrict__ hbt,
                                                              const int32_t* __restrict__ hctx,
                                                              const int32_t* __restrict__ hitems, int32_t hbt_ss,
@@ -80,7 +82,7 @@ __global__ void __launch_bounds__(kThreads) decode_mfma_bf16(const int32_t* __re
   // Prologue: the split's block ids, the context length, the query and the kernel arguments the first tiles need
   // are all requested before anything waits, so the first K/V loads follow one memory round trip.
   int ids[kIdsPerThread];
-  fetch_split_ids_flat(hp.bt, hp.bt_ss, hp.bt_w, s, start, w.end, ids);
+  fetch_split_ids_flat<kIdsPerThread, BS>(hp.bt, hp.bt_ss, hp.bt_w, s, start, w.end, ids);
   const uint16_t* const kbase = (const uint16_t*)a.k;
   const uint16_t* const vbase = (const uint16_t*)a.v;
   const int64_t kv_sh = a.kv_sh, kv_sn = a.kv_sn;
@@ -122,7 +124,7 @@ __global__ void __launch_bounds__(kThreads) decode_mfma_bf16(const int32_t* __re
   const bool past_end = w.nvalid < 0 && start >= ctx;  // grid: a split past this sequence's end
   const int end = max(start, min(w.end, ctx));
   const int nvalid = w.nvalid < 0 ? (ctx + hp.chunk - 1) / hp.chunk : w.nvalid;
-  commit_split_ids_flat(ids, bids, nblocks);
+  commit_split_ids_flat<kIdsPerThread, BS>(ids, bids, nblocks, start);
   __syncthreads();  // block ids staged
   if (past_end) return;
 
@@ -597,9 +599,9 @@ static int prefetch_tiles(int D) {
 }
 
 // The bf16 kernel takes its prologue's fields as leading scalars (preloaded into SGPRs), then the whole block.
-template <int D, int NB, bool PHL>
+template <int D, int NB, bool PHL, int BS = 0>
 static int launch_bf16(dim3 grid, const DecodeArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL((decode_mfma_bf16<D, NB, PHL>), grid, dim3(kThreads), 0, st, a.bt, a.ctx, a.items, (int32_t)a.bt_ss,
+  hipLaunchKernelGGL((decode_mfma_bf16<D, NB, PHL, BS>), grid, dim3(kThreads), 0, st, a.bt, a.ctx, a.items, (int32_t)a.bt_ss,
                      a.S * a.Hkv, a.S, a.chunk, a.max_ctx, a.bt_w, a);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(SIPA_EHIP, "decode launch failed: %s", hipGetErrorString(e));
@@ -607,7 +609,9 @@ static int launch_bf16(dim3 grid, const DecodeArgs& a, hipStream_t st) {
 }
 
 template <bool PHL>
-static int launch_mfma(int D, int nb, dim3 grid, const DecodeArgs& a, hipStream_t st) {
+static int launch_mfma(int D, int nb, int bs, dim3 grid, const DecodeArgs& a, hipStream_t st) {
+  if (bs == 1) return D == 64 ? launch_bf16<64, 2, PHL, 1>(grid, a, st) : launch_bf16<128, 2, PHL, 1>(grid, a, st);
+  if (bs == 2) return D == 64 ? launch_bf16<64, 2, PHL, 2>(grid, a, st) : launch_bf16<128, 2, PHL, 2>(grid, a, st);
   if (D == 64) {
     switch (nb) {
       case 1: return launch_bf16<64, 1, PHL>(grid, a, st);
@@ -989,9 +993,16 @@ static int decode_impl(const sipa_decode_params* p, void* stream, bool use_scrat
   }
 
   // The MFMA kernels: bf16 query, 16-token blocks, head_dim 64 / 128, 16-byte aligned rows, and for INT8 pools
-  // fp16 scales laid out for 8-byte (per-token) and 16-byte (per-channel) vector loads.
+  // fp16 scales laid out for 8-byte (per-token) and 16-byte (per-channel) vector loads. Blocks of 32 and 64 tokens
+  // run as 16-token blocks where the pool (and its per-token scales) can be read so: contiguous blocks, counts within
+  // int32. A per-channel scale spans its whole block, so that format keeps 16-token blocks only.
   const bool q_aligned = aligned16(p->q) && p->q_stride_s % 8 == 0 && p->q_stride_h % 8 == 0;
-  bool mfma_ok = p->q_dtype == SIPA_BF16 && B == 16 && (D == 64 || D == 128) && q_aligned;
+  const int bs = B == 64 ? 2 : B == 32 ? 1 : 0;
+  const bool as_16 = bs > 0 && p->kv_stride_n == (int64_t)B * D && p->num_blocks <= INT32_MAX >> bs &&
+                     p->bt_width <= INT32_MAX >> bs &&
+                     (mode == SIPA_KV_PLAIN ||
+                      (mode == SIPA_KV_INT8_TOKEN && p->vs_stride_n == B && p->ks_stride_n == B));
+  bool mfma_ok = p->q_dtype == SIPA_BF16 && (B == 16 || as_16) && (D == 64 || D == 128) && q_aligned;
   int int8_variant = 0;
   if (mfma_ok && mode != SIPA_KV_PLAIN) {
     auto tok_scales_ok = [](const void* ptr, int dt, int64_t sh, int64_t sn) {
@@ -1020,12 +1031,17 @@ static int decode_impl(const sipa_decode_params* p, void* stream, bool use_scrat
                "of 6-8, a bf16 pool or an int8 per-token pool with fp16 scales, and 16-byte aligned rows");
   }
   SIPA_CHECK(p->impl != SIPA_IMPL_MFMA_PBF16 || (mfma_ok && mode == SIPA_KV_PLAIN), SIPA_EUNSUPPORTED,
-             "the bf16-P MFMA variant needs a bf16 query and pool, block 16, head_dim 64/128, 16-byte aligned rows");
+             "the bf16-P MFMA variant needs a bf16 query and pool, block 16, 32 or 64, head_dim 64/128, 16-byte aligned rows");
   SIPA_CHECK(p->impl != SIPA_IMPL_MFMA || mfma_ok, SIPA_EUNSUPPORTED,
-             "the MFMA kernels need a bf16 query, block 16, head_dim 64/128, 16-byte aligned rows and fp16 scales "
+             "the MFMA kernels need a bf16 query, block 16 (32 or 64: not per channel), head_dim 64/128, 16-byte aligned rows and fp16 scales "
              "(or fp32 channel scales with a zero block stride)");
   const bool p_bf16 = p->impl == SIPA_IMPL_MFMA_PBF16;
   const bool use_mfma = mfma_ok && (p->impl == SIPA_IMPL_AUTO || p->impl == SIPA_IMPL_MFMA || p_bf16);
+  if (use_mfma && bs > 0) {
+    a.nb <<= bs;
+    a.kv_sn = 16 * D;
+    if (mode != SIPA_KV_PLAIN) a.vs_sn = a.ks_sn = 16;
+  }
 
   // Measured on C4 (sweeps of the ratio, alternating runs): format B 30.9 -> 30.1 us at 1.6; the per-token format
   // within noise at every ratio (and 0.2 us slower at 1.6 with its workgroup-wide scale staging), so it keeps equal
@@ -1040,10 +1056,10 @@ static int decode_impl(const sipa_decode_params* p, void* stream, bool use_scrat
   if (valu_stream)
     rc = launch_valu_stream(D, G, mode, p->impl == SIPA_IMPL_VALU_DOT2, grid, a, st);
   else if (use_mfma && mode == SIPA_KV_PLAIN)
-    rc = p_bf16 ? launch_mfma<false>(D, prefetch_tiles(D), grid, a, st)
-                : launch_mfma<true>(D, prefetch_tiles(D), grid, a, st);
+    rc = p_bf16 ? launch_mfma<false>(D, prefetch_tiles(D), bs, grid, a, st)
+                : launch_mfma<true>(D, prefetch_tiles(D), bs, grid, a, st);
   else if (use_mfma)
-    rc = launch_mfma_int8(D, int8_variant, prefetch_tiles(D), grid, a, st);
+    rc = launch_mfma_int8(D, int8_variant, prefetch_tiles(D), bs, grid, a, st);
   else if (p->q_dtype == SIPA_F32)
     rc = dispatch_valu<SIPA_F32>(D, mode, grid, a, st);
   else

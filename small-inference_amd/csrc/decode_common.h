@@ -425,23 +425,42 @@ __device__ __forceinline__ int fetch_split_ids(const int32_t* bt, int64_t bt_ss,
 // again, an empty split reads column 0 of its row), so no use of one id can be placed between the loads and the
 // next memory operations: the ids, the context length and the kernel arguments are then in flight together and
 // the first K/V loads wait for one round trip. N x kThreads ids: the longest split the kernel stages.
-template <int N>
+//
+// BS: blocks of 16 << BS tokens. The pool [Hkv, N, B, D] with contiguous blocks is, token for token, a pool of
+// N << BS 16-token blocks, so the ids staged are those of the 16-token parts ((id << BS) + part) and the rest of the
+// kernel works on 16-token blocks only.
+template <int N, int BS = 0>
 __device__ __forceinline__ int fetch_split_ids_flat(const int32_t* bt, int64_t bt_ss, int bt_w, int s, int start,
                                                     int end_spec, int (&ids)[N]) {
-  const int nb_spec = min((end_spec - start + 15) >> 4, bt_w - (start >> 4));  // never past the row's width
+  const int nb_spec = min((end_spec - start + 15) >> 4, (bt_w << BS) - (start >> 4));  // never past the row's width
   const int last = max(nb_spec - 1, 0);
-  const int32_t* btr = bt + (int64_t)s * bt_ss + (nb_spec > 0 ? (start >> 4) : 0);
+  const int first = nb_spec > 0 ? start >> 4 : 0;
+  const int32_t* btr = bt + (int64_t)s * bt_ss + (BS == 0 ? first : 0);
 #pragma unroll
-  for (int i = 0; i < N; ++i) ids[i] = btr[min((int)threadIdx.x + kThreads * i, last)];
+  for (int i = 0; i < N; ++i) {
+    const int j = min((int)threadIdx.x + kThreads * i, last);
+    ids[i] = btr[BS == 0 ? j : (first + j) >> BS];
+  }
   return nb_spec;
+}
+
+// The 16-token block of entry j of a split at `start` whose table entry is id, clamped into a pool of nblocks 16-token
+// blocks.
+template <int BS>
+__device__ __forceinline__ int block_id(int id, int start, int j, int nblocks) {
+  if (BS == 0) return min(max(id, 0), nblocks - 1);
+  return (min(max(id, 0), (nblocks >> BS) - 1) << BS) | (((start >> 4) + j) & ((1 << BS) - 1));
 }
 
 // Stages every thread's ids (N x kThreads entries of bids, those past the split unused), clamped into the pool,
 // without a branch.
-template <int N>
-__device__ __forceinline__ void commit_split_ids_flat(const int (&ids)[N], int* bids, int nblocks) {
+template <int N, int BS = 0>
+__device__ __forceinline__ void commit_split_ids_flat(const int (&ids)[N], int* bids, int nblocks, int start = 0) {
 #pragma unroll
-  for (int i = 0; i < N; ++i) bids[threadIdx.x + kThreads * i] = min(max(ids[i], 0), nblocks - 1);
+  for (int i = 0; i < N; ++i) {
+    const int j = threadIdx.x + kThreads * i;
+    bids[j] = block_id<BS>(ids[i], start, j, nblocks);
+  }
 }
 
 // Ids outside the pool are clamped into it: a bad table gives wrong results, never an access out of bounds.
@@ -544,6 +563,7 @@ int launch_valu_stream(int D, int G, int mode, int dot, dim3 grid, const DecodeA
 
 // INT8 MFMA kernels (decode_int8.hip). mode: 1 per-token K scales, 2 per-(block, channel) K scales,
 // 3 per-(head, channel) K scales (mode 2 with a zero block stride). nb: tiles in flight per wave.
-int launch_mfma_int8(int D, int mode, int nb, dim3 grid, const DecodeArgs& a, hipStream_t st);
+// bs: blocks of 16 << bs tokens (mode 1 only; 0 otherwise), with a's block counts and strides in 16-token blocks.
+int launch_mfma_int8(int D, int mode, int nb, int bs, dim3 grid, const DecodeArgs& a, hipStream_t st);
 
 }  // namespace sipa

@@ -73,7 +73,8 @@ constexpr int kWaveScaleBlocks = kScaleBlocks / kWaves;  // blocks of one wave's
 
 // MODE 1: per-token K scales; 2: per-(block, channel) K scales; 3: mode 2 with one channel scale per (head,
 // channel) for every block (a zero block stride), folded into the query once.
-template <int D, int MODE, int NB>
+// BS (mode 1): blocks of 16 << BS tokens, addressed as 16-token blocks with 16 token scales each.
+template <int D, int MODE, int NB, int BS>
 __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs a) {
   constexpr int KS = D / 32;   // QK k-steps per block
   constexpr int DT = D / 16;   // PV d-tiles
@@ -128,7 +129,7 @@ __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs
   // issued. The first K/V loads then follow one memory round trip.
   static_assert(kMaxInt8Split / 16 == kThreads, "one block id per thread");
   int ids[1];
-  fetch_split_ids_flat(a.bt, a.bt_ss, a.bt_w, s, start, wend, ids);
+  fetch_split_ids_flat<1, BS>(a.bt, a.bt_ss, a.bt_w, s, start, wend, ids);
   // The query group in bf16, channel order of the int8 K layout: k-step j of lane (r, q4) (zero for r >= G).
   const uint16_t* qrow = (const uint16_t*)a.q + (int64_t)s * a.q_ss + (int64_t)(h * G + min(r, G - 1)) * a.q_sh;
   auto load_qb = [&](int j) {
@@ -175,8 +176,8 @@ __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs
   };
   // Per-workgroup staging: thread t's block t, with the id it fetched (threads past the split read its last block
   // again, not staged).
-  if (!kWaveScales) load_scales(min(max(ids[0], 0), a.nb - 1));
-  commit_split_ids_flat(ids, bids, a.nb);
+  if (!kWaveScales) load_scales(block_id<BS>(ids[0], start, threadIdx.x, a.nb));
+  commit_split_ids_flat<1, BS>(ids, bids, a.nb, start);
   __syncthreads();
   if (past_end) return;
   const int nblk = (end - start + 15) >> 4;  // blocks of this split, <= kMaxInt8Split / 16
@@ -501,14 +502,20 @@ static int launch_int8(Kernel k, dim3 grid, const DecodeArgs& a, hipStream_t st)
 template <int D, int MODE>
 static int launch_int8_depth(int nb, dim3 grid, const DecodeArgs& a, hipStream_t st) {
   switch (nb) {
-    case 1: return launch_int8(decode_mfma_int8<D, MODE, 1>, grid, a, st);
-    case 2: return launch_int8(decode_mfma_int8<D, MODE, 2>, grid, a, st);
-    default: return launch_int8(decode_mfma_int8<D, MODE, 3>, grid, a, st);
+    case 1: return launch_int8(decode_mfma_int8<D, MODE, 1, 0>, grid, a, st);
+    case 2: return launch_int8(decode_mfma_int8<D, MODE, 2, 0>, grid, a, st);
+    default: return launch_int8(decode_mfma_int8<D, MODE, 3, 0>, grid, a, st);
   }
 }
 
 // mode: 1, 2, or 3 (mode 2 with a zero block stride of the channel scales).
-int launch_mfma_int8(int D, int mode, int nb, dim3 grid, const DecodeArgs& a, hipStream_t st) {
+int launch_mfma_int8(int D, int mode, int nb, int bs, dim3 grid, const DecodeArgs& a, hipStream_t st) {
+  if (bs == 1)
+    return D == 64 ? launch_int8(decode_mfma_int8<64, 1, 2, 1>, grid, a, st)
+                   : launch_int8(decode_mfma_int8<128, 1, 2, 1>, grid, a, st);
+  if (bs == 2)
+    return D == 64 ? launch_int8(decode_mfma_int8<64, 1, 2, 2>, grid, a, st)
+                   : launch_int8(decode_mfma_int8<128, 1, 2, 2>, grid, a, st);
   if (D == 64) {
     switch (mode) {
       case 1: return launch_int8_depth<64, 1>(nb, grid, a, st);

@@ -15,7 +15,7 @@ import pytest
 import torch
 
 from cases import HEADS, RAGGED, assert_decode_close, make_case, oracle_decode, ramp_scores
-from engine.hip_decode import choose_splits, paged_decode_attention, split_plan
+from engine.hip_decode import QuantKV, choose_splits, paged_decode_attention, split_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -374,3 +374,38 @@ def test_scores_trending_across_keys(direction, splits):
     torch.cuda.synchronize()
     ref32 = oracle_decode(q, k, v, tables, lengths, D ** -0.5, np.float32)
     assert_decode_close(out.double().cpu().numpy(), ref32, "trending scores")
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "int8"])
+@pytest.mark.parametrize("heads", list(HEADS))
+@pytest.mark.parametrize("B", [32, 64])
+@pytest.mark.parametrize("path", ["single", "split3", "auto", "work list", "bad ids"])
+def test_larger_blocks_equal_their_16_token_parts(fmt, heads, B, path):
+    """Blocks of 32 and 64 tokens run the MFMA kernels as 16-token blocks: the same bits as the pool and tables
+    rewritten in 16-token blocks (token for token the same memory), at lengths around the edges of both block sizes;
+    ids outside the pool are clamped to it first."""
+    Hq, Hkv, D = HEADS[heads]
+    lengths = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 96, 300, 1000, 2500]
+    q, k, v, bt, ctx, _ = make_case(lengths, Hq, Hkv, D, B, torch.bfloat16, seed=B)
+    N, part = k.shape[1], B // 16
+    quant = quant16 = None
+    if fmt == "int8":
+        g = torch.Generator(device="cuda").manual_seed(B)
+        k = torch.randint(-127, 128, k.shape, device="cuda", dtype=torch.int8, generator=g)
+        v = torch.randint(-127, 128, v.shape, device="cuda", dtype=torch.int8, generator=g)
+        ks, vs = ((torch.rand(k.shape[:3], device="cuda", generator=g) / 64 + 1 / 256).half() for _ in range(2))
+        quant = QuantKV(1, ks, vs)
+        quant16 = QuantKV(1, ks.view(Hkv, -1, 16), vs.view(Hkv, -1, 16))
+    if path == "bad ids":
+        bt = bt.clone()
+        bt[11, 0], bt[12, 1], bt[13, 2] = N + 3, -7, 2 ** 30
+    ids = bt.clamp(0, N - 1)[:, :, None] * part + torch.arange(part, device="cuda", dtype=torch.int32)
+    k16, v16 = k.view(Hkv, N * part, 16, D), v.view(Hkv, N * part, 16, D)
+    kw = dict(num_splits={"single": 1, "split3": 3}.get(path), impl="mfma")
+    if path == "work list":
+        kw.update(host_context_lens=lengths, work_list="on")
+    print(f"case block {B} {fmt} {heads} {path}", flush=True)
+    out = paged_decode_attention(q, k, v, bt, ctx, D ** -0.5, max(lengths), quant=quant, **kw)
+    ref = paged_decode_attention(q, k16, v16, ids.flatten(1).contiguous(), ctx, D ** -0.5, max(lengths), quant=quant16,
+                                 **kw)
+    assert torch.equal(out, ref)

@@ -55,7 +55,7 @@ constexpr int kHotArgBytes = 3 * 8 + 6 * 4;
 
 // NB: tiles in flight per wave (the register prefetch ring); PHL: P as a bf16 hi + lo pair (else one bf16 term).
 // BS: blocks of 16 << BS tokens, addressed as 16-token blocks (fetch_split_ids_flat). 24 x 3000 tokens of 32-token
-// blocks at head_dim 128: 94.4 us on the VALU kernel, which served every block size but 16; 18.5 here.
+// blocks at head_dim 128: 94.4 us on the VALU kernel, which served every block size but 16; 17.3 here.
 template <int D, int NB, bool PHL, int BS>
 __global__ void __launch_bounds__(kThreads) decode_mfma_bf16(const int32_t* __restrict__ hbt,
                                                              const int32_t* __restrict__ hctx,
@@ -520,6 +520,13 @@ static WorkspaceLayout workspace_layout(int64_t S, int64_t Hq, int64_t Hkv, int6
 
 static int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
+int split_chunk_host(int max_ctx, int splits) {
+  splits = std::max(1, splits);
+  const int per = ceil_div(std::max(1, max_ctx), splits);
+  // A split never exceeds the block ids the MFMA kernel stages in LDS (kMaxSplitBlocks blocks of 16 tokens).
+  return std::min(ceil_div(per, kChunkAlign) * kChunkAlign, kMaxSplitBlocks * 16);
+}
+
 // At most one workgroup per CU: each workgroup pays a fixed cost of two dependent memory round trips before its
 // first tile and the split merge after its last, so a few long-running workgroups beat many short ones (measured
 // on MI355X, bf16 32 x 8192: 4 splits 27.9 us, 8 splits 29.2 us, 16 splits 44.6 us). A small batch does not fill
@@ -528,24 +535,26 @@ static int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 // against 6.9 at 4; 1 x 8192 at 16, 9.8 against 10.3 at 32; 4 x 8192 at 16, 10.9 against 12.8 at 32; 8 x 4096
 // at 8, 10.4 against 11.5 at 16). The INT8 kernels, two workgroups per CU, take splits down to 256 tokens past 8
 // splits (1 x 4096: 9.8 us at 16 splits against 11.6 at 8; 1 x 1024: 7.6 us at 8 against 8.6 at 4). kMaxChunk
-// spreads a long sequence of a full grid over several CUs.
+// spreads a long sequence of a full grid over several CUs. Programs that do not divide the CUs, rounded down against
+// up: 24 x 3000 at head_dim 128 17.5 against 24.0 us (5 and 6 splits), 0.5B 100 x 1000
+// 12.5 against 14.6 (1 and 2), INT8 200 x 300 8.7 against 10.0.
 int choose_splits_host(int S, int Hkv, int max_ctx, int cu_count, bool int8) {
   if (S <= 0 || Hkv <= 0 || max_ctx <= 0) return 1;
   if (cu_count <= 0) cu_count = 256;
   const int64_t programs = (int64_t)S * Hkv;
   int64_t splits = (cu_count + programs - 1) / programs;
+  // Where the programs do not divide the CUs, rounding up puts two workgroups on some CUs and one on the others, and
+  // the launch ends with those few alone: rounding down is better when a CU then holds no more tokens.
+  const auto load = [&](int64_t n) {  // tokens of the CU with the most work
+    const int chunk = split_chunk_host(max_ctx, (int)n);
+    return (programs * ceil_div(max_ctx, chunk) + cu_count - 1) / cu_count * (int64_t)chunk;
+  };
+  if (splits > 1 && splits * programs > cu_count && load(splits - 1) <= load(splits)) --splits;
   const int64_t most = std::max<int64_t>(ceil_div(max_ctx, int8 ? kMinChunk : kLatencyChunk),
                                          std::min<int64_t>(kShortSplits, ceil_div(max_ctx, kShortChunk)));
   splits = std::min<int64_t>(splits, most);
   splits = std::max<int64_t>(splits, ceil_div(max_ctx, kMaxChunk));
   return (int)std::max<int64_t>(1, std::min<int64_t>(splits, 1 << 20));
-}
-
-int split_chunk_host(int max_ctx, int splits) {
-  splits = std::max(1, splits);
-  const int per = ceil_div(std::max(1, max_ctx), splits);
-  // A split never exceeds the block ids the MFMA kernel stages in LDS (kMaxSplitBlocks blocks of 16 tokens).
-  return std::min(ceil_div(per, kChunkAlign) * kChunkAlign, kMaxSplitBlocks * 16);
 }
 
 template <typename Kernel>

@@ -324,3 +324,15 @@ def bad_linear(**over):
 def test_fused_linear_refuses_bad_arguments(over, code):
     assert _hip.lib().sipa_fused_linear(ctypes.byref(bad_linear(**over)), None) == code
     assert _hip.lib().sipa_last_error()
+
+
+@pytest.mark.parametrize("S,ctx,mode,want", [
+    (24, 3000, 0, 5),   # 48 programs: 5 splits of 640 on 240 CUs, not 6 of 512 with two workgroups on some CUs
+    (100, 1000, 0, 1),  # 200 programs: whole sequences, not halves with two workgroups on some CUs
+    (100, 900, 0, 1),
+    (40, 2000, 0, 3),   # 80 programs: 3 splits of 704 against 4 of 512, two on some CUs
+    (96, 1100, 0, 1),
+    (200, 300, 1, 1),   # INT8, twice the CUs: 400 programs
+])
+def test_split_policy_where_programs_do_not_divide_the_cus(S, ctx, mode, want):
+    assert _hip.lib().sipa_choose_splits_for(S, 2, ctx, 256, mode) == want

@@ -454,7 +454,7 @@ int32_t sipa_kchan_write_rows(const sipa_kchan_write_params* p, void* stream);
  * The decoder layer's operations around the paged attention (reference engine/model.py:101-175), bf16 in and out with
  * fp32 arithmetic. Pointers are device pointers; strides are row strides in elements; the last dimension is contiguous.
  *
- * sipa_fused_linear: y = epilogue(norm(x) W^T), one launch, for few tokens (it streams W once per 64 tokens):
+ * sipa_fused_linear: y = epilogue(norm(x) W^T), one launch:
  *   x [T, K], weight [N, K] contiguous, K a multiple of 64; norm_weight [K] or NULL: x is RMS-normalised first,
  *   x * rsqrt(mean(x^2) + eps) * norm_weight (the row factor applied to the product's fp32 sums).
  *   SIPA_LINEAR_RESIDUAL: out[t, n] = y + bias[n] + residual[t, n] (each may be NULL);             N % 16 == 0
@@ -463,8 +463,11 @@ int32_t sipa_kchan_write_rows(const sipa_kchan_write_params* p, void* stream);
  *                         its head; rot_cos, rot_sin [T, head_dim] contiguous, sin with rotate-half's sign folded in;
  *                         N % 16 == 0, head_dim % 16 == 0
  *   SIPA_LINEAR_SILU:     out[t, i] = silu(y[t, i]) * y[t, N / 2 + i];                              N % 16 == 0
- * x, weight and norm_weight must be 16-byte aligned and x_stride a multiple of 8. out must not overlap the inputs,
- * except that it may be the residual itself.
+ * x, weight and norm_weight must be 16-byte aligned and x_stride a multiple of 8; the others 8-byte aligned with
+ * strides of a multiple of 4. out must not overlap the inputs, except that it may be the residual itself.
+ * A long K of the residual epilogue without norm may be shared by several workgroups (num_splits, 0: the library's
+ * choice); the call then needs sipa_linear_scratch_bytes(p) bytes of scratch (any contents) and zero counters, int32,
+ * one per tile: the counter region of a decode workspace serves (they are left at zero).
  */
 enum { SIPA_LINEAR_RESIDUAL = 0, SIPA_LINEAR_ROPE = 1, SIPA_LINEAR_SILU = 2 };
 
@@ -484,12 +487,47 @@ typedef struct sipa_linear_params {
   int64_t out_stride;
   const void* rot_cos;
   const void* rot_sin;
-  int32_t num_splits; /* RESIDUAL without norm: workgroups that share a row tile's K (0 or 1: none) */
-  void* part;         /* num_splits > 1: fp32 [N / 16][ceil(T / 16) rounded up to 1, 2 or a multiple of 4][num_splits][256] */
-  void* counters;     /* num_splits > 1: int32 [N / 16][ceil(T / 64)], zero; left at zero */
+  int32_t num_splits; /* 0: the library's choice */
+  int32_t tile;       /* 0: the library's choice; 1 .. 5: tiles of 32 x 32, 32 x 64, 64 x 64, 64 x 128, 128 x 128 tokens x
+                         rows of W; 6: the kernel for up to 16 tokens and 1536 in_features */
+  void* scratch;
+  int64_t scratch_bytes;
+  void* counters;
 } sipa_linear_params;
 
 int32_t sipa_fused_linear(const sipa_linear_params* p, void* stream);
+
+/* Scratch bytes the call needs (0: none), or a negative return code. Reads sizes, epilogue, norm_weight (NULL or not),
+ * num_splits and tile. */
+int64_t sipa_linear_scratch_bytes(const sipa_linear_params* p);
+
+/*
+ * A decoder layer after its attention, three launches: h = x + attn o_w^T; out = h + swiglu(rms_norm(h) gate_up_w^T)
+ * down_w^T. x, attn with row strides, out [T, hidden] contiguous; matrices [out, in] contiguous; sizes and alignment as
+ * for sipa_fused_linear. scratch: sipa_layer_out_scratch_bytes(p) bytes (any contents); counters as above.
+ */
+typedef struct sipa_layer_out_params {
+  int32_t struct_size; /* sizeof(sipa_layer_out_params) */
+  int32_t num_tokens, hidden, attn_features, inter;
+  float eps;
+  const void* x;
+  int64_t x_stride;
+  const void* attn;
+  int64_t attn_stride;
+  const void* o_w;
+  const void* post_norm;
+  const void* gate_up_w;
+  const void* down_w;
+  void* out;
+  void* scratch;
+  int64_t scratch_bytes;
+  void* counters;
+} sipa_layer_out_params;
+
+int32_t sipa_layer_out(const sipa_layer_out_params* p, void* stream);
+
+/* Reads the sizes only. */
+int64_t sipa_layer_out_scratch_bytes(const sipa_layer_out_params* p);
 
 /*
  * RMSNorm of T rows of K <= 8192 channels (K % 8 == 0): out = bf16(bf16(s * rsqrt(mean(s^2) + eps)) * weight), with

@@ -4,36 +4,23 @@
 //
 // Reference: engine/model.py:101-175 (RMSNorm, fused QKV with bias, rotary embedding, SwiGLU MLP, residuals), there
 // about 30 separate torch operations a layer.
+#include <algorithm>
+
 #include "decode_common.h"
 
 namespace sipa {
 
-// ---- skinny_linear: y = epilogue(norm(x) W^T), few tokens -----------------------------------------------------------
+// Two kernels compute y = epilogue(norm(x) W^T), a projection fused with what stands before and after it.
 //
-// Bound: the weights' read from HBM and, for a layer's 2 to 17 MB, as much the latency of one launch: load, reduce,
-// store. So a workgroup owns whole rows of W (16 rows times RT tiles, all of K), its WV waves take 64-channel slices
-// of K, the loads of two slices ahead are in flight, and nothing is written before the result: one launch, no
-// partials, no second pass. Against a GEMM library's tiles (56 workgroups of a 4864-long serial loop for the MLP's
-// down projection) every wave's share of K is a few loads.
+// W enters the MFMA as the A operand, x as the B operand, so D[n][t] comes out with lane (t, q4) holding outputs
+// n = 4 q4 .. 4 q4 + 3 of token t.
 //
-// W enters the MFMA as the A operand straight from memory, lane (r, q4) holding row r's channels 16 q4 .. 16 q4 + 15
-// of a slice (four lanes read one 128-byte line of a row), x as the B operand in the same channel order, so D[n][t]
-// comes out with lane (t, q4) holding outputs n = 4 q4 .. 4 q4 + 3 of token t. The waves' partial sums meet in LDS.
+// RMSNorm (NORM): the row factor rstd[t] factors out of the product, so x * w_norm is rounded to bf16 for the MFMA (one
+// rounding, where norm-then-multiply in bf16 has two), the squares of x are summed on the way, and the accumulators
+// are scaled at the end: no pass over x before the product.
 //
-// RMSNorm (NORM): the row scale rstd[t] factors out of the product, so x * w_norm is rounded to bf16 for the MFMA
-// (one rounding, where norm-then-multiply in bf16 has two), the squares of x are summed on the way, and the
-// accumulators are scaled in the epilogue: no pass over x before the product and no barrier.
-//
-// Split K (RESIDUAL): 896 outputs are 56 row tiles, and a CU's share of a 4864-long K, 155 KB, is more than one CU has
-// in flight; four workgroups share it and the last one adds their sums.
-//
-// Measured in a graph, weights from memory, 8 tokens, against the GEMM library and the operations around it one by one
-// (us): norm + QKV 1152 x 896 + bias + rotary 4.8 (library product 5.5, with 12 launches around it); o 896 x 896 +
-// residual 4.0 (5.5 + 2); norm + gate/up 9728 x 896 + SwiGLU 8.8 (8.5 + 10 launches); down 896 x 4864 + residual 7.0
-// with four splits, 8.8 with two, 11.6 with one (16.8 + 2). A whole decode step of 8 sequences (24 layers) 3018 -> 972.
-//
-// Row tiles: for ROPE and SILU a tile's 16 rows are 8 rows and their 8 partners (channels c and c + D/2 of a head;
-// gate and up), so one thread holds both halves of a pair.
+// Row tiles of 16: for ROPE and SILU they are 8 rows and their 8 partners (channels c and c + D/2 of a head; gate and
+// up), so that both halves of a pair meet in one tile.
 enum { kEpiResidual = 0, kEpiRope = 1, kEpiSilu = 2 };
 
 struct LinearArgs {
@@ -53,9 +40,9 @@ struct LinearArgs {
   int32_t tiles;           // row tiles in all
   int32_t inter;           // SILU: gate rows (the up rows follow)
   int32_t units;           // 64-channel slices of K a workgroup takes
-  int32_t splits;          // workgroups that share a row tile's K (RESIDUAL)
-  float* part;             // [row tile][token group][splits][RT][TT][256] partial sums
-  int32_t* counters;       // [row tile][token group] workgroups done, zero between calls
+  int32_t splits;          // workgroups that share a tile's K (RESIDUAL)
+  float* part;             // [tile][splits][tokens x rows of a tile] partial sums
+  int32_t* counters;       // [tile] workgroups done, zero between calls
 };
 
 template <int EPI>
@@ -69,7 +56,11 @@ __device__ __forceinline__ int linear_row(const LinearArgs& a, int tile, int r) 
   return tile * 16 + r;
 }
 
-__device__ __forceinline__ u32x4 weight_load(const uint16_t* p) { return stream_load(p); }
+// x / (1 + e^-x) in fp32: the hardware's exp2 and reciprocal, each within an ulp or two, 2^-8 of the bf16 step the
+// result is rounded to. (Very negative x: e^-x = inf, and x * 0 = -0.)
+__device__ __forceinline__ float silu(float x) {
+  return x * __builtin_amdgcn_rcpf(1.f + fast_exp2(-1.4426950408889634f * x));
+}
 
 // x * w per channel, rounded to bf16, and the sum of x's squares.
 __device__ __forceinline__ u32x4 scale_channels(u32x4 x, u32x4 w, float& ss) {
@@ -85,121 +76,250 @@ __device__ __forceinline__ u32x4 scale_channels(u32x4 x, u32x4 w, float& ss) {
   return o;
 }
 
-// U: 64-channel slices of a stage; NST: stages in flight (one where the wave's whole share is one stage).
-template <int EPI, bool NORM, int TT, int RT, int WV, int U, int NST>
-__global__ void __launch_bounds__(64 * WV) skinny_linear(const LinearArgs a) {
-  __shared__ __align__(16) float red[WV][RT][TT][256];
-  __shared__ float ssq[NORM ? WV : 1][TT * 16];
+// ---- skinny_linear: up to 16 tokens, few rows ---------------------------------------------------------------------------
+//
+// Bound: the latency of one launch (load, reduce, store) more than the 1.6 to 6 MB of weights. A workgroup owns 16 rows
+// and all of K, its 8 waves take 64-channel slices straight from memory into registers (lane (r, q4) channels
+// 16 q4 .. + 15 of row r: four lanes read one 128-byte line; x in the same channel order), at most U slices each, all in
+// flight together, and their sums meet in LDS.
+//
+// Measured in a graph, weights from memory, 8 tokens, against tile_linear's smallest tile and the GEMM library's product
+// alone (us): norm + QKV 1152 x 896 + bias + rotary 4.9, 6.1, 5.6; 2048 x 1536 6.1, 8.0, 7.2; 896 x 896 + residual 4.1,
+// 4.4, 5.6. An empty launch there is about 2.
+constexpr int kSkinnyWaves = 8;
+
+template <int EPI, bool NORM, int U>
+__global__ void __launch_bounds__(64 * kSkinnyWaves) skinny_linear(const LinearArgs a) {
+  constexpr int WV = kSkinnyWaves;
+  __shared__ __align__(16) float red[WV][256];
+  __shared__ float ssq[WV][16];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, r = lane & 15, q4 = lane >> 4;
-  const int tile0 = blockIdx.x * RT;
-  const int t_base = blockIdx.y * (16 * TT);
-  // slices [unit0, unit1) of K are this workgroup's; wave v takes unit0 + v, unit0 + v + WV, ...
-  const int unit0 = blockIdx.z * a.units, unit1 = min(unit0 + a.units, a.K >> 6);
-  const int units = unit1 - unit0;
-  const int mine = units > wave ? (units - wave + WV - 1) / WV : 0;
-
-  const uint16_t* wrow[RT];
+  const int tile = blockIdx.x;
+  const int units = a.K >> 6;
+  const uint16_t* const wrow = a.w + (int64_t)linear_row<EPI>(a, tile, r) * a.K + 16 * q4;
+  const uint16_t* const xrow = a.x + (int64_t)min(r, a.T - 1) * a.x_st + 16 * q4;
+  const uint16_t* const nrow = NORM ? a.norm_w + 16 * q4 : nullptr;
+  u32x4 w[U][2], x[U][2], nw[U][2];
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
-    wrow[i] = a.w + (int64_t)linear_row<EPI>(a, min(tile0 + i, a.tiles - 1), r) * a.K + 16 * q4;
-  const uint16_t* xrow[TT];
+  for (int u = 0; u < U; ++u) {
+    const int c = 64 * min(wave + WV * u, units - 1);  // past the end: the last slice again, masked below
 #pragma unroll
-  for (int i = 0; i < TT; ++i) xrow[i] = a.x + (int64_t)min(t_base + 16 * i + r, a.T - 1) * a.x_st + 16 * q4;
-  const uint16_t* nrow = NORM ? a.norm_w + 16 * q4 : nullptr;
-
-  struct Stage {
-    u32x4 w[U][RT][2], x[U][TT][2], n[U][2];
-  };
-  Stage st[NST];
-  // Slices past the wave's last re-read its last one and are not multiplied.
-  auto load = [&](Stage& s, int k) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int c = 64 * (unit0 + wave + WV * min(k + u, mine - 1));
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-#pragma unroll
-        for (int i = 0; i < RT; ++i) s.w[u][i][h] = weight_load(wrow[i] + c + 8 * h);
-#pragma unroll
-        for (int i = 0; i < TT; ++i) s.x[u][i][h] = *(const u32x4*)(xrow[i] + c + 8 * h);
-        if (NORM) s.n[u][h] = *(const u32x4*)(nrow + c + 8 * h);
-      }
-    }
-  };
-  f32x4 acc[RT][TT];
-  float ss[TT];
-#pragma unroll
-  for (int i = 0; i < RT; ++i)
-#pragma unroll
-    for (int j = 0; j < TT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int j = 0; j < TT; ++j) ss[j] = 0.f;
-  auto multiply = [&](Stage& s, int k) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      // A slice past the wave's share is masked to zeros, not branched around: with a branch here the compiler sinks
-      // the slice's loads into it, and their latencies add up instead of overlapping.
-      const uint32_t live = k + u < mine ? 0xffffffffu : 0u;
-#pragma unroll
-      for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) s.w[u][i][h] &= live;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < TT; ++j) {
-          u32x4 xv = s.x[u][j][h] & live;
-          if (NORM) xv = scale_channels(xv, s.n[u][h], ss[j]);
-#pragma unroll
-          for (int i = 0; i < RT; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, s.w[u][i][h]),
-                                                                __builtin_bit_cast(bf16x8, xv), acc[i][j], 0, 0, 0);
-        }
-    }
-  };
-  if (mine > 0) {
-    load(st[0], 0);
-    if constexpr (NST == 1) {
-      multiply(st[0], 0);
-    } else {
-      if (mine > U) load(st[1], U);
-      for (int k = 0; k < mine; k += 2 * U) {
-        multiply(st[0], k);
-        if (k + 2 * U < mine) load(st[0], k + 2 * U);
-        if (k + U < mine) {
-          multiply(st[1], k + U);
-          if (k + 3 * U < mine) load(st[1], k + 3 * U);
-        }
-      }
+    for (int h = 0; h < 2; ++h) {
+      w[u][h] = stream_load(wrow + c + 8 * h);
+      x[u][h] = *(const u32x4*)(xrow + c + 8 * h);
+      if (NORM) nw[u][h] = *(const u32x4*)(nrow + c + 8 * h);
     }
   }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
+  for (int u = 0; u < U; ++u) {
+    // masked to zeros, not branched around: with a branch the compiler sinks the slice's loads into it, and their
+    // latencies add up instead of overlapping
+    const uint32_t live = wave + WV * u < units ? 0xffffffffu : 0u;
 #pragma unroll
-    for (int j = 0; j < TT; ++j) *(f32x4*)&red[wave][i][j][lane * 4] = acc[i][j];
-  if (NORM) {
-#pragma unroll
-    for (int j = 0; j < TT; ++j) {
-      const float s = sum_over_rows(ss[j]);
-      if (q4 == 0) ssq[wave][16 * j + r] = s;
+    for (int h = 0; h < 2; ++h) {
+      u32x4 xv = x[u][h] & live;
+      if (NORM) xv = scale_channels(xv, nw[u][h], ss);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[u][h] & live),
+                                                    __builtin_bit_cast(bf16x8, xv), acc, 0, 0, 0);
     }
+  }
+  *(f32x4*)&red[wave][lane * 4] = acc;
+  if (NORM) {
+    const float s = sum_over_rows(ss);
+    if (q4 == 0) ssq[wave][r] = s;
   }
   __syncthreads();
 
-  if (EPI == kEpiResidual && a.splits > 1) {
-    // Split K: every workgroup stores its sums through to memory; the last to arrive adds them in split order.
-    constexpr int E = RT * TT * 256;
-    const int pair = blockIdx.y * gridDim.x + blockIdx.x;
-    float* const part = a.part + (int64_t)pair * a.splits * E;
-    float* const flat = &red[0][0][0][0];
-    __shared__ int last;
-    for (int e = threadIdx.x; e < E; e += 64 * WV) {
-      float s = 0.f;
+  // Pairs (n, n + 8) of the tile's outputs for one token; eight neighbouring threads store eight neighbouring channels.
+  const int n = threadIdx.x & 7, t = threadIdx.x >> 3;
+  if (t >= min(a.T, 16)) return;
+  const int at = ((n >> 2) * 16 + t) * 4 + (n & 3);  // output n's place; n + 8 is 128 words on
+  float lo = 0.f, hi = 0.f;
 #pragma unroll
-      for (int v = 0; v < WV; ++v) s += flat[v * E + e];
-      store_coherent(part + blockIdx.z * E + e, s);
+  for (int v = 0; v < WV; ++v) {
+    lo += red[v][at];
+    hi += red[v][at + 128];
+  }
+  if (NORM) {
+    float s = 0.f;
+#pragma unroll
+    for (int v = 0; v < WV; ++v) s += ssq[v][t];
+    const float rstd = rsqrtf(s / (float)a.K + a.eps);
+    lo *= rstd;
+    hi *= rstd;
+  }
+  const int nlo = linear_row<EPI>(a, tile, n), nhi = linear_row<EPI>(a, tile, n + 8);
+  if (EPI == kEpiSilu) {
+    a.out[t * a.out_st + nlo] = f32_to_bf16_bits(silu(lo) * hi);
+    return;
+  }
+  if (a.bias != nullptr) {
+    lo += bf16_bits_to_f32(a.bias[nlo]);
+    hi += bf16_bits_to_f32(a.bias[nhi]);
+  }
+  if (EPI == kEpiRope && tile * 16 < a.rot) {
+    const int c = nlo % a.D, c2 = c + (a.D >> 1);
+    const uint16_t *cs = a.cos + (int64_t)t * a.D, *sn = a.sin + (int64_t)t * a.D;
+    const float x0 = lo, x1 = hi;
+    lo = x0 * bf16_bits_to_f32(cs[c]) + x1 * bf16_bits_to_f32(sn[c]);
+    hi = x1 * bf16_bits_to_f32(cs[c2]) + x0 * bf16_bits_to_f32(sn[c2]);
+  }
+  if (EPI == kEpiResidual && a.res != nullptr) {
+    lo += bf16_bits_to_f32(a.res[t * a.res_st + nlo]);
+    hi += bf16_bits_to_f32(a.res[t * a.res_st + nhi]);
+  }
+  a.out[t * a.out_st + nlo] = f32_to_bf16_bits(lo);
+  a.out[t * a.out_st + nhi] = f32_to_bf16_bits(hi);
+}
+
+// ---- tile_linear: everything else -----------------------------------------------------------------------------------------
+//
+// Bound: at up to some hundred tokens neither HBM (2 to 17 MB of weights) nor the matrix cores (1 to 10 GFLOP) but the
+// latency of a short K loop on few workgroups, and for larger tiles the norm's VALU work. 4 waves (2 x 2) share a tile
+// of 32 TT tokens and 32 TN rows of W; both operands go through LDS (one read from L2 per workgroup), 64 channels a
+// step, two buffers, one barrier a step, with the loads of NR steps in flight in registers ahead of them. Rows of 128
+// bytes are stored with their 16-byte chunks xor-ed by the row, so the fragment reads of 16 rows spread over all
+// banks. The norm's products and squares are formed once per workgroup, on the way into LDS. A token's partner channel
+// is 32 lanes away, so the rotary and gated epilogues exchange accumulators with a shuffle.
+//
+// Split K (RESIDUAL): 896 outputs are 28 tiles of 32 rows, and one workgroup would take 76 steps of a 4864-long K; up to
+// six share it and the last one to arrive adds their sums in split order.
+//
+// Measured in a graph, weights from memory, against the GEMM library's product alone (us; the library needs a norm, 2.9,
+// a rotary, 2.1, a SwiGLU, 2.2 to 6, or a residual launch, 2, besides): 64 tokens: QKV 1152 x 896 6.3 (7.9), o 896 x 896
+// 4.5 (7.8), gate/up 9728 x 896 9.4 (11.8), down 896 x 4864 8.4 (13.7); 544 tokens: 9.6 (8.3), 5.6 (7.9), 25.3 (17.0),
+// 16.7 (15.9).
+template <int EPI, bool NORM, int TT, int TN, int NR>
+__global__ void __launch_bounds__(256) tile_linear(const LinearArgs a) {
+  static_assert(NR % 2 == 0, "a ring slot always meets the same LDS buffer");
+  constexpr int BT = 32 * TT, BN = 32 * TN;  // tokens, rows of W
+  __shared__ __align__(16) uint16_t xs[2][BT * 64];
+  __shared__ __align__(16) uint16_t wsh[2][BN * 64];
+  __shared__ float rstd_s[NORM ? BT : 1];
+  __shared__ int last;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wt = wave & 1, wn = wave >> 1;
+  const int lane = threadIdx.x & 63, r = lane & 15, q4 = lane >> 4;
+  const int tile0 = blockIdx.x * (2 * TN), t_base = blockIdx.y * BT;
+  const int unit0 = blockIdx.z * a.units;
+  const int n = min(a.units, (a.K >> 6) - unit0);
+
+  // this thread's chunk of rows (tid / 8) + 32 i
+  const int row0 = threadIdx.x >> 3, ch = threadIdx.x & 7;
+  const int lds_at = row0 * 64 + ((ch ^ (row0 & 7)) << 3);
+  const uint16_t *xp[TT], *wp[TN];
+#pragma unroll
+  for (int i = 0; i < TT; ++i)
+    xp[i] = a.x + (int64_t)min(t_base + row0 + 32 * i, a.T - 1) * a.x_st + 64 * unit0 + 8 * ch;
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    const int wr = row0 + 32 * i;
+    wp[i] = a.w + (int64_t)linear_row<EPI>(a, min(tile0 + (wr >> 4), a.tiles - 1), wr & 15) * a.K + 64 * unit0 + 8 * ch;
+  }
+  const uint16_t* np = NORM ? a.norm_w + 64 * unit0 + 8 * ch : nullptr;
+
+  struct Stage {
+    u32x4 x[TT], w[TN], nw;
+  };
+  Stage ring[NR];
+  auto load = [&](Stage& s, int k) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i) s.w[i] = *(const u32x4*)(wp[i] + 64 * k);
+#pragma unroll
+    for (int i = 0; i < TT; ++i) s.x[i] = *(const u32x4*)(xp[i] + 64 * k);
+    if (NORM) s.nw = *(const u32x4*)(np + 64 * k);
+  };
+  float ss[TT];
+  f32x4 acc[TN][TT];
+#pragma unroll
+  for (int j = 0; j < TT; ++j) {
+    ss[j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < TN; ++i) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // One step: the slot's operands into LDS buffer b, then (after the caller's next loads) the barrier and the products.
+  // A buffer is written again two steps on, behind a barrier that every wave passes after its reads of it.
+  auto stage = [&](Stage& s, int b) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i) *(u32x4*)(wsh[b] + lds_at + 32 * 64 * i) = s.w[i];
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+      u32x4 v = s.x[i];
+      if (NORM) v = scale_channels(v, s.nw, ss[i]);
+      *(u32x4*)(xs[b] + lds_at + 32 * 64 * i) = v;
     }
+  };
+  auto multiply = [&](int b) {
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int at = r * 64 + (((4 * h + q4) ^ (r & 7)) << 3);
+      bf16x8 wf[TN], xf[TT];
+#pragma unroll
+      for (int i = 0; i < TN; ++i) wf[i] = *(const bf16x8*)(wsh[b] + (wn * TN + i) * 16 * 64 + at);
+#pragma unroll
+      for (int j = 0; j < TT; ++j) xf[j] = *(const bf16x8*)(xs[b] + (wt * TT + j) * 16 * 64 + at);
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[j], acc[i][j], 0, 0, 0);
+    }
+  };
+  // NR steps in flight; the steady state refills every slot unconditionally, so the compiler's waits are exact there.
+#pragma unroll
+  for (int j = 0; j < NR; ++j) load(ring[j], min(j, n - 1));
+  int k = 0;
+  for (; k + 2 * NR <= n; k += NR) {
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+      stage(ring[j], j & 1);
+      load(ring[j], k + j + NR);
+      multiply(j & 1);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NR; ++j)
+    if (k + j < n) {  // uniform over the workgroup
+      stage(ring[j], j & 1);
+      if (k + j + NR < n) load(ring[j], k + j + NR);
+      multiply(j & 1);
+    }
+#pragma unroll
+  for (int j = 0; j < NR; ++j)
+    if (k + NR + j < n) {
+      stage(ring[j], j & 1);
+      multiply(j & 1);
+    }
+
+  if (NORM) {
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+      float s = ss[i];
+      s += __shfl_xor(s, 1);
+      s += __shfl_xor(s, 2);
+      s += __shfl_xor(s, 4);
+      if (ch == 0) rstd_s[row0 + 32 * i] = rsqrtf(s / (float)a.K + a.eps);
+    }
+    __syncthreads();
+  }
+
+  if (EPI == kEpiResidual && a.splits > 1) {
+    // Split K: the sums go through to memory, and the last workgroup to arrive adds them in split order (the split
+    // merge of the decode kernels: stores complete, then a relaxed counter).
+    const int pair = blockIdx.y * gridDim.x + blockIdx.x;
+    float* const part = a.part + (int64_t)pair * a.splits * (BT * BN);
+    const auto rows = __builtin_amdgcn_make_buffer_rsrc(part, (short)0, a.splits * BT * BN * 4, 0x00020000);
+    const auto at = [&](int sp, int i, int j) { return (((sp * TN + i) * TT + j) * 256 + (int)threadIdx.x) * 16; };
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TT; ++j)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), rows, at(blockIdx.z, i, j), 0,
+                                               kAuxSc1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0)
@@ -207,102 +327,134 @@ __global__ void __launch_bounds__(64 * WV) skinny_linear(const LinearArgs a) {
              a.splits - 1;
     __syncthreads();
     if (!last) return;
-    const auto rows = __builtin_amdgcn_make_buffer_rsrc(part, (short)0, a.splits * E * 4, 0x00020000);
-    for (int e = threadIdx.x; e < E; e += 64 * WV) {
-      float s = 0.f;
-      for (int v0 = 0; v0 < a.splits; v0 += 4) {
-        float x[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          x[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                               rows, (min(v0 + u, a.splits - 1) * E + e) * 4, 0, kAuxSc1));
-#pragma unroll
-        for (int u = 0; u < 4; ++u) s += v0 + u < a.splits ? x[u] : 0.f;
-      }
-      flat[e] = s;
-#pragma unroll
-      for (int v = 1; v < WV; ++v) flat[v * E + e] = 0.f;
-    }
     if (threadIdx.x == 0)
       __hip_atomic_store(a.counters + pair, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int sp = 0; sp < a.splits; ++sp)
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TT; ++j)
+          acc[i][j] += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, at(sp, i, j), 0, kAuxSc1));
   }
 
-  // Pairs (n, n + 8) of a tile's outputs for one token; eight neighbouring threads store eight neighbouring channels.
-  for (int p = threadIdx.x; p < RT * TT * 128; p += 64 * WV) {
-    const int n = p & 7, tl = (p >> 3) & 15, j = (p >> 7) % TT, i = p / (128 * TT);
-    const int t = t_base + 16 * j + tl, tile = tile0 + i;
-    if (t >= a.T || tile >= a.tiles) continue;
-    const int at = ((n >> 2) * 16 + tl) * 4 + (n & 3);  // output n's place; n + 8 is 128 words on
-    float lo = 0.f, hi = 0.f;
+  auto unpack = [](uint2 u) {
+    return f32x4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                 __uint_as_float(u.y & 0xffff0000u)};
+  };
 #pragma unroll
-    for (int v = 0; v < WV; ++v) {
-      lo += red[v][i][j][at];
-      hi += red[v][i][j][at + 128];
-    }
-    if (NORM) {
-      float s = 0.f;
+  for (int i = 0; i < TN; ++i) {
+    const int tile = tile0 + wn * TN + i;
+    const bool in = tile < a.tiles;
+    const int c = linear_row<EPI>(a, min(tile, a.tiles - 1), 4 * q4);  // this lane's 4 channels: c .. c + 3
 #pragma unroll
-      for (int v = 0; v < WV; ++v) s += ssq[v][16 * j + tl];
-      const float rstd = rsqrtf(s / (float)a.K + a.eps);
-      lo *= rstd;
-      hi *= rstd;
+    for (int j = 0; j < TT; ++j) {
+      const int tl = (wt * TT + j) * 16 + r, t = t_base + tl;
+      f32x4 v = acc[i][j];
+      if (NORM) v *= rstd_s[tl];
+      if (EPI == kEpiSilu) {
+        // Lanes q4 < 2 hold four gate channels, their partners the up channels: each side gives the other half of its
+        // own and finishes two channels.
+        const bool gate = q4 < 2;
+        const float s0 = __shfl_xor(gate ? v[2] : v[0], 32), s1 = __shfl_xor(gate ? v[3] : v[1], 32);
+        const float g0 = gate ? v[0] : s0, g1 = gate ? v[1] : s1, u0 = gate ? s0 : v[2], u1 = gate ? s1 : v[3];
+        if (in && t < a.T)
+          *(uint32_t*)(a.out + t * a.out_st + tile * 8 + 4 * (q4 & 1) + (gate ? 0 : 2)) =
+              pack_bf16x2(silu(g0) * u0, silu(g1) * u1);
+        continue;
+      } else {
+        if (a.bias != nullptr) v += unpack(*(const uint2*)(a.bias + c));
+        if (EPI == kEpiRope && tile * 16 < a.rot) {
+          f32x4 u;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) u[e] = __shfl_xor(v[e], 32);
+          const int64_t at = (int64_t)min(t, a.T - 1) * a.D + c % a.D;
+          v = v * unpack(*(const uint2*)(a.cos + at)) + u * unpack(*(const uint2*)(a.sin + at));
+        }
+        if (EPI == kEpiResidual && a.res != nullptr && t < a.T) v += unpack(*(const uint2*)(a.res + t * a.res_st + c));
+      }
+      if (!in || t >= a.T) continue;
+      *(uint2*)(a.out + t * a.out_st + c) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
     }
-    const int nlo = linear_row<EPI>(a, tile, n), nhi = linear_row<EPI>(a, tile, n + 8);
-    if (EPI == kEpiSilu) {
-      a.out[t * a.out_st + nlo] = f32_to_bf16_bits(lo / (1.f + expf(-lo)) * hi);
-      continue;
-    }
-    if (a.bias != nullptr) {
-      lo += bf16_bits_to_f32(a.bias[nlo]);
-      hi += bf16_bits_to_f32(a.bias[nhi]);
-    }
-    if (EPI == kEpiRope && tile * 16 < a.rot) {
-      const int c = nlo % a.D, c2 = c + (a.D >> 1);
-      const uint16_t *cs = a.cos + (int64_t)t * a.D, *sn = a.sin + (int64_t)t * a.D;
-      const float x0 = lo, x1 = hi;
-      lo = x0 * bf16_bits_to_f32(cs[c]) + x1 * bf16_bits_to_f32(sn[c]);
-      hi = x1 * bf16_bits_to_f32(cs[c2]) + x0 * bf16_bits_to_f32(sn[c2]);
-    }
-    if (EPI == kEpiResidual && a.res != nullptr) {
-      lo += bf16_bits_to_f32(a.res[t * a.res_st + nlo]);
-      hi += bf16_bits_to_f32(a.res[t * a.res_st + nhi]);
-    }
-    a.out[t * a.out_st + nlo] = f32_to_bf16_bits(lo);
-    a.out[t * a.out_st + nhi] = f32_to_bf16_bits(hi);
   }
 }
 
-template <int EPI, bool NORM, int TT, int RT, int WV, int U, int NST>
-static void launch_linear(LinearArgs& a, hipStream_t st) {
-  const dim3 grid((a.tiles + RT - 1) / RT, (a.T + 16 * TT - 1) / (16 * TT), a.splits);
-  skinny_linear<EPI, NORM, TT, RT, WV, U, NST><<<grid, 64 * WV, 0, st>>>(a);
+template <int EPI, bool NORM, int TT, int TN, int NR>
+static void launch_tile(const LinearArgs& a, hipStream_t st) {
+  const dim3 grid((a.tiles + 2 * TN - 1) / (2 * TN), (a.T + 32 * TT - 1) / (32 * TT), a.splits);
+  tile_linear<EPI, NORM, TT, TN, NR><<<grid, 256, 0, st>>>(a);
+}
+
+// Tile shapes of tile_linear by number: tokens and rows of W.
+struct TileShape {
+  int tokens, rows;
+};
+constexpr TileShape kTiles[] = {{32, 32}, {32, 64}, {64, 64}, {64, 128}, {128, 128}};
+constexpr int kNumTiles = 5, kSkinny = kNumTiles;
+
+struct LinearPlan {
+  int shape;   // index into kTiles, or kSkinny
+  int splits;  // workgroups that share a tile's K
+  int64_t part_bytes;
+  int64_t counters;
+};
+
+// The smallest tile whose grid stays within a number of workgroups that depends on the epilogue: small tiles fill the
+// chip, large ones read less. Measured at 8 to 1024 tokens on both model shapes; the rule is within 8% of the best tile
+// in all but two of 56 cases (1.5B gate/up at 64 tokens 20.6 us here, 24.4 one tile smaller; QKV 0.5B at 544 tokens 9.6
+// with 612 small workgroups, 10.9 with 162). ROPE: 640 (K is short and the tiles' norm is their cost). SILU: 200 (every
+// workgroup reads its own 57 to 230 KB of W; from 32 x 64 on). RESIDUAL: 256, and a K from 4096 on is then split until
+// the grid has about 256 again, at most six ways (the merge: 896 x 4864 at 8 tokens 7.5 us with six, 8.0 with eight,
+// 11.5 with one). num_splits and shape of the caller come first (0: the rule).
+static LinearPlan plan_linear(int epi, bool norm, int T, int tiles, int K, int want_splits, int want_shape) {
+  LinearPlan p{};
+  const int units = K >> 6;
+  auto grid = [&](int s) {
+    return (int64_t)((16 * tiles + kTiles[s].rows - 1) / kTiles[s].rows) * ((T + kTiles[s].tokens - 1) / kTiles[s].tokens);
+  };
+  if (want_shape > 0) {
+    p.shape = want_shape - 1;
+  } else if (T <= 16 && units <= 24 && tiles <= 256 && want_splits <= 1) {
+    p.shape = kSkinny;
+  } else {
+    const int most = epi == kEpiRope ? 640 : epi == kEpiSilu ? 200 : 256;
+    p.shape = epi == kEpiSilu ? 1 : 0;
+    while (p.shape + 1 < kNumTiles && grid(p.shape) > most) ++p.shape;
+  }
+  p.splits = 1;
+  if (p.shape != kSkinny && epi == kEpiResidual && !norm) {
+    const int64_t g = grid(p.shape);
+    if (want_splits > 0)
+      p.splits = want_splits;
+    else if (K >= 4096 && g * 5 <= 4 * 256)
+      p.splits = (int)std::min<int64_t>(6, (256 + g - 1) / g);
+    const int per = (units + p.splits - 1) / p.splits;
+    p.splits = (units + per - 1) / per;
+    if (p.splits > 1) {
+      p.part_bytes = g * p.splits * kTiles[p.shape].tokens * kTiles[p.shape].rows * 4;
+      p.counters = g;
+    }
+  }
+  return p;
 }
 
 template <int EPI, bool NORM>
-static void dispatch_linear(LinearArgs& a, hipStream_t st) {
-  const int units = a.K >> 6;
-  a.units = (units + a.splits - 1) / a.splits;
-  a.splits = (units + a.units - 1) / a.units;
-  if (a.T <= 16) {
-    if (a.units <= 16) return launch_linear<EPI, NORM, 1, 1, 8, 2, 1>(a, st);
-    if (a.units <= 24) return launch_linear<EPI, NORM, 1, 1, 8, 3, 1>(a, st);
-    if constexpr (!NORM) {
-      if (a.units >= 64) return launch_linear<EPI, NORM, 1, 1, 16, 2, 2>(a, st);
-    }
-    return launch_linear<EPI, NORM, 1, 1, 8, 2, 2>(a, st);
+static void launch_linear(const LinearArgs& a, int shape, hipStream_t st) {
+  switch (shape) {
+    case 0: return launch_tile<EPI, NORM, 1, 1, 4>(a, st);
+    case 1: return launch_tile<EPI, NORM, 1, 2, 4>(a, st);
+    case 2: return launch_tile<EPI, NORM, 2, 2, 4>(a, st);
+    case 3: return launch_tile<EPI, NORM, 2, 4, 4>(a, st);
+    case 4: return launch_tile<EPI, NORM, 4, 4, 2>(a, st);
+    default:
+      if (a.K <= 16 * 64)
+        skinny_linear<EPI, NORM, 2><<<a.tiles, 64 * kSkinnyWaves, 0, st>>>(a);
+      else
+        skinny_linear<EPI, NORM, 3><<<a.tiles, 64 * kSkinnyWaves, 0, st>>>(a);
   }
-  const int tt = a.T <= 32 ? 2 : 4;
-  if (a.tiles >= 512) {  // two row tiles a workgroup share its x loads and still fill the chip
-    if (tt == 2) return launch_linear<EPI, NORM, 2, 2, 8, 1, 2>(a, st);
-    return launch_linear<EPI, NORM, 4, 2, 8, 1, 2>(a, st);
-  }
-  if (a.units <= 16) {
-    if (tt == 2) return launch_linear<EPI, NORM, 2, 1, 8, 2, 1>(a, st);
-    return launch_linear<EPI, NORM, 4, 1, 8, 2, 1>(a, st);
-  }
-  if (tt == 2) return launch_linear<EPI, NORM, 2, 1, 8, NORM ? 1 : 2, 2>(a, st);
-  return launch_linear<EPI, NORM, 4, 1, 8, NORM ? 1 : 2, 2>(a, st);
 }
 
 // ---- the elementwise operations alone (large batches) -----------------------------------------------------------------
@@ -402,12 +554,13 @@ __global__ void __launch_bounds__(256) silu_mul_kernel(const uint16_t* __restric
   for (int i = 0; i < 4; ++i) {
     const float g0 = __uint_as_float(g[i] << 16), g1 = __uint_as_float(g[i] & 0xffff0000u);
     const float u0 = __uint_as_float(u[i] << 16), u1 = __uint_as_float(u[i] & 0xffff0000u);
-    o[i] = pack_bf16x2(g0 / (1.f + expf(-g0)) * u0, g1 / (1.f + expf(-g1)) * u1);
+    o[i] = pack_bf16x2(silu(g0) * u0, silu(g1) * u1);
   }
   *(u32x4*)(out + t * out_st + c) = o;
 }
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+static bool aligned8(const void* p) { return ((uintptr_t)p & 7) == 0; }
 
 static int launched(const char* what) {
   const hipError_t e = hipGetLastError();
@@ -418,20 +571,60 @@ static int launched(const char* what) {
 
 using namespace sipa;
 
-extern "C" int32_t sipa_fused_linear(const sipa_linear_params* p, void* stream) {
+static int check_linear(const sipa_linear_params* p) {
   SIPA_CHECK(p != nullptr && p->struct_size == (int32_t)sizeof(sipa_linear_params), SIPA_EINVAL,
              "sipa_linear_params: wrong size");
-  SIPA_CHECK(p->num_tokens >= 0 && p->in_features > 0 && p->out_features > 0, SIPA_EINVAL, "linear: bad sizes");
+  const int T = p->num_tokens, K = p->in_features, N = p->out_features;
+  SIPA_CHECK(T >= 0 && K > 0 && N > 0, SIPA_EINVAL, "linear: bad sizes");
+  SIPA_CHECK(T <= 1 << 20 && N <= 1 << 22 && K <= 1 << 20, SIPA_EUNSUPPORTED, "linear: sizes out of range");
+  SIPA_CHECK(K % 64 == 0, SIPA_EUNSUPPORTED, "linear: in_features %d is not a multiple of 64", K);
+  SIPA_CHECK(N % 16 == 0, SIPA_EUNSUPPORTED, "linear: out_features %d is not a multiple of 16", N);
+  SIPA_CHECK(p->epilogue >= SIPA_LINEAR_RESIDUAL && p->epilogue <= SIPA_LINEAR_SILU, SIPA_EINVAL, "linear: epilogue %d",
+             p->epilogue);
+  SIPA_CHECK(p->tile >= 0 && p->tile <= kNumTiles + 1 && p->num_splits >= 0 && p->num_splits <= 64, SIPA_EINVAL,
+             "linear: tile %d, %d splits", p->tile, p->num_splits);
+  SIPA_CHECK(p->tile != kSkinny + 1 || (T <= 16 && K <= 24 * 64 && p->num_splits <= 1), SIPA_EUNSUPPORTED,
+             "linear: the skinny kernel takes up to 16 tokens and %d in_features, unsplit", 24 * 64);
+  if (p->epilogue == SIPA_LINEAR_ROPE) {
+    SIPA_CHECK(p->head_dim > 0 && p->head_dim % 16 == 0, SIPA_EUNSUPPORTED, "linear: heads of %d channels", p->head_dim);
+    SIPA_CHECK(p->rot_channels >= 0 && p->rot_channels <= N && p->rot_channels % p->head_dim == 0, SIPA_EINVAL,
+               "linear: %d rotated channels", p->rot_channels);
+  }
+  SIPA_CHECK(p->num_splits <= 1 || (p->epilogue == SIPA_LINEAR_RESIDUAL && p->norm_weight == nullptr), SIPA_EINVAL,
+             "linear: only the residual epilogue without norm splits K");
+  return SIPA_OK;
+}
+
+static LinearPlan plan_of(const sipa_linear_params* p) {
+  const int tiles = p->out_features / 16;  // SILU: 8 gate and 8 up rows each
+  return plan_linear(p->epilogue, p->norm_weight != nullptr, p->num_tokens, tiles, p->in_features, p->num_splits,
+                     p->tile);
+}
+
+extern "C" int64_t sipa_linear_scratch_bytes(const sipa_linear_params* p) {
+  const int rc = check_linear(p);
+  if (rc != SIPA_OK) return rc;
+  return p->num_tokens == 0 ? 0 : plan_of(p).part_bytes;
+}
+
+extern "C" int32_t sipa_fused_linear(const sipa_linear_params* p, void* stream) {
+  const int rc = check_linear(p);
+  if (rc != SIPA_OK) return rc;
   if (p->num_tokens == 0) return SIPA_OK;
-  SIPA_CHECK(p->num_tokens <= 1 << 20 && p->out_features <= 1 << 24 && p->in_features <= 1 << 20, SIPA_EUNSUPPORTED,
-             "linear: sizes out of range");
-  SIPA_CHECK(p->in_features % 64 == 0, SIPA_EUNSUPPORTED, "linear: in_features %d is not a multiple of 64",
-             p->in_features);
   SIPA_CHECK(p->x && p->weight && p->out, SIPA_EINVAL, "linear: null pointer");
   SIPA_CHECK(aligned16(p->x) && aligned16(p->weight) && aligned16(p->norm_weight) && p->x_stride % 8 == 0,
              SIPA_EUNSUPPORTED, "linear: x, weight and norm weight need 16-byte rows");
+  SIPA_CHECK(aligned8(p->bias) && aligned8(p->residual) && aligned8(p->out) && aligned8(p->rot_cos) &&
+                 aligned8(p->rot_sin) && p->res_stride % 4 == 0 && p->out_stride % 4 == 0,
+             SIPA_EUNSUPPORTED, "linear: bias, residual, rotary tables and out need 8-byte rows");
   SIPA_CHECK(p->x_stride >= 0 && p->out_stride >= 0 && p->res_stride >= 0, SIPA_EINVAL, "linear: negative stride");
   SIPA_CHECK(p->norm_weight == nullptr || p->eps >= 0.f, SIPA_EINVAL, "linear: eps");
+  SIPA_CHECK(p->epilogue == SIPA_LINEAR_RESIDUAL || p->residual == nullptr, SIPA_EINVAL,
+             "linear: only the residual epilogue takes a residual");
+  SIPA_CHECK(p->epilogue != SIPA_LINEAR_SILU || p->bias == nullptr, SIPA_EINVAL, "linear: no bias with SiLU");
+  SIPA_CHECK(p->epilogue != SIPA_LINEAR_ROPE || p->rot_channels == 0 || (p->rot_cos && p->rot_sin), SIPA_EINVAL,
+             "linear: rotary tables missing");
+  const LinearPlan plan = plan_of(p);
   LinearArgs a{};
   a.x = (const uint16_t*)p->x, a.x_st = p->x_stride, a.w = (const uint16_t*)p->weight;
   a.norm_w = (const uint16_t*)p->norm_weight, a.eps = p->eps, a.bias = (const uint16_t*)p->bias;
@@ -439,45 +632,94 @@ extern "C" int32_t sipa_fused_linear(const sipa_linear_params* p, void* stream) 
   a.out = (uint16_t*)p->out, a.out_st = p->out_stride;
   a.cos = (const uint16_t*)p->rot_cos, a.sin = (const uint16_t*)p->rot_sin;
   a.T = p->num_tokens, a.K = p->in_features, a.D = p->head_dim;
-  a.splits = 1;
-  if (p->num_splits > 1) {
-    SIPA_CHECK(p->epilogue == SIPA_LINEAR_RESIDUAL && p->norm_weight == nullptr, SIPA_EINVAL,
-               "linear: only the residual epilogue without norm splits K");
-    SIPA_CHECK(p->num_splits <= 64 && p->part && p->counters, SIPA_EWORKSPACE, "linear: split buffers missing");
-    a.splits = p->num_splits, a.part = (float*)p->part, a.counters = (int32_t*)p->counters;
+  a.tiles = p->out_features / 16, a.inter = p->out_features / 2;
+  a.rot = p->epilogue == SIPA_LINEAR_ROPE ? p->rot_channels : 0;
+  a.splits = plan.splits;
+  const int units = a.K >> 6;
+  a.units = (units + a.splits - 1) / a.splits;
+  if (plan.splits > 1) {
+    SIPA_CHECK(p->scratch != nullptr && p->scratch_bytes >= plan.part_bytes && aligned16(p->scratch) && p->counters,
+               SIPA_EWORKSPACE, "linear: %lld bytes of scratch needed for %d splits", (long long)plan.part_bytes,
+               plan.splits);
+    SIPA_CHECK(plan.counters <= kMaxCounters, SIPA_EUNSUPPORTED, "linear: %lld tiles exceed the %d merge counters",
+               (long long)plan.counters, kMaxCounters);
+    a.part = (float*)p->scratch, a.counters = (int32_t*)p->counters;
   }
   const hipStream_t st = (hipStream_t)stream;
-  const int N = p->out_features;
-  switch (p->epilogue) {
-    case SIPA_LINEAR_RESIDUAL:
-      SIPA_CHECK(N % 16 == 0, SIPA_EUNSUPPORTED, "linear: out_features %d is not a multiple of 16", N);
-      a.tiles = N / 16;
-      if (a.norm_w) dispatch_linear<kEpiResidual, true>(a, st);
-      else dispatch_linear<kEpiResidual, false>(a, st);
-      break;
-    case SIPA_LINEAR_ROPE:
-      SIPA_CHECK(N % 16 == 0 && a.D > 0 && a.D % 16 == 0, SIPA_EUNSUPPORTED, "linear: heads of %d channels", a.D);
-      SIPA_CHECK(p->rot_channels >= 0 && p->rot_channels <= N && p->rot_channels % a.D == 0, SIPA_EINVAL,
-                 "linear: %d rotated channels", p->rot_channels);
-      SIPA_CHECK(p->rot_channels == 0 || (a.cos && a.sin), SIPA_EINVAL, "linear: rotary tables missing");
-      SIPA_CHECK(p->residual == nullptr, SIPA_EINVAL, "linear: no residual with the rotary epilogue");
-      a.rot = p->rot_channels;
-      a.tiles = N / 16;
-      if (a.norm_w) dispatch_linear<kEpiRope, true>(a, st);
-      else dispatch_linear<kEpiRope, false>(a, st);
-      break;
-    case SIPA_LINEAR_SILU:
-      SIPA_CHECK(N % 16 == 0, SIPA_EUNSUPPORTED, "linear: out_features %d is not a multiple of 16", N);
-      SIPA_CHECK(p->residual == nullptr && p->bias == nullptr, SIPA_EINVAL, "linear: no residual or bias with SiLU");
-      a.inter = N / 2;
-      a.tiles = a.inter / 8;
-      if (a.norm_w) dispatch_linear<kEpiSilu, true>(a, st);
-      else dispatch_linear<kEpiSilu, false>(a, st);
-      break;
-    default:
-      return fail(SIPA_EINVAL, "linear: epilogue %d", p->epilogue);
+  switch (p->epilogue * 2 + (a.norm_w != nullptr)) {
+    case 0: launch_linear<kEpiResidual, false>(a, plan.shape, st); break;
+    case 1: launch_linear<kEpiResidual, true>(a, plan.shape, st); break;
+    case 2: launch_linear<kEpiRope, false>(a, plan.shape, st); break;
+    case 3: launch_linear<kEpiRope, true>(a, plan.shape, st); break;
+    case 4: launch_linear<kEpiSilu, false>(a, plan.shape, st); break;
+    default: launch_linear<kEpiSilu, true>(a, plan.shape, st); break;
   }
   return launched("linear");
+}
+
+// The three projections of sipa_layer_out over its scratch: h, the gated activations, then one split's partial sums at
+// a time.
+static int layer_out_parts(const sipa_layer_out_params* p, sipa_linear_params (&l)[3], int64_t* bytes) {
+  SIPA_CHECK(p != nullptr && p->struct_size == (int32_t)sizeof(sipa_layer_out_params), SIPA_EINVAL,
+             "sipa_layer_out_params: wrong size");
+  SIPA_CHECK(p->num_tokens >= 0 && p->num_tokens <= 1 << 20 && p->hidden > 0 && p->hidden <= 1 << 20 && p->inter > 0 &&
+                 p->inter <= 1 << 20,
+             SIPA_EINVAL, "layer: bad sizes");
+  auto align = [](int64_t n) { return (n + 255) & ~(int64_t)255; };
+  const int64_t h_bytes = align((int64_t)p->num_tokens * p->hidden * 2);
+  const int64_t act_bytes = align((int64_t)p->num_tokens * p->inter * 2);
+  char* const base = (char*)p->scratch;
+  char* const h = base;
+  char* const act = base == nullptr ? nullptr : base + h_bytes;
+  for (auto& q : l) {
+    q = sipa_linear_params{};
+    q.struct_size = sizeof(q);
+    q.num_tokens = p->num_tokens;
+    q.scratch = base == nullptr ? nullptr : act + act_bytes;
+    q.scratch_bytes = p->scratch_bytes - h_bytes - act_bytes;
+    q.counters = p->counters;
+  }
+  l[0].epilogue = SIPA_LINEAR_RESIDUAL, l[0].in_features = p->attn_features, l[0].out_features = p->hidden;
+  l[0].x = p->attn, l[0].x_stride = p->attn_stride, l[0].weight = p->o_w, l[0].residual = p->x;
+  l[0].res_stride = p->x_stride, l[0].out = h, l[0].out_stride = p->hidden;
+  l[1].epilogue = SIPA_LINEAR_SILU, l[1].in_features = p->hidden, l[1].out_features = 2 * p->inter, l[1].eps = p->eps;
+  l[1].x = h, l[1].x_stride = p->hidden, l[1].weight = p->gate_up_w, l[1].norm_weight = p->post_norm;
+  l[1].out = act, l[1].out_stride = p->inter;
+  l[2].epilogue = SIPA_LINEAR_RESIDUAL, l[2].in_features = p->inter, l[2].out_features = p->hidden;
+  l[2].x = act, l[2].x_stride = p->inter, l[2].weight = p->down_w, l[2].residual = h, l[2].res_stride = p->hidden;
+  l[2].out = p->out, l[2].out_stride = p->hidden;
+  int64_t part = 0;
+  for (const auto& q : l) {
+    const int64_t b = sipa_linear_scratch_bytes(&q);
+    if (b < 0) return (int)b;
+    part = std::max(part, b);
+  }
+  *bytes = h_bytes + act_bytes + part;
+  return SIPA_OK;
+}
+
+extern "C" int64_t sipa_layer_out_scratch_bytes(const sipa_layer_out_params* p) {
+  sipa_linear_params l[3];
+  int64_t bytes = 0;
+  const int rc = layer_out_parts(p, l, &bytes);
+  return rc != SIPA_OK ? rc : bytes;
+}
+
+extern "C" int32_t sipa_layer_out(const sipa_layer_out_params* p, void* stream) {
+  sipa_linear_params l[3];
+  int64_t bytes = 0;
+  const int rc = layer_out_parts(p, l, &bytes);
+  if (rc != SIPA_OK) return rc;
+  if (p->num_tokens == 0) return SIPA_OK;
+  SIPA_CHECK(p->x && p->attn && p->o_w && p->post_norm && p->gate_up_w && p->down_w && p->out && p->counters,
+             SIPA_EINVAL, "layer: null pointer");
+  SIPA_CHECK(p->scratch != nullptr && p->scratch_bytes >= bytes && ((uintptr_t)p->scratch & 255) == 0, SIPA_EWORKSPACE,
+             "layer: %lld bytes of 256-byte aligned scratch needed", (long long)bytes);
+  for (const auto& q : l) {
+    const int r = sipa_fused_linear(&q, stream);
+    if (r != SIPA_OK) return r;
+  }
+  return SIPA_OK;
 }
 
 extern "C" int32_t sipa_rms_norm(const void* x, int64_t x_stride, const void* add, int64_t add_stride,

@@ -9,6 +9,7 @@ Each function takes bf16 GPU tensors with a contiguous last dimension, unchecked
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 import torch.nn.functional as F
@@ -17,13 +18,14 @@ from . import _hip
 from .hip_decode import reserve_workspace
 
 RESIDUAL, ROPE, SILU = 0, 1, 2  # SIPA_LINEAR_*
-# Up to here the projections run fused_linear; larger batches go to the GEMM library with the fused operations around
-# it. At 32 tokens (0.5B layer, us) 33 against 51; at 64, 46 against 56 with the gated projection alone slower, at 128
-# 60 against 52.
-MAX_TOKENS = 32
-# From here on four workgroups share a row tile's K: 11.6 -> 7.0 us at 896 x 4864 and 8 tokens, 19.1 -> 12.9 at
-# 1536 x 8960; at 896 x 896 the merge would cost more than the rows' whole read.
-SPLIT_FEATURES = 4096
+
+# Up to here a layer's projections run the fused kernels; larger batches go to the GEMM library with the fused
+# operations around it. A 0.5B layer's projections and what they fuse (us, fused against library): 64 tokens 29 / 54,
+# 256 41 / 59, 544 57 / 64, 1024 81 / 84.
+MAX_TOKENS = 1024
+# The gated projection goes to the library above this many operations, where its large tiles are better: 0.5B at 1024
+# tokens (17.9 GFLOP) 37.9 us against 27.3 + norm and SwiGLU (10), 1.5B at 256 (14.1) 40.6 / 39, at 544 (30) 61.8 / 47.
+MAX_GATED_FLOPS = 18e9
 
 
 def _ok(t, device: torch.device, dim: int) -> bool:
@@ -58,27 +60,39 @@ def supported(x: torch.Tensor, w, rot, heads: int, head_dim: int) -> bool:
             _ok(sin, dev, 3) and tuple(sin.shape) == (T, 1, head_dim))
 
 
+@functools.lru_cache(maxsize=1024)
+def _linear_scratch(epilogue: int, norm: bool, T: int, K: int, N: int, head_dim: int, num_splits: int, tile: int) -> int:
+    p = _hip.LinearParams(struct_size=ctypes.sizeof(_hip.LinearParams), epilogue=epilogue, num_tokens=T, in_features=K,
+                          out_features=N, head_dim=head_dim, norm_weight=16 if norm else None, num_splits=num_splits,
+                          tile=tile)
+    n = _hip.lib().sipa_linear_scratch_bytes(ctypes.byref(p))
+    if n < 0:
+        _hip.check(n, "fused_linear")
+    return n
+
+
 def fused_linear(x: torch.Tensor, weight: torch.Tensor, epilogue: int, *, norm_weight: torch.Tensor | None = None,
                  eps: float = 0.0, bias: torch.Tensor | None = None, residual: torch.Tensor | None = None,
-                 rot: tuple[torch.Tensor, torch.Tensor] | None = None, head_dim: int = 0,
-                 rot_channels: int = 0, num_splits: int = 1) -> torch.Tensor:
+                 rot: tuple[torch.Tensor, torch.Tensor] | None = None, head_dim: int = 0, rot_channels: int = 0,
+                 num_splits: int = 0, tile: int = 0) -> torch.Tensor:
     """epilogue(norm(x) W^T) in one launch (sipa_fused_linear): x [T, K], weight [N, K]; RESIDUAL adds bias and
     residual, ROPE adds bias and rotates the first rot_channels channels by rot = (cos, signed sin), SILU multiplies
-    the second half of the channels by silu of the first."""
+    the second half of the channels by silu of the first. num_splits, tile: 0 for the library's choice."""
     T, K = x.shape
     N = weight.shape[0]
     out = torch.empty(T, N // 2 if epilogue == SILU else N, device=x.device, dtype=torch.bfloat16)
-    part = counters = None
-    if num_splits > 1:
-        groups = 1 if T <= 16 else 2 if T <= 32 else 4 * -(-T // 64)
-        part = torch.empty(N // 16 * groups * num_splits * 256, device=x.device, dtype=torch.float32)
-        counters = reserve_workspace(x.device, _hip.stream_of(x), 0)
+    stream = _hip.stream_of(x)
+    n = _linear_scratch(epilogue, norm_weight is not None, T, K, N, head_dim, num_splits, tile)
+    scratch = counters = None
+    if n:
+        scratch = torch.empty(n, device=x.device, dtype=torch.uint8)
+        counters = reserve_workspace(x.device, stream, 0).data_ptr()
     p = _hip.LinearParams(ctypes.sizeof(_hip.LinearParams), epilogue, T, K, N, head_dim, rot_channels, eps,
                           x.data_ptr(), x.stride(0), weight.data_ptr(), _hip.ptr(norm_weight), _hip.ptr(bias),
                           _hip.ptr(residual), residual.stride(0) if residual is not None else 0, out.data_ptr(),
                           out.stride(0), *((rot[0].data_ptr(), rot[1].data_ptr()) if rot is not None else (None, None)),
-                          num_splits, _hip.ptr(part), _hip.ptr(counters))
-    _hip.check(_hip.lib().sipa_fused_linear(ctypes.byref(p), _hip.stream_of(x)), "fused_linear")
+                          num_splits, tile, _hip.ptr(scratch), n, counters)
+    _hip.check(_hip.lib().sipa_fused_linear(ctypes.byref(p), stream), "fused_linear")
     return out
 
 
@@ -110,7 +124,7 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
 
 def layer_qkv(x: torch.Tensor, w, eps: float, rot, rotated: int, head_dim: int) -> torch.Tensor:
     """[T, heads * head_dim]: the fused projection of the normalised x, its first `rotated` heads (queries and keys)
-    rotated. One launch for a few tokens."""
+    rotated. One launch up to MAX_TOKENS."""
     if x.shape[0] <= MAX_TOKENS:
         return fused_linear(x, w.qkv_w, ROPE, norm_weight=w.input_norm, eps=eps, bias=w.qkv_b, rot=rot,
                             head_dim=head_dim, rot_channels=rotated * head_dim)
@@ -119,12 +133,33 @@ def layer_qkv(x: torch.Tensor, w, eps: float, rot, rotated: int, head_dim: int) 
     return qkv
 
 
+@functools.lru_cache(maxsize=1024)
+def _layer_out_scratch(T: int, hidden: int, attn_features: int, inter: int) -> int:
+    p = _hip.LayerOutParams(ctypes.sizeof(_hip.LayerOutParams), T, hidden, attn_features, inter)
+    n = _hip.lib().sipa_layer_out_scratch_bytes(ctypes.byref(p))
+    if n < 0:
+        _hip.check(n, "layer_out")
+    return n
+
+
 def layer_out(x: torch.Tensor, attn: torch.Tensor, w, eps: float) -> torch.Tensor:
-    """x + attn W_o, then that plus its MLP. Three launches for a few tokens."""
-    if x.shape[0] <= MAX_TOKENS:
+    """x + attn W_o, then that plus its MLP: three launches from one call, up to MAX_TOKENS and MAX_GATED_FLOPS."""
+    T, hidden = x.shape
+    inter = w.down_w.shape[1]
+    if T > MAX_TOKENS:
+        n, h = rms_norm(x, w.post_norm, eps, add=F.linear(attn, w.o_w))
+        return h + F.linear(silu_mul(F.linear(n, w.gate_up_w)), w.down_w)
+    if 4.0 * T * hidden * inter > MAX_GATED_FLOPS:
         h = fused_linear(attn, w.o_w, RESIDUAL, residual=x)
-        act = fused_linear(h, w.gate_up_w, SILU, norm_weight=w.post_norm, eps=eps)
-        return fused_linear(act, w.down_w, RESIDUAL, residual=h,
-                            num_splits=4 if w.down_w.shape[1] >= SPLIT_FEATURES else 1)
-    n, h = rms_norm(x, w.post_norm, eps, add=F.linear(attn, w.o_w))
-    return h + F.linear(silu_mul(F.linear(n, w.gate_up_w)), w.down_w)
+        act = silu_mul(F.linear(rms_norm(h, w.post_norm, eps), w.gate_up_w))
+        return fused_linear(act, w.down_w, RESIDUAL, residual=h)
+    out = torch.empty(T, hidden, device=x.device, dtype=torch.bfloat16)
+    stream = _hip.stream_of(x)
+    nbytes = _layer_out_scratch(T, hidden, attn.shape[1], inter)
+    scratch = torch.empty(nbytes, device=x.device, dtype=torch.uint8)
+    p = _hip.LayerOutParams(ctypes.sizeof(_hip.LayerOutParams), T, hidden, attn.shape[1], inter, eps, x.data_ptr(),
+                            x.stride(0), attn.data_ptr(), attn.stride(0), w.o_w.data_ptr(), w.post_norm.data_ptr(),
+                            w.gate_up_w.data_ptr(), w.down_w.data_ptr(), out.data_ptr(), scratch.data_ptr(), nbytes,
+                            reserve_workspace(x.device, stream, 0).data_ptr())
+    _hip.check(_hip.lib().sipa_layer_out(ctypes.byref(p), stream), "layer_out")
+    return out

@@ -320,7 +320,11 @@ def bad_linear(**over):
     (dict(epilogue=3), _hip.EINVAL), (dict(epilogue=1, head_dim=24), _hip.EUNSUPPORTED),
     (dict(epilogue=1, rot_channels=96), _hip.EINVAL), (dict(epilogue=1, rot_channels=64, rot_cos=None), _hip.EINVAL),
     (dict(epilogue=2, bias=4096), _hip.EINVAL), (dict(num_splits=2), _hip.EWORKSPACE),
-    (dict(num_splits=2, part=4096, counters=4096, epilogue=2), _hip.EINVAL), (dict(num_tokens=-1), _hip.EINVAL)])
+    (dict(num_splits=2, scratch=4096, scratch_bytes=64, counters=4096), _hip.EWORKSPACE),
+    (dict(num_splits=2, epilogue=2), _hip.EINVAL), (dict(num_splits=65), _hip.EINVAL), (dict(tile=7), _hip.EINVAL),
+    (dict(tile=6, num_tokens=17), _hip.EUNSUPPORTED), (dict(tile=6, in_features=1600, x_stride=1600), _hip.EUNSUPPORTED),
+    (dict(bias=4100), _hip.EUNSUPPORTED), (dict(residual=4096, res_stride=894), _hip.EUNSUPPORTED),
+    (dict(num_tokens=-1), _hip.EINVAL)])
 def test_fused_linear_refuses_bad_arguments(over, code):
     assert _hip.lib().sipa_fused_linear(ctypes.byref(bad_linear(**over)), None) == code
     assert _hip.lib().sipa_last_error()
@@ -336,3 +340,21 @@ def test_fused_linear_refuses_bad_arguments(over, code):
 ])
 def test_split_policy_where_programs_do_not_divide_the_cus(S, ctx, mode, want):
     assert _hip.lib().sipa_choose_splits_for(S, 2, ctx, 256, mode) == want
+
+
+def test_layer_out_refuses_bad_arguments():
+    lib = _hip.lib()
+    p = _hip.LayerOutParams(ctypes.sizeof(_hip.LayerOutParams), 8, 896, 896, 4864, 1e-6)
+    need = lib.sipa_layer_out_scratch_bytes(ctypes.byref(p))
+    # the hidden states and activations of 8 tokens, and the split sums of 6 x 28 tiles of 32 x 32
+    assert need == 8 * 896 * 2 + 8 * 4864 * 2 + 6 * 28 * 32 * 32 * 4
+    assert lib.sipa_layer_out(ctypes.byref(p), None) == _hip.EINVAL  # no tensors
+    for name in ("x", "attn", "o_w", "post_norm", "gate_up_w", "down_w", "out", "counters", "scratch"):
+        setattr(p, name, 4096)
+    p.x_stride = p.attn_stride = 896
+    p.scratch_bytes = need - 1
+    assert lib.sipa_layer_out(ctypes.byref(p), None) == _hip.EWORKSPACE
+    p.struct_size = 8
+    assert lib.sipa_layer_out_scratch_bytes(ctypes.byref(p)) == _hip.EINVAL
+    p.struct_size, p.inter = ctypes.sizeof(_hip.LayerOutParams), 100
+    assert lib.sipa_layer_out_scratch_bytes(ctypes.byref(p)) == _hip.EUNSUPPORTED

@@ -21,7 +21,7 @@ pytestmark = pytest.mark.gpu
 
 BOUND = 2.0 ** -8
 EPS = 1e-6
-TOKENS = [1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 130]
+TOKENS = [1, 2, 15, 16, 17, 31, 32, 33, 64, 65, 129, 300]
 
 
 def rel(a, b):
@@ -73,8 +73,8 @@ def test_gated_projection(T, inter, hidden):
 
 
 @pytest.mark.parametrize("out_f,in_f", [(896, 4864), (1536, 8960), (896, 896), (16, 64), (48, 320)])
-@pytest.mark.parametrize("splits", [1, 2, 4, 7])
-@pytest.mark.parametrize("T", [1, 16, 17, 33, 64, 65])
+@pytest.mark.parametrize("splits", [0, 1, 2, 7])
+@pytest.mark.parametrize("T", [1, 16, 17, 33, 65, 300])
 def test_projection_with_residual(T, splits, out_f, in_f):
     """Split K too: more splits than slices of K among them; a second call finds the counters at zero."""
     g = torch.Generator(device="cuda").manual_seed(T)
@@ -85,6 +85,33 @@ def test_projection_with_residual(T, splits, out_f, in_f):
     again = hip_layer.fused_linear(x, w, hip_layer.RESIDUAL, residual=res, num_splits=splits)
     assert rel(first, ref) < BOUND
     assert torch.equal(first, again)
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("T", [1, 16, 33, 129])
+def test_every_tile_shape(tile, T):
+    """Each tile of the projection kernels with each epilogue, at row counts that fill no whole tile (120 rows of 16 for
+    tiles of up to 128) and a K of 5 slices (less and more than the slices in flight)."""
+    if tile == 6 and T > 16:
+        return
+    g = torch.Generator(device="cuda").manual_seed(T)
+    K, d, heads, inter = 320, 48, 5, 120
+    x, nw, res, b = randn(g, T, K), 1 + 0.1 * randn(g, K), randn(g, T, heads * d), randn(g, heads * d)
+    w, gu = randn(g, heads * d, K) * 0.05, randn(g, 2 * inter, K) * 0.05
+    rot = randn(g, T, 1, d), randn(g, T, 1, d)
+    print(f"case tile {tile} T {T}", flush=True)
+    xn = norm64(x, nw)
+    y = (xn @ w.double().t() + b.double()).view(T, heads, d)
+    out = hip_layer.fused_linear(x, w, hip_layer.ROPE, norm_weight=nw, eps=EPS, bias=b, rot=rot, head_dim=d,
+                                 rot_channels=3 * d, tile=tile)
+    assert rel(out, torch.cat([rotate64(y[:, :3], *rot), y[:, 3:]], 1).view(T, -1)) < BOUND
+    out = hip_layer.fused_linear(x, gu, hip_layer.SILU, norm_weight=nw, eps=EPS, tile=tile)
+    y = xn @ gu.double().t()
+    assert rel(out, F.silu(y[:, :inter]) * y[:, inter:]) < BOUND
+    ref = x.double() @ w.double().t() + res.double() + b.double()
+    for splits in (1, 2) if tile < 6 else (1,):
+        out = hip_layer.fused_linear(x, w, hip_layer.RESIDUAL, bias=b, residual=res, num_splits=splits, tile=tile)
+        assert rel(out, ref) < BOUND
 
 
 @pytest.mark.parametrize("K", [8, 896, 1024, 1032, 1536, 2056, 8192])
@@ -116,18 +143,18 @@ def test_rope_and_silu_rows(T, heads, extra, d):
     assert rel(hip_layer.silu_mul(gu), F.silu(gu[:, :half].double()) * gu[:, half:].double()) < 2 ** -9
 
 
-@pytest.mark.parametrize("T", [1, 16, 33, 130])
+@pytest.mark.parametrize("T", [1, 16, 33, 130, 1025])
 def test_layer_on_kernels_matches_torch_operations(T):
     """layer_forward under inference_mode (the kernels) against the same call outside it (the torch operations), and
     what the layer wrote into the cache."""
     cfg = ModelConfig(vocab_size=64, hidden_size=896, intermediate_size=4864, num_layers=1, num_q_heads=14,
                       num_kv_heads=2, head_dim=64)
-    model = Qwen2Model(cfg, "cuda", torch.bfloat16, seed=1, max_positions=512, std=0.05)
+    model = Qwen2Model(cfg, "cuda", torch.bfloat16, seed=1, max_positions=2048, std=0.05)
     g = torch.Generator(device="cuda").manual_seed(2)
     x = randn(g, T, 896)
     results = []
     for fused in (True, False):
-        m = fragmented_manager(64, 16, torch.Generator().manual_seed(3))
+        m = fragmented_manager(128, 16, torch.Generator().manual_seed(3))
         cache = PagedKVCache(cfg, m.num_blocks, 16, "cuda", torch.bfloat16, attn_backend="hip")
         cache.k.zero_()
         cache.v.zero_()

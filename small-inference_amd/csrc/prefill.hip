@@ -5,8 +5,11 @@
 // (query at position p sees keys 0 .. p, query head g uses KV head g / G, softmax in fp32, probabilities rounded
 // to the model dtype before P.V). This kernel computes the same rows in place from the pool.
 //
-// Work unit: (sequence s, KV head h, 16 tt consecutive new tokens). The unit's keys are positions [0, P0 + ntok)
-// of the sequence, P0 the position of the unit's first token; they are cut into splits of `chunk` keys, one
+// Work unit: (sequence s, KV head h, NC column tiles). The column tiles of a (sequence, KV head) are its (16 new tokens,
+// query head) pairs, heads fastest; unit j takes columns NC j .. NC j + NC - 1, so that every unit but a sequence's last
+// one fills its waves whatever the group size (whole 16-token steps of G = 6 or 7 heads left 4 or 2 of 16 waves idle).
+// The unit's keys are positions [0, P0 + ntok) of the sequence, P0 the position of its first token and ntok the tokens
+// its columns span; they are cut into splits of `chunk` keys, one
 // workgroup each, so that a short chunk over a long context still fills the chip. The four waves of a workgroup
 // stream the same key tiles (64 keys at head_dim 64, 32 at 128), which the workgroup loads cooperatively into
 // double-buffered LDS (one HBM read per split), and each wave owns its own column tiles (a query head and 16 of
@@ -38,9 +41,8 @@ struct PrefillArgs {
   const int32_t* qlen;    // [S] new tokens per sequence
   void* out;
   int64_t o_st, o_sh;
-  int32_t S, G, qtiles;   // qtiles = ceil(max new tokens / (16 tt))
+  int32_t S, G, qtiles;   // qtiles: units of the longest sequence, ceil(ceil(max new tokens / 16) G / NC)
   int32_t npair;           // S * Hkv
-  int32_t tt;              // 16-token subtiles per unit: G * tt <= 8 column tiles
   int32_t T, nb, max_ctx;  // rows of q / out, pool blocks, context clamp
   int32_t nsplit, chunk;   // key splits per unit, keys per split (a multiple of 64)
   // INT8 pools (kernel MODE 1, 2): scales and format B's staging, as in sipa_prefill_params
@@ -84,8 +86,11 @@ static inline PfShape prefill_shape(int layout) {
   }
 }
 
-// 16-token subtiles per unit for a GQA group of G heads: as many as fit the workgroup's NC column tiles (NC 8:
-// G = 7: 1, G = 4: 2, G = 1: 8), so every group size keeps the waves busy.
+// Units of a (sequence, KV head) with n new tokens.
+static inline int64_t prefill_units(int n, int G, int nc) { return ((n + 15) / 16 * (int64_t)G + nc - 1) / nc; }
+
+// Whole 16-token steps of G heads that fit NC column tiles: the unit of the split policy and of the workspace size (at
+// least as many units as prefill_units gives).
 static inline int prefill_subtiles(int G, int nc) { return G >= nc ? 1 : nc / G; }
 constexpr int kPrefillMaxSplits = 32;
 
@@ -196,14 +201,17 @@ __global__ void __launch_bounds__(64 * NC / CW * KH) prefill_mfma_bf16(const Pre
   const int pair = u % a.npair;
   const int j = a.qtiles - 1 - u / a.npair;
   const int s = pair % a.S, h = pair / a.S;
-  const int G = a.G, TT = a.tt, NT = 16 * a.tt;  // query heads, token subtiles, tokens per unit
+  const int G = a.G;
   const int n = a.qlen[s];
-  if (NT * j >= n) return;
-  const int row0 = a.qstart[s] + NT * j;
+  const int c_base = NC * j;                              // the unit's first column
+  const int tok0 = 16 * (c_base / G);                     // its first token,
+  const int span = 16 * ((c_base + NC - 1) / G + 1) - tok0;  // and the tokens its columns span
+  if (tok0 >= n) return;
+  const int row0 = a.qstart[s] + tok0;
   const int ctx = min(a.ctx[s], a.max_ctx);
-  const int ntok = min(min(NT, n - NT * j), a.T - row0);  // rows past T are not touched
+  const int ntok = min(min(span, n - tok0), a.T - row0);  // rows past T are not touched
   if (ntok <= 0 || row0 < 0) return;
-  const int P0 = ctx - n + NT * j;  // position of the unit's first token
+  const int P0 = ctx - n + tok0;  // position of the unit's first token
   // keys [0, kv_vis) are visible to some token of the unit; this split takes [k_lo, kv_end), KH chunks of
   // a.chunk keys, key half x the x-th of them (the last half may be shorter or empty)
   const int kv_vis = max(1, min(ctx, P0 + ntok));
@@ -227,18 +235,18 @@ __global__ void __launch_bounds__(64 * NC / CW * KH) prefill_mfma_bf16(const Pre
     bids[i] = MODE == 0 ? (int)(uint32_t)((uint64_t)blk * (uint64_t)(a.kv_sn >> 3)) : blk;
   }
 
-  // Column tiles c = wcol + (NC / CW) ci of the unit: query head g = c % G of the group, tokens 16 tt .. 16 tt + 15
-  // with tt = c / G (G * TT <= NC). A column tile's B operand holds token r of head g (zero past the unit's
-  // tokens).
+  // Column tiles wcol + (NC / CW) ci of the unit, c with c_base: query head g = c % G of the group, the sequence's new
+  // tokens 16 (c / G) .. + 15, ctok the first of them within the unit. A column tile's B operand holds token r of head
+  // g (zero past the unit's tokens).
   int cg[CW], ctok[CW];
   bool cvalid[CW];  // wave-uniform
   bf16x8 qop[CW][KS];
 #pragma unroll
   for (int ci = 0; ci < CW; ++ci) {
-    const int c = wcol + CWV * ci;
+    const int c = c_base + wcol + CWV * ci;
     cg[ci] = c % G;
-    ctok[ci] = 16 * (c / G);
-    cvalid[ci] = c / G < TT && ctok[ci] < ntok;
+    ctok[ci] = 16 * (c / G) - tok0;
+    cvalid[ci] = ctok[ci] < ntok;
     const bool valid = cvalid[ci] && ctok[ci] + r < ntok;
     const uint16_t* qrow = (const uint16_t*)a.q + (int64_t)(row0 + min(ctok[ci] + r, ntok - 1)) * a.q_st +
                            (int64_t)(h * G + cg[ci]) * a.q_sh;
@@ -377,9 +385,12 @@ __global__ void __launch_bounds__(64 * NC / CW * KH) prefill_mfma_bf16(const Pre
   bf16x8 ones = kOnes;
   asm volatile("" : "+v"(ones));
 
+  // The last position some token of the wave's column tiles has: tiles past it are all hidden from them, and skipped.
+  const int last_seen = P0 + ctok[CW - 1] + 15;
   auto tile = [&](int t) {
     const int buf = t & 1;
     const int t0 = h_lo + KT * t;
+    if (t0 > last_seen) return;  // wave-uniform
     const bool masked = t0 + KT - 1 > P0 || t0 + KT > h_end;  // some key of the tile is hidden from some token
     const uint16_t* ks = sm[buf][whalf][0];
     const uint16_t* vs = sm[buf][whalf][1];
@@ -612,9 +623,9 @@ __global__ void __launch_bounds__(64 * NC / CW * KH) prefill_mfma_bf16(const Pre
       constexpr int AUX = decltype(aux_tag)::value;
       constexpr int TPR = PT / kSlots, CPT = D / TPR, CB = CPT < 32 ? CPT : 32, KB = 4;  // threads per row
       const int slot = threadIdx.x / TPR, part = threadIdx.x % TPR;
-      const int c = slot >> 4, rr = slot & 15;
-      const int g = c % G, tok = 16 * (c / G) + rr;
-      if (c / G < TT && tok < ntok) {
+      const int c = c_base + (slot >> 4), rr = slot & 15;
+      const int g = c % G, tok = 16 * (c / G) - tok0 + rr;
+      if (tok < ntok) {
         uint16_t* orow = (uint16_t*)a.out + (int64_t)(row0 + tok) * a.o_st + (int64_t)(h * G + g) * a.o_sh;
         for (int c0 = CPT * part; c0 < CPT * (part + 1); c0 += CB) {
           float M = kNegInf, den = 0.f;
@@ -879,9 +890,10 @@ extern "C" int32_t sipa_prefill(const sipa_prefill_params* p, void* stream) {
              SIPA_EUNSUPPORTED, "format B pools take SIPA_PREFILL_W4X2 or _W8X1 (16-wave workgroups cannot hold "
              "their registers)");
   const PfShape shape = prefill_shape(layout);
-  const int tt = prefill_subtiles(G, shape.nc);
-  const int qtiles = (p->max_query_len + 16 * tt - 1) / (16 * tt);
-  const int64_t units = (int64_t)S * Hkv * qtiles;
+  const int64_t qtiles64 = prefill_units(p->max_query_len, G, shape.nc);
+  const int64_t units = (int64_t)S * Hkv * qtiles64;
+  SIPA_CHECK(units <= 0x7fffffff, SIPA_EINVAL, "%lld units exceed the grid limit", (long long)units);
+  const int qtiles = (int)qtiles64;
   const int nsplit = (nchunk + shape.kh - 1) / shape.kh;  // workgroups per unit
   const int64_t wgs = grid_of(units, shape.kh);
   SIPA_CHECK(wgs <= 0x7fffffff, SIPA_EINVAL, "%lld workgroups exceed the grid limit", (long long)wgs);
@@ -917,7 +929,6 @@ extern "C" int32_t sipa_prefill(const sipa_prefill_params* p, void* stream) {
   a.G = G;
   a.qtiles = qtiles;
   a.npair = S * Hkv;
-  a.tt = tt;
   a.T = p->num_tokens;
   a.nb = p->num_blocks;
   a.max_ctx = p->max_context;

@@ -485,3 +485,24 @@ def test_wave_layouts_agree(shape, pool, splits):
         for lay in ("w16x1", "w16h2"):
             with pytest.raises(ValueError, match="format B"):
                 run(lay)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(10, 2, 64), (12, 2, 64), (14, 2, 128), (24, 8, 128), (5, 1, 64)])
+@pytest.mark.parametrize("layout", ["w4x2", "w8x1", "w16x1", "w16h2"])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_units_packed_across_token_steps(Hq, Hkv, D, layout, splits):
+    """Groups of 3 to 7 heads: a unit's 8 or 16 columns start and end inside a 16-token step, so a step's heads can sit in
+    two units and a unit can span several steps; new-token counts around the steps' edges, fresh and mid-context,
+    against the oracle."""
+    ctx, qlen = [17, 33, 100, 700, 900], [17, 33, 47, 129, 16]
+    q, k, v, bt, c, st, ln, tables, starts, T = make_prefill(ctx, qlen, Hq, Hkv, D, seed=Hq, gap=2)
+    out = torch.full_like(q, SENTINEL)
+    print(f"case packed {Hq}/{Hkv}/{D} {layout} splits {splits}", flush=True)
+    paged_prefill_attention(q, k, v, bt, c, st, ln, D ** -0.5, max(ctx), max(qlen), out=out, num_splits=splits,
+                            wg_layout=layout)
+    torch.cuda.synchronize()
+    got = out.double().cpu().numpy()
+    ref = paged_ref.prefill(as_np32(q), as_np32(k), as_np32(v), tables, ctx, starts, qlen, D ** -0.5, dtype=np.float32)
+    rows = np.concatenate([np.arange(s, s + n) for s, n in zip(starts, qlen)])
+    assert_bf16_close(got[rows], ref[rows], f"packed {layout}")
+    assert (got[np.setdiff1d(np.arange(T), rows)] == SENTINEL).all()

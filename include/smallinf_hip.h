@@ -279,12 +279,11 @@ enum {
 
 int32_t sipa_prefill(const sipa_prefill_params* p, void* stream);
 
-/* Key splits for a prefill call (no counterpart in the reference, whose gather path has no grid): about two
- * workgroups per CU over the call's 8-column units, at least 256 keys per split, at most 32 splits. An 8-column
- * unit is here a KV head and 16 tt new tokens of one sequence, tt = 8 / G 16-token subtiles (at least 1) for a group
- * of G = Hq / Hkv query heads (the kernel packs (16 tokens, head) columns into fewer, full units; head_dim is part of the policy's signature and does not change it today);
- * query_tiles = sum over sequences of ceil(query_len / 16). A 16-column layout keeps the split count and runs
- * half as many units. cu_count <= 0 asks the current device. */
+/* Key splits for a prefill call (no counterpart in the reference, whose gather path has no grid): one under 512 keys
+ * of context; about two workgroups per CU over the call's 8-column units from 4096 keys (from 2048 where not even two
+ * splits fit one workgroup per CU); between, at most one workgroup per CU and 8 splits. At least 256 keys per split
+ * and at most 32 splits. query_tiles = sum over sequences of ceil(query_len / 16) (head_dim is part of the policy's
+ * signature and does not change it today). cu_count <= 0 asks the current device. */
 int32_t sipa_prefill_splits(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t query_tiles,
                             int32_t max_context, int32_t cu_count);
 

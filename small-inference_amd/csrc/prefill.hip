@@ -724,13 +724,31 @@ static int prefill_chunk(int max_context, int splits) {
   return std::max(256, (c + 63) / 64 * 64);
 }
 
-// Split count policy: about two workgroups per CU over all units (units = KV heads x query tiles of
-// 16 tokens), no split under 256 keys, at most 32.
-static int prefill_splits_host(int64_t units, int max_context, int cu_count) {
-  if (units <= 0 || max_context <= 0) return 1;
-  const int64_t target = 2LL * std::max(cu_count, 1);
-  const int want = (int)std::min<int64_t>((target + units - 1) / units, kPrefillMaxSplits);
-  const int chunk = prefill_chunk(max_context, want);
+// Split count policy, over `tiles` 16-token query tiles of all sequences and the longest context:
+//  - under 512 keys: one split (two of 256 or less cost their merge: 448 keys 18.2 against 19.0 us, 343 11.6 / 12.2).
+//  - from 4096 keys, or from 2048 where not even two whole splits a unit fit one workgroup per CU: about two workgroups
+//    per CU over units of whole 16-token steps (512 tokens at 8K 28.6 us with 8 splits, two chunks a workgroup, 30.8
+//    with 4; 241 tokens at 6.8K at head_dim 128 35.7 with 16, 41.5 with 8).
+//  - between: at most one workgroup per CU, at most 8 splits, of at least 256 keys. More put a second workgroup on some
+//    CUs and lengthen the merge: three 797-token chunks at 1.5K 25.0 us with one split, 34.0 with two; 593 at 1.1K 12.5
+//    with three, 16.2 with five; 22 at 2.4K 11.9 with 8, 12.6 with 10; 298 at 3.8K (format B) 34.7 with 8, 64.6 with 12.
+// At least 256 keys a split and at most 32 splits in any case. (Graph replays of 73 shapes, this rule's time over the
+// best of all layouts and split counts: 1.02 in the geometric mean, 1.13 with two workgroups per CU throughout.)
+static int prefill_splits_host(int Hkv, int G, int64_t tiles, int max_context, int cu_count) {
+  if (tiles <= 0 || max_context <= 0) return 1;
+  const int64_t cu = std::max(cu_count, 1);
+  const int64_t fit = cu / std::max<int64_t>(1, Hkv * ((tiles * G + 7) / 8));  // splits at one workgroup per CU
+  int64_t want;
+  if (max_context < 512) {
+    want = 1;
+  } else if (max_context >= 4096 || (fit < 2 && max_context >= 2048)) {
+    const int tt = prefill_subtiles(G, 8);
+    const int64_t units = (int64_t)Hkv * ((tiles + tt - 1) / tt);
+    want = std::min<int64_t>((2 * cu + units - 1) / units, kPrefillMaxSplits);
+  } else {
+    want = std::min<int64_t>(std::min<int64_t>((max_context + 255) / 256, 8), std::max<int64_t>(1, fit));
+  }
+  const int chunk = prefill_chunk(max_context, (int)want);
   return (max_context + chunk - 1) / chunk;
 }
 
@@ -754,8 +772,7 @@ extern "C" int32_t sipa_prefill_splits(int32_t num_q_heads, int32_t num_kv_heads
                                        int64_t query_tiles, int32_t max_context, int32_t cu_count) {
   if (num_kv_heads <= 0 || num_q_heads < num_kv_heads) return 1;
   if (cu_count <= 0) cu_count = sipa_device_cu_count(-1);
-  const int tt = prefill_subtiles(num_q_heads / num_kv_heads, 8);
-  return prefill_splits_host((int64_t)num_kv_heads * ((query_tiles + tt - 1) / tt), max_context, cu_count);
+  return prefill_splits_host(num_kv_heads, num_q_heads / num_kv_heads, query_tiles, max_context, cu_count);
 }
 
 extern "C" int64_t sipa_prefill_workspace_bytes(int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
@@ -835,13 +852,13 @@ extern "C" int32_t sipa_prefill(const sipa_prefill_params* p, void* stream) {
   }
   SIPA_CHECK(p->wg_layout >= SIPA_PREFILL_AUTO && p->wg_layout <= SIPA_PREFILL_W16H2, SIPA_EINVAL,
              "wg_layout %d is not a SIPA_PREFILL_* layout", p->wg_layout);
-  // The split count and the layout choice are made over 8-column units; a 16-column layout then runs half as
-  // many units with the same splits.
-  const int tt8 = prefill_subtiles(G, 8);
-  const int64_t units8 = (int64_t)S * Hkv * ((p->max_query_len + 16 * tt8 - 1) / (16 * tt8));
+  // The layout choice is made over 8-column units; a 16-column layout then runs half as many units with the same
+  // splits.
+  const int64_t units8 = (int64_t)S * Hkv * prefill_units(p->max_query_len, G, 8);
   const int cus = sipa_device_cu_count(-1);
   int splits = p->num_splits;
-  if (splits <= 0) splits = prefill_splits_host(units8, p->max_context, cus);
+  if (splits <= 0)
+    splits = prefill_splits_host(Hkv, G, (int64_t)S * ((p->max_query_len + 15) / 16), p->max_context, cus);
   const int chunk = prefill_chunk(p->max_context, splits);
   const int nchunk = (p->max_context + chunk - 1) / chunk;  // key chunks per unit
   // split launches: whole groups of 8 units, one XCD each (the kernel's workgroup-to-unit mapping); a
@@ -850,41 +867,37 @@ extern "C" int32_t sipa_prefill(const sipa_prefill_params* p, void* stream) {
     const int ns = (nchunk + kh - 1) / kh;
     return (ns > 1 ? (units + 7) / 8 * 8 : units) * ns;
   };
-  // Layout (SIPA_PREFILL_AUTO), from g8, the grid of 8-column workgroups (warm A/B on one MI355X, 0.5B and 1.5B
-  // shapes, us per call):
-  //  - g8 <= CUs: 8-wave workgroups, one per CU (16-wave ones would leave half the CUs idle).
+  // Layout (SIPA_PREFILL_AUTO), from g8, the grid of 8-column workgroups (graph replays on one MI355X, 73 shapes of both
+  // model shapes, us per call):
+  //  - g8 <= CUs: 8-wave workgroups, one per CU (16-wave ones would leave half the CUs idle), except past 16 key chunks,
+  //    whose merge W16H2 halves: 14 tokens at 8K, 32 chunks, 34.9 -> 25.2.
   //  - a chunk at least its own length into its context (balanced units: the causal triangle varies a unit's keys
   //    by at most a factor of two):
-  //    . bf16 pools, 8 or more key chunks of at most 1024 keys: 16 waves over 8 column tiles and two consecutive
-  //      key chunks (INT8 pools: each half dequantizes its own tiles, twice the store work per CU; 512 at 8K
-  //      32.4 -> 34.8, so they keep W16X1),
-  //      combined in the workgroup, so that half as many splits store partials and merge (one merging workgroup
-  //      per unit reads 4 partials, not 8): 512 new tokens at 8K 29.0 -> 28.2, 256 at 8K 23.1 -> 20.5, 128 at 8K
-  //      25.5 -> 18.5, at head_dim 128 512 at 8K 46.5 -> 43.8, 256 at 8K 39.2 -> 30.1 (best of the others ->);
+  //    . 8 or more key chunks of at most 1024 keys, bf16 pools or head_dim 128: 16 waves over 8 column tiles and two
+  //      consecutive key chunks, combined in the workgroup, so that half as many splits store partials and merge: 512
+  //      new tokens at 8K 30.8 (best of the others) -> 28.6, at head_dim 128 241 at 6.8K over INT8 41.5 -> 35.7. (INT8 at
+  //      head_dim 64 keeps W16X1: each half dequantizes its own tiles, 512 at 8K 32.4 -> 34.8.)
   //    . otherwise, with one chunk or chunks of at least 1024 keys: 16-wave workgroups of 16 column tiles, one per
   //      CU at a time. Two co-resident 8-column workgroups do not share a CU evenly (the later-dispatched ran ~30%
-  //      longer and finished alone), and 16 column tiles share each K/V tile load: 512 new tokens at 16K
-  //      48.9 -> 46.3 (8-wave), 16 chunks of 512 at 8K 313.8 -> 290.6 (4-wave), 1024 at 8K 47.2 -> 44.0;
+  //      longer and finished alone), and 16 column tiles share each K/V tile load: two 677-token chunks at 3K 29.2 ->
+  //      27.9, INT8 chunks up to 461 at 4.4K 74.9 -> 67.3.
   //    . else 8-wave workgroups.
-  //  - fresh prompts: 8-wave workgroups up to 3 per CU (two 2048-token prompts 31.9 against 40.3 at 16 waves:
-  //    32-token units double the longest CU's keys); above, 16-wave ones (four 2048-token prompts 48.6 against
-  //    50.4 at 4 waves; at head_dim 128 76.0 against 87.9), except at head_dim 64 beyond 4 per CU, where 4-wave
-  //    workgroups of two column tiles per wave share each K/V operand read among more tokens (six prompts 67.3
-  //    against 76.9; at head_dim 128 their 206 registers leave two waves per SIMD, never the best).
-  // Format B's one-column waves hold too many registers for 16 waves; it takes the 4-wave layout.
+  //  - fresh prompts: 8-wave workgroups up to 3 per CU (1260-token prompts, 2.2 per CU, 28.9 against 31.4 at 16 waves and
+  //    29.6 at 4; 1501-token ones at head_dim 128 57.4 against 61.1 and 67.9), above them 16-wave ones (four 2048-token
+  //    prompts 46.4 against 48.3, five 1895-token ones at head_dim 128 76.7 against 84.4).
+  // Format B's one-column waves hold too many registers for 16 waves: 8 waves up to 1.5 workgroups per CU (298 tokens at
+  // 3.8K 34.7 against 42.0 at 4 waves, 58 at 1.2K 23.7 against 28.2), 4 waves above (1092 tokens 61.7 against 70.8).
   int layout = p->wg_layout;
   if (layout == SIPA_PREFILL_AUTO) {
     const int64_t g8 = grid_of(units8, 1);
     const bool balanced = p->max_context >= 2LL * p->max_query_len;
-    if (mode == SIPA_KV_INT8_KCHAN) layout = SIPA_PREFILL_W4X2;
-    else if (g8 <= cus) layout = SIPA_PREFILL_W8X1;
+    if (mode == SIPA_KV_INT8_KCHAN) layout = 2 * g8 <= 3LL * cus ? SIPA_PREFILL_W8X1 : SIPA_PREFILL_W4X2;
+    else if (g8 <= cus) layout = nchunk > 16 ? SIPA_PREFILL_W16H2 : SIPA_PREFILL_W8X1;
     else if (balanced)
-      layout = mode == SIPA_KV_PLAIN && nchunk >= 8 && chunk <= 1024 ? SIPA_PREFILL_W16H2
-               : nchunk == 1 || chunk >= 1024                      ? SIPA_PREFILL_W16X1
-                                                                   : SIPA_PREFILL_W8X1;
-    else if (g8 <= 3LL * cus) layout = SIPA_PREFILL_W8X1;
-    else if (D == 64 && g8 > 4LL * cus) layout = SIPA_PREFILL_W4X2;
-    else layout = SIPA_PREFILL_W16X1;
+      layout = (mode == SIPA_KV_PLAIN || D == 128) && nchunk >= 8 && chunk <= 1024 ? SIPA_PREFILL_W16H2
+               : nchunk == 1 || chunk >= 1024                                    ? SIPA_PREFILL_W16X1
+                                                                                 : SIPA_PREFILL_W8X1;
+    else layout = g8 <= 3LL * cus ? SIPA_PREFILL_W8X1 : SIPA_PREFILL_W16X1;
   }
   SIPA_CHECK(mode != SIPA_KV_INT8_KCHAN || layout == SIPA_PREFILL_W4X2 || layout == SIPA_PREFILL_W8X1,
              SIPA_EUNSUPPORTED, "format B pools take SIPA_PREFILL_W4X2 or _W8X1 (16-wave workgroups cannot hold "

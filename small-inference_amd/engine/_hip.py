@@ -193,11 +193,23 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 def stream_of(t: torch.Tensor) -> int:
     """The current torch stream of t's device, as a hipStream_t value."""
-    return torch._C._cuda_getCurrentRawStream(t.device.index)  # current_stream(t.device).cuda_stream, at a tenth of its time
+    return torch._C._cuda_getCurrentRawStream(t.get_device())  # current_stream(t.device).cuda_stream, at a tenth of its time
 
 
-def require_gpu(*tensors: torch.Tensor) -> None:
+def require_gpu(first: torch.Tensor, *rest: torch.Tensor | None) -> None:
     """The kernels read device memory: every tensor must live on one GPU."""
-    devs = {t.device for t in tensors if t is not None}
-    if len(devs) != 1 or next(iter(devs)).type != "cuda":
+    dev = first.get_device() if first.is_cuda else -1
+    for t in rest:
+        if t is not None and not (t.is_cuda and t.get_device() == dev):
+            dev = -1
+    if dev < 0:
+        devs = {t.device for t in (first, *rest) if t is not None}
         raise ValueError(f"HIP kernels need all tensors on one GPU, got {sorted(map(str, devs))}")
+
+
+def layer_ptr(pools: torch.Tensor, layer: int) -> int:
+    """Address of pools[layer], without making the view. IndexError past the layers, as indexing gives."""
+    n = pools.shape[0]
+    if not -n <= layer < n:
+        raise IndexError(f"layer {layer} of {n}")
+    return pools.data_ptr() + (layer + n if layer < 0 else layer) * pools.stride(0) * pools.element_size()

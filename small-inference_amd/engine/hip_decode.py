@@ -198,6 +198,7 @@ class DecodePlan:
             raise ValueError(f"impl {impl!r} / combine {combine!r}")
         self.shape, self.dtype, self.device = (S, Hq, D), q.dtype, q.device
         self.pool_shape, self.pool_dtype = tuple(k_cache.shape), k_cache.dtype
+        self.row_strides = (Hq * D, D)  # of the outputs made here
         self.quant_mode = 0 if quant is None else quant.mode
         self._keep = [block_tables, context_lens.contiguous()]  # tensors the parameter block points into
         self.lib = _hip.lib()
@@ -271,37 +272,69 @@ class DecodePlan:
             self.workspace = ws
             self._keep.append(ws)
             p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
+        p.kv_stride_h, p.kv_stride_n = k_cache.stride(0), k_cache.stride(1)  # contiguous pools of one shape
+        self._launch, self._params_ref = self.lib.sipa_decode, ctypes.byref(p)
         self._bind(q, k_cache, v_cache, quant)
 
     def _bind(self, q, k_cache, v_cache, quant) -> None:
         """Point the parameter block at this call's tensors (same shapes and dtypes as the plan's)."""
-        if tuple(q.shape) != self.shape or q.dtype != self.dtype or q.stride(-1) != 1:
-            raise ValueError("q does not match the plan")
-        if tuple(k_cache.shape) != self.pool_shape or tuple(v_cache.shape) != self.pool_shape or \
+        if k_cache.shape != self.pool_shape or v_cache.shape != self.pool_shape or \
                 k_cache.dtype != self.pool_dtype or v_cache.dtype != self.pool_dtype or \
                 not (k_cache.is_contiguous() and v_cache.is_contiguous()):
             raise ValueError("the pools do not match the plan")
-        self._q, self._k, self._v, self._quant = q, k_cache, v_cache, quant
+        self._bind_q(q)
+        self._k, self._v, self._quant = k_cache, v_cache, quant
         p = self.params
-        p.q, p.q_stride_s, p.q_stride_h = q.data_ptr(), q.stride(0), q.stride(1)
         p.k_cache, p.v_cache = k_cache.data_ptr(), v_cache.data_ptr()
-        p.kv_stride_h, p.kv_stride_n = k_cache.stride(0), k_cache.stride(1)
         if self.quant_mode:
             ks, vs = quant.k_scale, quant.v_scale
-            if ks.stride(-1) != 1 or vs.stride(-1) != 1:
-                raise ValueError("scales need a contiguous last dim")
-            p.k_scale, p.k_scale_dtype, p.ks_stride_h, p.ks_stride_n = \
-                ks.data_ptr(), _hip.dtype_code(ks.dtype), ks.stride(0), ks.stride(1)
-            p.v_scale, p.v_scale_dtype, p.vs_stride_h, p.vs_stride_n = \
-                vs.data_ptr(), _hip.dtype_code(vs.dtype), vs.stride(0), vs.stride(1)
+            self._bind_scales(ks.data_ptr(), ks.dtype, ks.stride(), vs.data_ptr(), vs.dtype, vs.stride())
             if self.quant_mode == 2:
                 st = quant.stage
-                if st.dtype != torch.bfloat16 or st.stride(-1) != 1:
-                    raise ValueError("stage must be bf16 with a contiguous last dim")
-                if st.shape[1] != self.num_stage:
-                    raise ValueError("stage does not match the plan's staging slots")
-                p.stage, p.st_stride_h, p.st_stride_n, p.st_stride_b = \
-                    st.data_ptr(), st.stride(0), st.stride(1), st.stride(2)
+                self._bind_stage(st.data_ptr(), st.dtype, st.shape[1], st.stride())
+
+    def _bind_q(self, q) -> None:
+        ss, sh, sd = q.stride() if q.shape == self.shape else (0, 0, 0)
+        if sd != 1 or q.dtype != self.dtype:
+            raise ValueError("q does not match the plan")
+        self._q = q
+        p = self.params
+        p.q, p.q_stride_s, p.q_stride_h = q.data_ptr(), ss, sh
+
+    def _bind_scales(self, ks: int, ks_dtype, ks_strides, vs: int, vs_dtype, vs_strides) -> None:
+        if ks_strides[-1] != 1 or vs_strides[-1] != 1:
+            raise ValueError("scales need a contiguous last dim")
+        p = self.params
+        p.k_scale, p.k_scale_dtype, p.ks_stride_h, p.ks_stride_n = ks, _hip.dtype_code(ks_dtype), *ks_strides[-3:-1]
+        p.v_scale, p.v_scale_dtype, p.vs_stride_h, p.vs_stride_n = vs, _hip.dtype_code(vs_dtype), *vs_strides[-3:-1]
+
+    def _bind_stage(self, st: int, dtype, slots: int, strides) -> None:
+        if dtype != torch.bfloat16 or strides[-1] != 1:
+            raise ValueError("stage must be bf16 with a contiguous last dim")
+        if slots != self.num_stage:
+            raise ValueError("stage does not match the plan's staging slots")
+        p = self.params
+        p.stage, p.st_stride_h, p.st_stride_n, p.st_stride_b = st, *strides[-4:-1]
+
+    def run_layer(self, layer: int, q: torch.Tensor, k_pools: torch.Tensor, v_pools: torch.Tensor,
+                  quant: QuantKV | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
+        """The decode over layer `layer` of pools [L, Hkv, N, B, D] (quant: scales and staging with a leading layer
+        dimension too): the plan called with pools[layer] and the like, without making those views."""
+        for pools in (k_pools, v_pools):
+            if pools.shape[1:] != self.pool_shape or pools.dtype != self.pool_dtype or not pools.is_contiguous():
+                raise ValueError("the pools do not match the plan")
+        self._bind_q(q)
+        p = self.params
+        p.k_cache, p.v_cache = _hip.layer_ptr(k_pools, layer), _hip.layer_ptr(v_pools, layer)
+        self._k, self._v, self._quant = k_pools, v_pools, quant
+        if self.quant_mode:
+            ks, vs = quant.k_scale, quant.v_scale
+            self._bind_scales(_hip.layer_ptr(ks, layer), ks.dtype, ks.stride(), _hip.layer_ptr(vs, layer), vs.dtype,
+                              vs.stride())
+            if self.quant_mode == 2:
+                st = quant.stage
+                self._bind_stage(_hip.layer_ptr(st, layer), st.dtype, st.shape[2], st.stride())
+        return self._run(out)
 
     def __call__(self, q: torch.Tensor | None = None, k_cache: torch.Tensor | None = None,
                  v_cache: torch.Tensor | None = None, quant: QuantKV | None = None,
@@ -310,15 +343,23 @@ class DecodePlan:
         if q is not None or k_cache is not None or v_cache is not None or quant is not None:
             self._bind(q if q is not None else self._q, k_cache if k_cache is not None else self._k,
                        v_cache if v_cache is not None else self._v, quant if quant is not None else self._quant)
+        return self._run(out)
+
+    def _run(self, out: torch.Tensor | None) -> torch.Tensor:
+        p = self.params
         if out is None:
-            out = torch.empty(self.shape, device=self.device, dtype=self.dtype)
-        elif tuple(out.shape) != self.shape or out.dtype != self.dtype or out.stride(-1) != 1:
+            out = self._q.new_empty(self.shape)
+            p.out_stride_s, p.out_stride_h = self.row_strides
+        elif out.shape != self.shape or out.dtype != self.dtype or out.stride(-1) != 1:
             raise ValueError("out must be [S, Hq, D] in q's dtype with a contiguous last dim")
+        else:
+            p.out_stride_s, p.out_stride_h = out.stride(0), out.stride(1)
         if self.shape[0] == 0:
             return out
-        p = self.params
-        p.out, p.out_stride_s, p.out_stride_h = out.data_ptr(), out.stride(0), out.stride(1)
-        _hip.check(self.lib.sipa_decode(ctypes.byref(p), self.stream), "paged_decode_attention")
+        p.out = out.data_ptr()
+        rc = self._launch(self._params_ref, self.stream)
+        if rc:
+            _hip.check(rc, "paged_decode_attention")
         return out
 
     def launch_raw(self, k_ptr: int, v_ptr: int, out_ptr: int) -> int:

@@ -28,36 +28,37 @@ MAX_TOKENS = 1024
 MAX_GATED_FLOPS = 18e9
 
 
-def _ok(t, device: torch.device, dim: int) -> bool:
-    return (type(t) is torch.Tensor or type(t) is torch.nn.Parameter) and t.dtype == torch.bfloat16 and \
-        t.device == device and t.dim() == dim and t.is_contiguous() and t.data_ptr() % 16 == 0
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _ok(t, device: int, *shape: int) -> bool:
+    return type(t) in _PLAIN and t.dtype is torch.bfloat16 and t.get_device() == device and t.shape == shape and \
+        t.is_contiguous() and t.data_ptr() % 16 == 0
 
 
 def rows_ok(x: torch.Tensor, norm_weight: torch.Tensor) -> bool:
     """Whether rms_norm can run on rows x [T, K]. Only under torch.inference_mode: the kernels record nothing for
     autograd, and forward-mode derivatives and saved-tensor hooks do not reach them there."""
-    return torch.is_inference_mode_enabled() and x.is_cuda and _ok(x, x.device, 2) and x.shape[1] % 8 == 0 and \
-        x.shape[1] <= 8192 and _ok(norm_weight, x.device, 1) and norm_weight.shape[0] == x.shape[1]
+    if not (torch.is_inference_mode_enabled() and x.is_cuda and x.dim() == 2):
+        return False
+    T, K = x.shape
+    dev = x.get_device()
+    return K % 8 == 0 and K <= 8192 and _ok(x, dev, T, K) and _ok(norm_weight, dev, K)
 
 
 def supported(x: torch.Tensor, w, rot, heads: int, head_dim: int) -> bool:
     """Whether the layer w (engine.model.Layer) with `heads` query, key and value heads can run on hidden states
     x [T, hidden] with the kernels below: bf16, contiguous, 16-byte aligned tensors of one GPU whose sizes are whole
     tiles. The model's torch operations serve everything else, and raise their own errors for sizes that disagree."""
-    if not (rows_ok(x, w.input_norm) and head_dim % 16 == 0):
+    if not rows_ok(x, w.input_norm):
         return False
     T, hidden = x.shape
-    dev, width, inter = x.device, heads * head_dim, w.down_w.shape[-1]
+    dev, width, inter, attn = x.get_device(), heads * head_dim, w.down_w.shape[-1], w.o_w.shape[-1]
     cos, sin = rot
-    return (hidden % 64 == 0 and inter % 64 == 0 and w.o_w.shape[-1] % 64 == 0 and
-            _ok(w.qkv_w, dev, 2) and tuple(w.qkv_w.shape) == (width, hidden) and
-            _ok(w.qkv_b, dev, 1) and w.qkv_b.shape[0] == width and
-            _ok(w.o_w, dev, 2) and w.o_w.shape[0] == hidden and
-            _ok(w.post_norm, dev, 1) and w.post_norm.shape[0] == hidden and
-            _ok(w.gate_up_w, dev, 2) and tuple(w.gate_up_w.shape) == (2 * inter, hidden) and
-            _ok(w.down_w, dev, 2) and w.down_w.shape[0] == hidden and
-            _ok(cos, dev, 3) and tuple(cos.shape) == (T, 1, head_dim) and
-            _ok(sin, dev, 3) and tuple(sin.shape) == (T, 1, head_dim))
+    return (head_dim % 16 == 0 and hidden % 64 == 0 and inter % 64 == 0 and attn % 64 == 0 and
+            _ok(w.qkv_w, dev, width, hidden) and _ok(w.qkv_b, dev, width) and _ok(w.o_w, dev, hidden, attn) and
+            _ok(w.post_norm, dev, hidden) and _ok(w.gate_up_w, dev, 2 * inter, hidden) and
+            _ok(w.down_w, dev, hidden, inter) and _ok(cos, dev, T, 1, head_dim) and _ok(sin, dev, T, 1, head_dim))
 
 
 @functools.lru_cache(maxsize=1024)

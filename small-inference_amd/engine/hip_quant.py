@@ -21,18 +21,19 @@ def _i64(t: torch.Tensor) -> torch.Tensor:
     return t if (t.dtype == torch.int64 and t.is_contiguous()) else t.to(torch.int64).contiguous()
 
 
-def _require(ok: bool, msg: str) -> None:
-    """The kernels index the pools with the shapes given here: a mismatch is refused before any launch."""
+def _require(ok: bool, msg) -> None:
+    """The kernels index the pools with the shapes given here: a mismatch is refused before any launch. msg: a text, or
+    a function that makes it (formatted only when it is needed)."""
     if not ok:
-        raise ValueError(msg)
+        raise ValueError(msg if isinstance(msg, str) else msg())
 
 
 def _token_pools(x: torch.Tensor, q_pool: torch.Tensor, s_pool: torch.Tensor) -> None:
     T, H, D = x.shape
     _require(q_pool.dim() == 4 and q_pool.shape[0] == H and q_pool.shape[3] == D,
-             f"q_pool {tuple(q_pool.shape)} must be [H={H}, N, B, D={D}]")
+             lambda: f"q_pool {tuple(q_pool.shape)} must be [H={H}, N, B, D={D}]")
     _require(tuple(s_pool.shape) == tuple(q_pool.shape[:3]),
-             f"s_pool {tuple(s_pool.shape)} must be [H, N, B] = {tuple(q_pool.shape[:3])}")
+             lambda: f"s_pool {tuple(s_pool.shape)} must be [H, N, B] = {tuple(q_pool.shape[:3])}")
     _require(q_pool.dtype == torch.int8 and s_pool.dtype == torch.float16, "q_pool must be int8 and s_pool fp16")
     _require(q_pool.is_contiguous() and s_pool.is_contiguous(), "the pools must be contiguous")
 
@@ -47,7 +48,7 @@ def quantize_store_tokens(x: torch.Tensor, blocks: torch.Tensor, offsets: torch.
     if T == 0:
         return
     _require(x.stride(-1) == 1, "x needs a contiguous last dim")
-    _require(blocks.numel() == T and offsets.numel() == T, f"{T} tokens need {T} blocks and offsets")
+    _require(blocks.numel() == T and offsets.numel() == T, lambda: f"{T} tokens need {T} blocks and offsets")
     _token_pools(x, q_pool, s_pool)
     _hip.require_gpu(x, blocks, offsets, q_pool, s_pool)
     blocks, offsets = _i64(blocks), _i64(offsets)
@@ -81,10 +82,10 @@ def quantize_store_blocks(src_pool: torch.Tensor, src: torch.Tensor, dst: torch.
     if src.numel() == 0:
         return
     H, _, B, D = src_pool.shape
-    _require(src.numel() == dst.numel(), f"{src.numel()} sources for {dst.numel()} destinations")
+    _require(src.numel() == dst.numel(), lambda: f"{src.numel()} sources for {dst.numel()} destinations")
     _require(q_pool.dim() == 4 and (q_pool.shape[0], q_pool.shape[2], q_pool.shape[3]) == (H, B, D),
-             f"q_pool {tuple(q_pool.shape)} must be [H={H}, N, B={B}, D={D}]")
-    _require(tuple(s_pool.shape) == (H, q_pool.shape[1], D), f"s_pool {tuple(s_pool.shape)} must be [H, N, D]")
+             lambda: f"q_pool {tuple(q_pool.shape)} must be [H={H}, N, B={B}, D={D}]")
+    _require(tuple(s_pool.shape) == (H, q_pool.shape[1], D), lambda: f"s_pool {tuple(s_pool.shape)} must be [H, N, D]")
     _require(q_pool.dtype == torch.int8 and s_pool.dtype == torch.float16, "q_pool must be int8 and s_pool fp16")
     _require(src_pool.is_contiguous() and q_pool.is_contiguous() and s_pool.is_contiguous(),
              "the pools must be contiguous")
@@ -106,11 +107,11 @@ def quantize_store_block_rows(x: torch.Tensor, rows: torch.Tensor, dst: torch.Te
         return
     H, _, B, D = q_pool.shape
     _require(x.dim() == 3 and x.shape[1] == H and x.shape[2] == D and x.stride(-1) == 1,
-             f"x {tuple(x.shape)} must be [T, H={H}, D={D}] with a contiguous last dim")
-    _require(tuple(s_pool.shape) == (H, q_pool.shape[1], D), f"s_pool {tuple(s_pool.shape)} must be [H, N, D]")
+             lambda: f"x {tuple(x.shape)} must be [T, H={H}, D={D}] with a contiguous last dim")
+    _require(tuple(s_pool.shape) == (H, q_pool.shape[1], D), lambda: f"s_pool {tuple(s_pool.shape)} must be [H, N, D]")
     _require(q_pool.dtype == torch.int8 and s_pool.dtype == torch.float16, "q_pool must be int8 and s_pool fp16")
     _require(q_pool.is_contiguous() and s_pool.is_contiguous(), "the pools must be contiguous")
-    _require(rows.numel() == dst.numel() * B, f"{rows.numel()} rows for {dst.numel()} blocks of {B}")
+    _require(rows.numel() == dst.numel() * B, lambda: f"{rows.numel()} rows for {dst.numel()} blocks of {B}")
     _hip.require_gpu(x, rows, dst, q_pool, s_pool)
     rows, dst = _i64(rows), _i64(dst)
     rc = _hip.lib().sipa_quantize_store_block_rows(
@@ -132,8 +133,8 @@ def store_tokens(x: torch.Tensor, blocks: torch.Tensor, offsets: torch.Tensor, p
     T, H, D = x.shape
     _require(x.stride(-1) == 1 and pool.stride(-1) == 1, "x and the pool need a contiguous last dim")
     _require(pool.dim() == 4 and pool.shape[0] == H and pool.shape[3] == D,
-             f"pool {tuple(pool.shape)} must be [H={H}, N, B, D={D}]")
-    _require(offsets.numel() == n, f"{n} blocks but {offsets.numel()} offsets")
+             lambda: f"pool {tuple(pool.shape)} must be [H={H}, N, B, D={D}]")
+    _require(offsets.numel() == n, lambda: f"{n} blocks but {offsets.numel()} offsets")
     _require(n <= T if rows is None else rows.numel() == n, "one source row per stored token")
     if x2 is not None:
         _require(x2.shape == x.shape and x2.stride(-1) == 1 and x2.dtype == x.dtype,
@@ -152,6 +153,65 @@ def store_tokens(x: torch.Tensor, blocks: torch.Tensor, offsets: torch.Tensor, p
     _hip.check(rc, "store_tokens")
 
 
+def store_layer(layer: int, k: torch.Tensor, v: torch.Tensor, blocks: torch.Tensor, offsets: torch.Tensor,
+                k_pools: torch.Tensor, v_pools: torch.Tensor) -> None:
+    """store_tokens(k, blocks, offsets, k_pools[layer], x2=v, pool2=v_pools[layer]) for pools [L, H, N, B, D], without
+    making the layer's views. One launch."""
+    n = blocks.numel()
+    if n == 0:
+        return
+    T, H, D = k.shape
+    _require(v.shape == k.shape and v.dtype == k.dtype and k.stride(-1) == 1 and v.stride(-1) == 1,
+             "k and v must match in shape and dtype, last dim contiguous")
+    _require(offsets.numel() == n and n <= T, lambda: f"{n} blocks but {offsets.numel()} offsets and {T} rows")
+    shape, strides = k_pools.shape, k_pools.stride()
+    _require(len(shape) == 5 and shape[1] == H and shape[4] == D and strides[4] == 1 and v_pools.shape == shape and
+             v_pools.stride() == strides and v_pools.dtype == k_pools.dtype,
+             lambda: f"pools {tuple(shape)} and {tuple(v_pools.shape)} must both be [L, H={H}, N, B, D={D}]")
+    _hip.require_gpu(k, v, blocks, offsets, k_pools, v_pools)
+    blocks, offsets = _i64(blocks), _i64(offsets)
+    (kt, kh, _), (vt, vh, _) = k.stride(), v.stride()
+    rc = _hip.lib().sipa_store_tokens(
+        k.data_ptr(), v.data_ptr(), _hip.dtype_code(k.dtype), kt, kh, vt, vh, None, n, H, D, blocks.data_ptr(),
+        offsets.data_ptr(), _hip.layer_ptr(k_pools, layer), _hip.layer_ptr(v_pools, layer),
+        _hip.dtype_code(k_pools.dtype), strides[1], strides[2], strides[3], _hip.stream_of(k))
+    if rc:
+        _hip.check(rc, "store_tokens")
+
+
+def quantize_store_layer(layer: int, k: torch.Tensor, v: torch.Tensor, blocks: torch.Tensor, offsets: torch.Tensor,
+                         k_pools: torch.Tensor, k_scales: torch.Tensor, v_pools: torch.Tensor,
+                         v_scales: torch.Tensor) -> None:
+    """quantize_store_tokens of v and k into layer `layer` of pools [L, H, N, B, D] and scales [L, H, N, B], without
+    making the layer's views. One launch."""
+    T, H, D = k.shape
+    if T == 0:
+        return
+    _require(v.shape == k.shape and v.dtype == k.dtype and k.stride(-1) == 1 and v.stride(-1) == 1,
+             "k and v must match in shape and dtype, last dim contiguous")
+    _require(blocks.numel() == T and offsets.numel() == T, lambda: f"{T} tokens need {T} blocks and offsets")
+    shape = k_pools.shape
+    _require(len(shape) == 5 and shape[1] == H and shape[4] == D and v_pools.shape == shape,
+             lambda: f"pools {tuple(shape)} and {tuple(v_pools.shape)} must both be [L, H={H}, N, B, D={D}]")
+    _require(k_scales.shape == shape[:4] and v_scales.shape == shape[:4],
+             lambda: f"scales must be [L, H, N, B] = {tuple(shape[:4])}")
+    _require(k_pools.dtype == torch.int8 and v_pools.dtype == torch.int8 and k_scales.dtype == torch.float16 and
+             v_scales.dtype == torch.float16, "pools must be int8 and scales fp16")
+    _require(k_pools.is_contiguous() and v_pools.is_contiguous() and k_scales.is_contiguous() and
+             v_scales.is_contiguous(), "the pools must be contiguous")
+    _hip.require_gpu(k, v, blocks, offsets, k_pools, v_pools, k_scales, v_scales)
+    blocks, offsets = _i64(blocks), _i64(offsets)
+    (kt, kh, _), (vt, vh, _) = k.stride(), v.stride()
+    _, qh, qn, _, _ = k_pools.stride()
+    _, sh, sn, _ = k_scales.stride()
+    rc = _hip.lib().sipa_quantize_store_tokens_kv(
+        v.data_ptr(), k.data_ptr(), _hip.dtype_code(v.dtype), vt, vh, kt, kh, T, H, D, blocks.data_ptr(),
+        offsets.data_ptr(), _hip.layer_ptr(v_pools, layer), _hip.layer_ptr(k_pools, layer), qh, qn, shape[3],
+        _hip.layer_ptr(v_scales, layer), _hip.layer_ptr(k_scales, layer), sh, sn, _hip.stream_of(v))
+    if rc:
+        _hip.check(rc, "quantize_store_tokens")
+
+
 def kchan_write_rows(k: torch.Tensor, v: torch.Tensor, blocks: torch.Tensor, offsets: torch.Tensor,
                      stage_slots: torch.Tensor, quant_dst: torch.Tensor | None, v_pool: torch.Tensor,
                      v_scale: torch.Tensor, k_pool: torch.Tensor, k_scale: torch.Tensor, stage: torch.Tensor) -> None:
@@ -167,17 +227,17 @@ def kchan_write_rows(k: torch.Tensor, v: torch.Tensor, blocks: torch.Tensor, off
     _require(k.shape == v.shape and k.dtype == v.dtype, "k and v must match in shape and dtype")
     _require(k.stride(-1) == 1 and v.stride(-1) == 1, "k and v need a contiguous last dim")
     _require(blocks.numel() == T and offsets.numel() == T and stage_slots.numel() == T,
-             f"{T} rows need {T} blocks, offsets and staging slots")
-    _require(quant_dst is None or quant_dst.numel() == T, f"quant_dst needs {T} entries")
+             lambda: f"{T} rows need {T} blocks, offsets and staging slots")
+    _require(quant_dst is None or quant_dst.numel() == T, lambda: f"quant_dst needs {T} entries")
     _token_pools(v, v_pool, v_scale)
     N, B = v_pool.shape[1], v_pool.shape[2]
     _require(tuple(k_pool.shape) == tuple(v_pool.shape) and k_pool.dtype == torch.int8 and k_pool.is_contiguous(),
-             f"k_pool {tuple(k_pool.shape)} must be int8 {tuple(v_pool.shape)}, contiguous")
+             lambda: f"k_pool {tuple(k_pool.shape)} must be int8 {tuple(v_pool.shape)}, contiguous")
     _require(tuple(k_scale.shape) == (H, N, D) and k_scale.dtype == torch.float16 and k_scale.is_contiguous(),
-             f"k_scale {tuple(k_scale.shape)} must be fp16 [H={H}, N={N}, D={D}], contiguous")
+             lambda: f"k_scale {tuple(k_scale.shape)} must be fp16 [H={H}, N={N}, D={D}], contiguous")
     _require(stage.dim() == 4 and (stage.shape[0], stage.shape[2], stage.shape[3]) == (H, B, D)
              and stage.dtype == torch.bfloat16 and stage.stride(-1) == 1,
-             f"stage {tuple(stage.shape)} must be bf16 [H={H}, n_stage, B={B}, D={D}]")
+             lambda: f"stage {tuple(stage.shape)} must be bf16 [H={H}, n_stage, B={B}, D={D}]")
     _hip.require_gpu(k, v, blocks, offsets, stage_slots, v_pool, v_scale, k_pool, k_scale, stage)
     blocks, offsets, stage_slots = _i64(blocks), _i64(offsets), _i64(stage_slots)
     if quant_dst is not None:

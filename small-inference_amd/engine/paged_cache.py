@@ -26,6 +26,9 @@ import torch
 from .attention import attention
 from .block_manager import BlockManager
 from .config import ModelConfig
+from .hip_decode import DecodePlan
+from .hip_prefill import paged_prefill_attention, prefill_splits, prefill_supported
+from .hip_quant import store_layer
 
 BACKENDS = ("gather", "hip", "triton")
 KERNEL_BACKENDS = ("hip", "triton")
@@ -156,6 +159,13 @@ def build_metadata(manager: BlockManager, batch: list[tuple[int, int, int]],
     )
 
 
+def _run(seqs: list[int]) -> slice | None:
+    """The slice of increasing indices that are consecutive, None for others: a forward's decode rows (or its chunks)
+    usually stand together, and slices of the metadata and of the rows are views, where lists of indices are uploads,
+    gathers and scatters."""
+    return slice(seqs[0], seqs[-1] + 1) if seqs[-1] - seqs[0] + 1 == len(seqs) else None
+
+
 class PagedKVCache:
     def __init__(self, cfg: ModelConfig, num_blocks: int, block_size: int, device: str | torch.device,
                  dtype: torch.dtype, attn_backend: str = "gather"):
@@ -208,13 +218,10 @@ class PagedKVCache:
             pf = self._prefill
             host = [meta.query_starts[i] for i in pf] + [per_seq[i] for i in pf]
             rows = torch.tensor(host, dtype=torch.int32).to(self.device, non_blocking=True)
-            if len(pf) == meta.num_seqs:
-                bt, ctx = meta.block_tables, meta.context_lens_t
-            else:
+            idx = _run(pf)
+            if idx is None:
                 idx = torch.tensor(pf, device=meta.positions.device)
-                bt, ctx = meta.block_tables[idx], meta.context_lens_t[idx]
-            from .hip_prefill import prefill_splits
-
+            bt, ctx = meta.block_tables[idx], meta.context_lens_t[idx]
             max_ctx = max(meta.context_lens[i] for i in pf)
             cfg = self.cfg
             splits = prefill_splits(cfg.num_q_heads, cfg.num_kv_heads, cfg.head_dim, [per_seq[i] for i in pf], max_ctx)
@@ -226,6 +233,9 @@ class PagedKVCache:
             # Once per forward, shared by every layer: the decode rows and their slice of the metadata.
             if len(dec) == meta.num_seqs:
                 rows, bt, ctx = None, meta.block_tables, meta.context_lens_t
+            elif (idx := _run(dec)) is not None:  # one token each: consecutive rows too
+                first = meta.query_starts[idx.start]
+                rows, bt, ctx = slice(first, first + len(dec)), meta.block_tables[idx], meta.context_lens_t[idx]
             else:
                 idx = torch.tensor(dec, device=meta.positions.device)
                 rows, bt, ctx = meta.last_token_indices[idx], meta.block_tables[idx], meta.context_lens_t[idx]
@@ -236,9 +246,7 @@ class PagedKVCache:
         """Scatter this forward's k, v [T, H_kv, d] into their slots."""
         m = self.meta
         if self.on_gpu:
-            from .hip_quant import store_tokens
-
-            store_tokens(k, m.slot_blocks, m.slot_offsets, self.k[layer], x2=v, pool2=self.v[layer])
+            store_layer(layer, k, v, m.slot_blocks, m.slot_offsets, self.k, self.v)
             return
         self.k[layer][:, m.slot_blocks, m.slot_offsets] = k.transpose(0, 1)
         self.v[layer][:, m.slot_blocks, m.slot_offsets] = v.transpose(0, 1)
@@ -267,16 +275,12 @@ class PagedKVCache:
     def _prefill_kernel_ok(self, max_context: int) -> bool:
         """Whether this forward's multi-token rows can run the paged prefill kernel (bf16 model, bf16 or INT8 pool,
         16-token blocks, head_dim 64/128, group <= 8, contexts <= 32768)."""
-        from .hip_prefill import prefill_supported
-
         cfg = self.cfg
         return prefill_supported(self.dtype, self.k.dtype, self.block_size, cfg.head_dim,
                                  cfg.num_q_heads // cfg.num_kv_heads, max_context)
 
     def _attend_prefill(self, layer: int, q: torch.Tensor, scale: float, out: torch.Tensor) -> None:
         """Multi-token rows of the forward, written into their rows of out [T, Hq, d] by the prefill kernel."""
-        from .hip_prefill import paged_prefill_attention
-
         bt, ctx, qs, ql, max_ctx, max_q, splits = self._prefill_launch
         paged_prefill_attention(q, self.k[layer], self.v[layer], bt, ctx, qs, ql, scale, max_ctx, max_q, out=out,
                                 num_splits=splits, quant=self._prefill_quant(layer))
@@ -296,28 +300,34 @@ class PagedKVCache:
                 return out.view(T, Hq * d)
             outs = [self._attend_gather(layer, i, q, positions, scale) for i in range(m.num_seqs)]
             return outs[0] if len(outs) == 1 else torch.cat(outs)
-        from .hip_decode import DecodePlan
-
         rows, bt, ctx, lens = self._decode
+        # Consecutive decode rows are read and written in place; others are gathered and scattered.
+        in_place = type(rows) is slice
+        out = None if rows is None else torch.empty(T, Hq * d, device=q.device, dtype=q.dtype)
         q_dec = q if rows is None else q[rows]
-        quant = self._kernel_quant(layer)
+        dec_out = out[rows].view(-1, Hq, d) if in_place else None
         if self._plan is None or self._plan_scale != scale:  # first layer of the forward: validate once
             # The host-side lengths let a ragged batch run from a work list (built once, used by every layer).
-            self._plan = DecodePlan(q_dec, self.k[layer], self.v[layer], bt, ctx, scale, max(lens), quant=quant,
-                                    host_context_lens=lens)
+            self._plan = DecodePlan(q_dec, self.k[layer], self.v[layer], bt, ctx, scale, max(lens),
+                                    quant=self._kernel_quant(layer), host_context_lens=lens)
             self._plan_scale = scale
-            dec = self._plan()
+            self._quant_pools = self._all_quant()
+            dec = self._plan(out=dec_out)
         else:
-            dec = self._plan(q=q_dec, k_cache=self.k[layer], v_cache=self.v[layer], quant=quant)
+            dec = self._plan.run_layer(layer, q_dec, self.k, self.v, self._quant_pools, dec_out)
         if rows is None:
             return dec.view(T, Hq * d)
-        out = torch.empty(T, Hq * d, device=q.device, dtype=q.dtype)
-        out[rows] = dec.view(-1, Hq * d)
+        if not in_place:
+            out[rows] = dec.view(-1, Hq * d)
         if self._prefill_launch is not None:
             self._attend_prefill(layer, q, scale, out.view(T, Hq, d))
         for i in self._prefill:
             out[m.query_starts[i]:m.query_starts[i + 1]] = self._attend_gather(layer, i, q, positions, scale)
         return out
+
+    def _all_quant(self):
+        """_kernel_quant's inputs for every layer (a leading layer dimension); None for the model-dtype pool."""
+        return None
 
     def _kernel_quant(self, layer: int):
         """Extra kernel inputs of INT8 caches; None for the model-dtype pool."""

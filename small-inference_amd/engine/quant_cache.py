@@ -27,7 +27,9 @@ import torch
 from .block_manager import BlockManager
 from .config import ModelConfig
 from .hip_decode import QuantKV
-from .paged_cache import PagedKVCache, PagedMetadata
+from .hip_quant import (kchan_write_rows, quantize_store_block_rows, quantize_store_blocks, quantize_store_layer,
+                        quantize_store_tokens, store_tokens)
+from .paged_cache import PagedKVCache, PagedMetadata, _run
 from .quant import dequantize, quantize_per_channel, quantize_per_token
 
 FORMATS = ("bf16", "int8", "int8-kchannel")
@@ -239,7 +241,8 @@ class QuantPagedKVCache(PagedKVCache):
         """per_seq restricted to the sequences a kernel launch of this forward covers (all of them: itself)."""
         if used is None or seqs is None or len(seqs) == per_seq.numel():
             return per_seq
-        return per_seq[torch.tensor(seqs, device=dev)]
+        run = _run(seqs)
+        return per_seq[run if run is not None else torch.tensor(seqs, device=dev)]
 
     # ---- writes ------------------------------------------------------------------------------------------------
 
@@ -287,13 +290,9 @@ class QuantPagedKVCache(PagedKVCache):
 
     def _write_fused(self, layer: int, k: torch.Tensor, v: torch.Tensor) -> None:
         """write() through the HIP kernels: one launch per step below."""
-        from .hip_quant import (kchan_write_rows, quantize_store_block_rows, quantize_store_blocks,
-                                quantize_store_tokens, store_tokens)
-
         m = self.meta
         if self.fmt == "int8":  # V and K in one launch
-            quantize_store_tokens(v, m.slot_blocks, m.slot_offsets, self.v[layer], self.v_scale[layer],
-                                  x2=k, q_pool2=self.k[layer], s_pool2=self.k_scale[layer])
+            quantize_store_layer(layer, k, v, m.slot_blocks, m.slot_offsets, self.k, self.k_scale, self.v, self.v_scale)
             return
         if self._rows_write is not None:  # a decode step: V, the K staging store and completed blocks in one launch
             slots, dst = self._rows_write
@@ -339,3 +338,8 @@ class QuantPagedKVCache(PagedKVCache):
         if self.fmt == "int8":
             return QuantKV(1, self.k_scale[layer], self.v_scale[layer])
         return QuantKV(2, self.k_scale[layer], self.v_scale[layer], self.stage[layer], self._tails_dec)
+
+    def _all_quant(self) -> QuantKV:
+        if self.fmt == "int8":
+            return QuantKV(1, self.k_scale, self.v_scale)
+        return QuantKV(2, self.k_scale, self.v_scale, self.stage, self._tails_dec)

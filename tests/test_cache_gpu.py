@@ -149,3 +149,51 @@ def test_model_mixed_batch_kernel_vs_gather():
         ids = torch.tensor([5] + list(range(20, 33)) + [7], device="cuda")
         outs[backend] = model.forward(ids, meta.positions, cache, meta, last_only=False)
     torch.testing.assert_close(outs["triton"], outs["gather"], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "int8", "int8-kchannel"])
+@pytest.mark.parametrize("order", ["decodes first", "chunks first", "interleaved"])
+def test_rows_in_any_order_match_the_gather_backend(fmt, order):
+    """A packed forward of decode rows and chunks over two layers: consecutive rows of a kind are read and written in
+    place, others through gathers; each order's rows equal the same rows computed by a forward of their own."""
+    from engine.quant_cache import QuantPagedKVCache
+
+    cfg = ModelConfig(vocab_size=64, hidden_size=896, intermediate_size=64, num_layers=2, num_q_heads=14, num_kv_heads=2,
+                      head_dim=64)
+    dec, chunks = [(0, 40, 1), (1, 63, 1), (2, 200, 1)], [(3, 0, 37), (4, 100, 20)]
+    batch = {"decodes first": dec + chunks, "chunks first": chunks + dec,
+             "interleaved": [dec[0], chunks[0], dec[1], chunks[1], dec[2]]}[order]
+    results = []
+    for together in (True, False):
+        m = fragmented_manager(128, 16, torch.Generator().manual_seed(1))
+        g = torch.Generator(device="cuda").manual_seed(2)
+        if fmt == "bf16":
+            cache = PagedKVCache(cfg, m.num_blocks, 16, "cuda", torch.bfloat16, attn_backend="hip")
+        else:
+            cache = QuantPagedKVCache(cfg, m.num_blocks, 16, "cuda", torch.bfloat16, "hip", fmt, m, n_stage=32)
+        for s, start, n in sorted(dec + chunks):  # the contexts so far, written through the cache
+            m.allocate(s, start + n)
+            if start:
+                meta = build_metadata(m, [(s, 0, start)], "cuda")
+                cache.begin(start, meta)
+                for layer in range(2):
+                    cache.write(layer, *torch.randn(2, start, 2, 64, generator=g, device="cuda").bfloat16())
+        rows = {s: torch.randn(2, 18, n, 64, generator=g, device="cuda").bfloat16() for s, _, n in sorted(dec + chunks)}
+        outs = {}
+        for b in ([batch] if together else [[x] for x in batch]):
+            T = sum(n for _, _, n in b)
+            meta = build_metadata(m, b, "cuda")
+            cache.begin(T, meta)
+            for layer in range(2):
+                x = torch.cat([rows[s][layer].transpose(0, 1) for s, _, _ in b])  # [T, 18, 64]
+                cache.write(layer, x[:, 14:16], x[:, 16:])
+                out = cache.attend(layer, x[:, :14], meta.positions, 0.125)
+                at = 0
+                for s, _, n in b:
+                    outs[s, layer] = out[at:at + n].clone()
+                    at += n
+        results.append(outs)
+    for key, a in results[0].items():
+        b = results[1][key]
+        # other split counts, another order of fp32 sums: a bf16 step of outputs below 4
+        assert (a.float() - b.float()).abs().max() <= 2.0 ** -6, key

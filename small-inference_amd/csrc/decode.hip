@@ -718,6 +718,8 @@ extern "C" int32_t sipa_decode_split_grid(int32_t num_seqs, int32_t num_kv_heads
   return splits;
 }
 
+constexpr int kMaxPairPieces = 32;
+
 extern "C" int32_t sipa_build_work_list(const int32_t* ctx, int32_t S, int32_t Hkv, int32_t cu_count,
                                         int32_t items_per_cu, int32_t max_piece, int32_t* items, int32_t capacity,
                                         int32_t* max_splits) {
@@ -736,9 +738,13 @@ extern "C" int32_t sipa_build_work_list(const int32_t* ctx, int32_t S, int32_t H
   // The smallest piece: 512 tokens (small ragged batches, bf16: a 16,000-token sequence of 8 cut into 256-token
   // pieces merged 63 partials, 15.1 us, into 512-token ones 32, 12.3 us); 256 for the INT8 kernels, which pass
   // their 4096-token cap (their small batches: 10.5 us at 256 against 12.1 at 512).
-  const int min_piece = (max_piece > 0 && max_piece <= kMaxInt8Split) ? kMinChunk : kLatencyChunk;
-  piece = std::min<int64_t>(std::max<int64_t>((piece + kChunkAlign - 1) / kChunkAlign * kChunkAlign, min_piece),
-                            cap / kChunkAlign * kChunkAlign);
+  int64_t min_piece = (max_piece > 0 && max_piece <= kMaxInt8Split) ? kMinChunk : kLatencyChunk;
+  // and at most kMaxPairPieces pieces of the longest sequence, two rounds of its merge (14 INT8 sequences of up to 16384
+  // tokens: 52 pieces of 320 30.4 us, 32 of 512 21.4)
+  const int longest = S > 0 ? *std::max_element(ctx, ctx + S) : 0;
+  min_piece = std::min(cap, std::max<int64_t>(min_piece, ceil_div(longest, kMaxPairPieces)));
+  piece = std::max(piece, min_piece);
+  piece = std::min<int64_t>((piece + kChunkAlign - 1) / kChunkAlign * kChunkAlign, cap / kChunkAlign * kChunkAlign);
   struct Item {
     int32_t s, h, sp, n, start, end;
   };

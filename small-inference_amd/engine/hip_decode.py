@@ -75,7 +75,8 @@ def build_work_list(context_lens: list[int], num_kv_heads: int, cu_count: int | 
                     items_per_cu: int = 3, max_piece: int = 0) -> tuple[np.ndarray, int]:
     """Work list for a ragged batch from host-side context lengths: ([n, 8] int32 items, largest split count of
     a pair). Each (sequence, KV head) pair is cut into near-equal pieces of about sum(ctx) * Hkv /
-    (cu_count * items_per_cu) tokens (at most max_piece; 0: 32768); items are ordered longest first. Three items
+    (cu_count * items_per_cu) tokens (at most max_piece; 0: 32768; max_piece aside, at most 32 a
+    pair); items are ordered longest first. Three items
     per CU measured best on MI355X (C3 ragged 256: 30.4 -> 29.4 us against two; 512 x U[1024, 16384]: 390 -> 382 us;
     four to six were no better)."""
     cu = device_cu_count() if cu_count is None else cu_count

@@ -163,6 +163,15 @@ def test_work_list_partitions_every_pair(seed):
     assert maxs == max(len(ps) for ps in pieces.values())
 
 
+@pytest.mark.parametrize("longest", [8192, 8193, 16384, 100_000, 140_000])
+def test_work_list_caps_the_pieces_of_a_pair(longest):
+    """At most 32 pieces of the longest sequence unless max_piece makes more necessary."""
+    items, maxs = work_list([longest] + [64] * 13, 2, max_piece=4096)
+    assert maxs <= max(32, -(-longest // 4096))
+    first = [i for i in items if i[0] == 0 and i[1] == 0]
+    assert len(first) == maxs and sum(i[5] - i[4] for i in first) == longest
+
+
 def test_work_list_piece_size_and_errors():
     """Pieces are about total / (cu * items_per_cu) tokens, at least 256; bad lengths and short buffers fail."""
     items, maxs = work_list([8192] * 32, 2, cu=256, per_cu=2)  # 524288 token-heads / 512 -> 1024-token pieces

@@ -493,6 +493,15 @@ typedef struct sipa_linear_params {
   void* scratch;
   int64_t scratch_bytes;
   void* counters;
+  /* ROPE, kv_heads > 0: the last rotated heads (K) and the heads after them (V), kv_heads each, are stored to the paged
+   * pools [kv_heads, N, B, head_dim] at (kv_blocks[t], kv_offsets[t]) instead of to out, as sipa_store_tokens stores
+   * them (indices as given) */
+  int32_t kv_heads;
+  void* k_pool;
+  void* v_pool;
+  int64_t kv_stride_h, kv_stride_n, kv_stride_b;
+  const int64_t* kv_blocks;
+  const int64_t* kv_offsets;
 } sipa_linear_params;
 
 int32_t sipa_fused_linear(const sipa_linear_params* p, void* stream);

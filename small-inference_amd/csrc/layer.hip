@@ -37,6 +37,12 @@ struct LinearArgs {
   const uint16_t* cos;     // [T, D] (ROPE)
   const uint16_t* sin;     // [T, D], the sign of rotate-half folded in
   int32_t T, K, D, rot;    // rot: output channels that are rotated (whole heads, the first ones)
+  // ROPE: the K and V channels (from kv0 on, kv_heads heads each) go straight to the paged pools [heads, blocks, offsets,
+  // D] instead of out, token t at (blocks[t], offsets[t]); kv_heads 0: everything to out
+  int32_t kv_heads, kv0;
+  uint16_t *k_pool, *v_pool;
+  int64_t kv_sh, kv_sn, kv_sb;
+  const int64_t *blocks, *offsets;
   int32_t tiles;           // row tiles in all
   int32_t inter;           // SILU: gate rows (the up rows follow)
   int32_t units;           // 64-channel slices of K a workgroup takes
@@ -54,6 +60,21 @@ __device__ __forceinline__ int linear_row(const LinearArgs& a, int tile, int r) 
     return head * a.D + c0 + (r & 7) + (r < 8 ? 0 : a.D >> 1);
   }
   return tile * 16 + r;
+}
+
+// Where channel c of token t is stored. K and V straight to the pools: a separate store launch took 2.5 to 3.8 us a layer
+// (kernel and the gap before it) for a few KB; without it a replayed 24-layer step of 8 sequences takes 889 us, 950 with it,
+// and 24 layers over 544 mixed tokens 2230 us, 2306 with it.
+template <int EPI>
+__device__ __forceinline__ uint16_t* out_at(const LinearArgs& a, int t, int c) {
+  if (EPI == kEpiRope && a.kv_heads > 0 && c >= a.kv0) {
+    int h = (c - a.kv0) / a.D;
+    const int ch = c - a.kv0 - h * a.D;
+    uint16_t* pool = a.k_pool;
+    if (h >= a.kv_heads) h -= a.kv_heads, pool = a.v_pool;
+    return pool + h * a.kv_sh + a.blocks[t] * a.kv_sn + a.offsets[t] * a.kv_sb + ch;
+  }
+  return a.out + t * a.out_st + c;
 }
 
 // x / (1 + e^-x) in fp32: the hardware's exp2 and reciprocal, each within an ulp or two, 2^-8 of the bf16 step the
@@ -171,8 +192,8 @@ __global__ void __launch_bounds__(64 * kSkinnyWaves) skinny_linear(const LinearA
     lo += bf16_bits_to_f32(a.res[t * a.res_st + nlo]);
     hi += bf16_bits_to_f32(a.res[t * a.res_st + nhi]);
   }
-  a.out[t * a.out_st + nlo] = f32_to_bf16_bits(lo);
-  a.out[t * a.out_st + nhi] = f32_to_bf16_bits(hi);
+  *out_at<EPI>(a, t, nlo) = f32_to_bf16_bits(lo);
+  *out_at<EPI>(a, t, nhi) = f32_to_bf16_bits(hi);
 }
 
 // ---- tile_linear: everything else -----------------------------------------------------------------------------------------
@@ -377,7 +398,7 @@ __global__ void __launch_bounds__(256) tile_linear(const LinearArgs a) {
         if (EPI == kEpiResidual && a.res != nullptr && t < a.T) v += unpack(*(const uint2*)(a.res + t * a.res_st + c));
       }
       if (!in || t >= a.T) continue;
-      *(uint2*)(a.out + t * a.out_st + c) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      *(uint2*)out_at<EPI>(a, t, c) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
     }
   }
 }
@@ -590,6 +611,12 @@ static int check_linear(const sipa_linear_params* p) {
     SIPA_CHECK(p->rot_channels >= 0 && p->rot_channels <= N && p->rot_channels % p->head_dim == 0, SIPA_EINVAL,
                "linear: %d rotated channels", p->rot_channels);
   }
+  SIPA_CHECK(p->kv_heads >= 0 && (p->kv_heads == 0 || p->epilogue == SIPA_LINEAR_ROPE), SIPA_EINVAL,
+             "linear: only the rotary epilogue stores to K and V pools");
+  SIPA_CHECK(p->kv_heads == 0 || (p->kv_heads <= (1 << 16) && p->rot_channels >= p->kv_heads * p->head_dim &&
+                                  N == p->rot_channels + p->kv_heads * p->head_dim),
+             SIPA_EINVAL, "linear: %d K and V heads of %d channels do not end %d rotated of %d channels", p->kv_heads,
+             p->head_dim, p->rot_channels, N);
   SIPA_CHECK(p->num_splits <= 1 || (p->epilogue == SIPA_LINEAR_RESIDUAL && p->norm_weight == nullptr), SIPA_EINVAL,
              "linear: only the residual epilogue without norm splits K");
   return SIPA_OK;
@@ -624,8 +651,20 @@ extern "C" int32_t sipa_fused_linear(const sipa_linear_params* p, void* stream) 
   SIPA_CHECK(p->epilogue != SIPA_LINEAR_SILU || p->bias == nullptr, SIPA_EINVAL, "linear: no bias with SiLU");
   SIPA_CHECK(p->epilogue != SIPA_LINEAR_ROPE || p->rot_channels == 0 || (p->rot_cos && p->rot_sin), SIPA_EINVAL,
              "linear: rotary tables missing");
+  SIPA_CHECK(p->kv_heads == 0 || (p->k_pool && p->v_pool && p->kv_blocks && p->kv_offsets), SIPA_EINVAL,
+             "linear: K and V pools or slots missing");
+  SIPA_CHECK(p->kv_heads == 0 || (aligned8(p->k_pool) && aligned8(p->v_pool) && p->kv_stride_h % 4 == 0 &&
+                                  p->kv_stride_n % 4 == 0 && p->kv_stride_b % 4 == 0),
+             SIPA_EUNSUPPORTED, "linear: K and V pools need 8-byte rows");
   const LinearPlan plan = plan_of(p);
   LinearArgs a{};
+  a.kv_heads = p->kv_heads;
+  if (p->kv_heads > 0) {
+    a.kv0 = p->rot_channels - p->kv_heads * p->head_dim;
+    a.k_pool = (uint16_t*)p->k_pool, a.v_pool = (uint16_t*)p->v_pool;
+    a.kv_sh = p->kv_stride_h, a.kv_sn = p->kv_stride_n, a.kv_sb = p->kv_stride_b;
+    a.blocks = p->kv_blocks, a.offsets = p->kv_offsets;
+  }
   a.x = (const uint16_t*)p->x, a.x_st = p->x_stride, a.w = (const uint16_t*)p->weight;
   a.norm_w = (const uint16_t*)p->norm_weight, a.eps = p->eps, a.bias = (const uint16_t*)p->bias;
   a.res = (const uint16_t*)p->residual, a.res_st = p->res_stride;

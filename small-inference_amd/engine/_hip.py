@@ -90,6 +90,8 @@ class LinearParams(ctypes.Structure):
         ("x", vp), ("x_stride", i64), ("weight", vp), ("norm_weight", vp), ("bias", vp),
         ("residual", vp), ("res_stride", i64), ("out", vp), ("out_stride", i64), ("rot_cos", vp), ("rot_sin", vp),
         ("num_splits", i32), ("tile", i32), ("scratch", vp), ("scratch_bytes", i64), ("counters", vp),
+        ("kv_heads", i32), ("k_pool", vp), ("v_pool", vp), ("kv_stride_h", i64), ("kv_stride_n", i64),
+        ("kv_stride_b", i64), ("kv_blocks", vp), ("kv_offsets", vp),
     ]
 
 

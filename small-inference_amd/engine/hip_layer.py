@@ -75,10 +75,11 @@ def _linear_scratch(epilogue: int, norm: bool, T: int, K: int, N: int, head_dim:
 def fused_linear(x: torch.Tensor, weight: torch.Tensor, epilogue: int, *, norm_weight: torch.Tensor | None = None,
                  eps: float = 0.0, bias: torch.Tensor | None = None, residual: torch.Tensor | None = None,
                  rot: tuple[torch.Tensor, torch.Tensor] | None = None, head_dim: int = 0, rot_channels: int = 0,
-                 num_splits: int = 0, tile: int = 0) -> torch.Tensor:
+                 num_splits: int = 0, tile: int = 0, store: tuple | None = None) -> torch.Tensor:
     """epilogue(norm(x) W^T) in one launch (sipa_fused_linear): x [T, K], weight [N, K]; RESIDUAL adds bias and
     residual, ROPE adds bias and rotates the first rot_channels channels by rot = (cos, signed sin), SILU multiplies
-    the second half of the channels by silu of the first. num_splits, tile: 0 for the library's choice."""
+    the second half of the channels by silu of the first. num_splits, tile: 0 for the library's choice. store (ROPE):
+    PagedKVCache.store_target's tuple; the K and V channels then go to the pools and are undefined in the result."""
     T, K = x.shape
     N = weight.shape[0]
     out = torch.empty(T, N // 2 if epilogue == SILU else N, device=x.device, dtype=torch.bfloat16)
@@ -92,7 +93,7 @@ def fused_linear(x: torch.Tensor, weight: torch.Tensor, epilogue: int, *, norm_w
                           x.data_ptr(), x.stride(0), weight.data_ptr(), _hip.ptr(norm_weight), _hip.ptr(bias),
                           _hip.ptr(residual), residual.stride(0) if residual is not None else 0, out.data_ptr(),
                           out.stride(0), *((rot[0].data_ptr(), rot[1].data_ptr()) if rot is not None else (None, None)),
-                          num_splits, tile, _hip.ptr(scratch), n, counters)
+                          num_splits, tile, _hip.ptr(scratch), n, counters, *(store or ()))
     _hip.check(_hip.lib().sipa_fused_linear(ctypes.byref(p), stream), "fused_linear")
     return out
 
@@ -123,12 +124,15 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def layer_qkv(x: torch.Tensor, w, eps: float, rot, rotated: int, head_dim: int) -> torch.Tensor:
+def layer_qkv(x: torch.Tensor, w, eps: float, rot, rotated: int, head_dim: int, store: tuple | None = None) -> torch.Tensor:
     """[T, heads * head_dim]: the fused projection of the normalised x, its first `rotated` heads (queries and keys)
-    rotated. One launch up to MAX_TOKENS."""
-    if x.shape[0] <= MAX_TOKENS:
-        return fused_linear(x, w.qkv_w, ROPE, norm_weight=w.input_norm, eps=eps, bias=w.qkv_b, rot=rot,
-                            head_dim=head_dim, rot_channels=rotated * head_dim)
+    rotated; with store, K and V in the cache's pools instead. One launch, up to MAX_TOKENS."""
+    return fused_linear(x, w.qkv_w, ROPE, norm_weight=w.input_norm, eps=eps, bias=w.qkv_b, rot=rot, head_dim=head_dim,
+                        rot_channels=rotated * head_dim, store=store)
+
+
+def layer_qkv_large(x: torch.Tensor, w, eps: float, rot, rotated: int, head_dim: int) -> torch.Tensor:
+    """The same for more tokens, the product in the GEMM library: three launches."""
     qkv = F.linear(rms_norm(x, w.input_norm, eps), w.qkv_w, w.qkv_b)
     rope_(qkv, rot, rotated, head_dim)
     return qkv

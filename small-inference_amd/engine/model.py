@@ -86,8 +86,16 @@ class Qwen2Model:
         cfg, w = self.cfg, self.layers[i]
         T, Hq, Hkv, d = x.shape[0], cfg.num_q_heads, cfg.num_kv_heads, cfg.head_dim
         if hip_layer.supported(x, w, rot, Hq + 2 * Hkv, d):
-            qkv = hip_layer.layer_qkv(x, w, cfg.rms_norm_eps, rot, Hq + Hkv, d).view(T, Hq + 2 * Hkv, d)
-            cache.write(i, qkv[:, Hq:Hq + Hkv], qkv[:, Hq + Hkv:])
+            store = None
+            if T > hip_layer.MAX_TOKENS:
+                qkv = hip_layer.layer_qkv_large(x, w, cfg.rms_norm_eps, rot, Hq + Hkv, d)
+            else:
+                target = getattr(cache, "store_target", None)  # caches that take K and V straight from the projection
+                store = target(i, x, Hkv, d) if target is not None else None
+                qkv = hip_layer.layer_qkv(x, w, cfg.rms_norm_eps, rot, Hq + Hkv, d, store)
+            qkv = qkv.view(T, Hq + 2 * Hkv, d)
+            if store is None:
+                cache.write(i, qkv[:, Hq:Hq + Hkv], qkv[:, Hq + Hkv:])
             return hip_layer.layer_out(x, cache.attend(i, qkv[:, :Hq], positions, self.scale), w, cfg.rms_norm_eps)
         qkv = F.linear(rms_norm(x, w.input_norm, cfg.rms_norm_eps), w.qkv_w, w.qkv_b)
         qk = rotate(qkv[:, :cfg.q_size + cfg.kv_size].view(T, Hq + Hkv, d), *rot)

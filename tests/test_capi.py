@@ -333,6 +333,10 @@ def bad_linear(**over):
     (dict(num_splits=2, epilogue=2), _hip.EINVAL), (dict(num_splits=65), _hip.EINVAL), (dict(tile=7), _hip.EINVAL),
     (dict(tile=6, num_tokens=17), _hip.EUNSUPPORTED), (dict(tile=6, in_features=1600, x_stride=1600), _hip.EUNSUPPORTED),
     (dict(bias=4100), _hip.EUNSUPPORTED), (dict(residual=4096, res_stride=894), _hip.EUNSUPPORTED),
+    (dict(kv_heads=2), _hip.EINVAL), (dict(epilogue=1, rot_channels=1024, kv_heads=3), _hip.EINVAL),
+    (dict(epilogue=1, rot_channels=1024, kv_heads=2), _hip.EINVAL),  # no pools
+    (dict(epilogue=1, rot_channels=1024, kv_heads=2, k_pool=4096, v_pool=4096, kv_blocks=4096, kv_offsets=4096,
+          kv_stride_b=66), _hip.EUNSUPPORTED),
     (dict(num_tokens=-1), _hip.EINVAL)])
 def test_fused_linear_refuses_bad_arguments(over, code):
     assert _hip.lib().sipa_fused_linear(ctypes.byref(bad_linear(**over)), None) == code

@@ -176,3 +176,56 @@ def test_rotate_reference_matches_the_model():
     g = torch.Generator(device="cuda").manual_seed(9)
     x, rot = randn(g, 5, 3, 32), (randn(g, 5, 1, 32), randn(g, 5, 1, 32))
     assert rel(rotate(x, *rot), rotate64(x.double(), *rot)) < BOUND
+
+
+@pytest.mark.parametrize("T", [1, 16, 17, 64, 300])
+@pytest.mark.parametrize("d,Hq,Hkv", [(64, 14, 2), (128, 12, 2), (16, 4, 4)])
+def test_projection_stores_to_the_paged_pools(T, d, Hq, Hkv):
+    """K and V stored by the projection: the bits that the projection without pools and store_tokens give, nothing else
+    in the pools touched, and the same queries."""
+    from engine.hip_quant import store_tokens
+
+    hidden, heads = 320, Hq + 2 * Hkv
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x, nw, w, b = randn(g, T, hidden), 1 + 0.1 * randn(g, hidden), randn(g, heads * d, hidden) * 0.05, randn(g, heads * d)
+    rot = randn(g, T, 1, d), randn(g, T, 1, d)
+    cfg = ModelConfig(vocab_size=64, hidden_size=hidden, intermediate_size=64, num_layers=3, num_q_heads=Hq,
+                      num_kv_heads=Hkv, head_dim=d)
+    m = fragmented_manager(64, 16, torch.Generator().manual_seed(4))
+    cache = PagedKVCache(cfg, m.num_blocks, 16, "cuda", torch.bfloat16, attn_backend="hip")
+    m.allocate(0, T + 5)
+    meta = build_metadata(m, [(0, 5, T)], "cuda")
+    cache.begin(T, meta)
+    cache.k.fill_(7)
+    cache.v.fill_(9)
+    kw = dict(norm_weight=nw, eps=EPS, bias=b, rot=rot, head_dim=d, rot_channels=(Hq + Hkv) * d)
+    store = cache.store_target(1, x, Hkv, d)
+    q = hip_layer.fused_linear(x, w, hip_layer.ROPE, store=store, **kw).view(T, heads, d)[:, :Hq]
+    ref = hip_layer.fused_linear(x, w, hip_layer.ROPE, **kw).view(T, heads, d)
+    k, v = torch.full_like(cache.k, 7), torch.full_like(cache.v, 9)
+    store_tokens(ref[:, Hq:Hq + Hkv], meta.slot_blocks, meta.slot_offsets, k[1], x2=ref[:, Hq + Hkv:], pool2=v[1])
+    assert torch.equal(q, ref[:, :Hq]) and torch.equal(cache.k, k) and torch.equal(cache.v, v)
+
+
+def test_caches_that_write_their_own_way_are_asked_to():
+    cfg = ModelConfig(vocab_size=64, hidden_size=896, intermediate_size=64, num_layers=1, num_q_heads=14, num_kv_heads=2,
+                      head_dim=64)
+    m = fragmented_manager(64, 16, torch.Generator().manual_seed(4))
+
+    class Own(PagedKVCache):
+        def write(self, layer, k, v):
+            super().write(layer, k, v)
+
+    x = torch.zeros(4, 896, device="cuda", dtype=torch.bfloat16)
+    m.allocate(0, 4)
+    meta = build_metadata(m, [(0, 0, 4)], "cuda")
+    for make, dtype, taken in ((PagedKVCache, torch.bfloat16, True), (Own, torch.bfloat16, False),
+                               (PagedKVCache, torch.float32, False)):
+        cache = make(cfg, m.num_blocks, 16, "cuda", dtype, attn_backend="hip")
+        assert cache.store_target(0, x, 2, 64) is None  # no forward begun
+        cache.begin(4, meta)
+        assert (cache.store_target(0, x, 2, 64) is not None) == taken
+        assert cache.store_target(0, x[:3], 2, 64) is None and cache.store_target(0, x, 4, 64) is None
+        assert cache.store_target(0, x.cpu(), 2, 64) is None
+        cache.write = lambda layer, k, v: None
+        assert cache.store_target(0, x, 2, 64) is None

@@ -61,6 +61,15 @@ def supported(x: torch.Tensor, w, rot, heads: int, head_dim: int) -> bool:
             _ok(w.down_w, dev, hidden, inter) and _ok(cos, dev, T, 1, head_dim) and _ok(sin, dev, T, 1, head_dim))
 
 
+def attention_ok(attn: torch.Tensor, x: torch.Tensor, w) -> bool:
+    """Whether layer_out can read attn, what a cache's attend returned for a supported layer w: bf16 rows [T, o_w's
+    features] on x's device, 16-byte aligned. The kernels take its size for the projection's, so one that differs would
+    be read past its end."""
+    return type(attn) in _PLAIN and attn.dtype is torch.bfloat16 and attn.get_device() == x.get_device() and \
+        attn.shape == (x.shape[0], w.o_w.shape[1]) and attn.stride(1) == 1 and attn.stride(0) >= attn.shape[1] and \
+        attn.stride(0) % 8 == 0 and attn.data_ptr() % 16 == 0
+
+
 @functools.lru_cache(maxsize=1024)
 def _linear_scratch(epilogue: int, norm: bool, T: int, K: int, N: int, head_dim: int, num_splits: int, tile: int) -> int:
     p = _hip.LinearParams(struct_size=ctypes.sizeof(_hip.LinearParams), epilogue=epilogue, num_tokens=T, in_features=K,

@@ -96,13 +96,17 @@ class Qwen2Model:
             qkv = qkv.view(T, Hq + 2 * Hkv, d)
             if store is None:
                 cache.write(i, qkv[:, Hq:Hq + Hkv], qkv[:, Hq + Hkv:])
-            return hip_layer.layer_out(x, cache.attend(i, qkv[:, :Hq], positions, self.scale), w, cfg.rms_norm_eps)
-        qkv = F.linear(rms_norm(x, w.input_norm, cfg.rms_norm_eps), w.qkv_w, w.qkv_b)
-        qk = rotate(qkv[:, :cfg.q_size + cfg.kv_size].view(T, Hq + Hkv, d), *rot)
-        q, k = qk[:, :Hq], qk[:, Hq:]
-        v = qkv[:, cfg.q_size + cfg.kv_size:].view(T, Hkv, d)
-        cache.write(i, k, v)
-        x = x + F.linear(cache.attend(i, q, positions, self.scale), w.o_w)
+            attn = cache.attend(i, qkv[:, :Hq], positions, self.scale)
+            if hip_layer.attention_ok(attn, x, w):
+                return hip_layer.layer_out(x, attn, w, cfg.rms_norm_eps)
+        else:
+            qkv = F.linear(rms_norm(x, w.input_norm, cfg.rms_norm_eps), w.qkv_w, w.qkv_b)
+            qk = rotate(qkv[:, :cfg.q_size + cfg.kv_size].view(T, Hq + Hkv, d), *rot)
+            q, k = qk[:, :Hq], qk[:, Hq:]
+            v = qkv[:, cfg.q_size + cfg.kv_size:].view(T, Hkv, d)
+            cache.write(i, k, v)
+            attn = cache.attend(i, q, positions, self.scale)
+        x = x + F.linear(attn, w.o_w)
         gate, up = F.linear(rms_norm(x, w.post_norm, cfg.rms_norm_eps), w.gate_up_w).chunk(2, dim=-1)
         return x + F.linear(F.silu(gate) * up, w.down_w)
 

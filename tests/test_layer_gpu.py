@@ -229,3 +229,41 @@ def test_caches_that_write_their_own_way_are_asked_to():
         assert cache.store_target(0, x.cpu(), 2, 64) is None
         cache.write = lambda layer, k, v: None
         assert cache.store_target(0, x, 2, 64) is None
+
+
+@pytest.mark.parametrize("T", [1, 3, 40])
+def test_attention_results_of_other_forms(T):
+    """What a cache's attend returns is read by the kernels only in the form that they take: other strides and offsets
+    give the layer's result all the same, other types and sizes raise as the torch operations do."""
+    cfg = ModelConfig(vocab_size=64, hidden_size=128, intermediate_size=64, num_layers=1, num_q_heads=4, num_kv_heads=2,
+                      head_dim=32)
+    model = Qwen2Model(cfg, "cuda", torch.bfloat16, seed=1, max_positions=64, std=0.05)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x, pos, attn = randn(g, T, 128), torch.arange(T, device="cuda"), randn(g, T, 128)
+    rot = model.rotary.rows(pos, torch.bfloat16)
+
+    class Given:
+        def write(self, layer, k, v):
+            pass
+
+        def attend(self, layer, q, positions, scale):
+            return self.out
+
+    cache = Given()
+
+    def layer(out):
+        cache.out = out
+        with torch.inference_mode():
+            return model.layer_forward(0, x, pos, cache, rot)
+
+    ref = layer(attn)
+    wide = torch.zeros(T, 256, device="cuda", dtype=torch.bfloat16)
+    odd = torch.zeros(T * 128 + 1, device="cuda", dtype=torch.bfloat16)
+    for view in (wide[:, 64:192], wide[:, ::2], wide[:, 3:131], odd[1:].view(T, 128),
+                 torch.zeros(128, T, device="cuda", dtype=torch.bfloat16).t()):
+        view.copy_(attn)
+        assert rel(layer(view), ref.double()) < 2.0 ** -6  # torch operations against kernels, as above
+    bad_rows = [attn.repeat(2, 1)] if T > 1 else []  # one row of x broadcasts over them
+    for bad in [attn.float(), attn[:, :64].contiguous(), torch.cat([attn, attn], 1), attn.cpu()] + bad_rows:
+        with pytest.raises(RuntimeError):
+            layer(bad)

@@ -38,8 +38,9 @@ def _ok(t, device: int, *shape: int) -> bool:
 
 def rows_ok(x: torch.Tensor, norm_weight: torch.Tensor) -> bool:
     """Whether rms_norm can run on rows x [T, K]. Only under torch.inference_mode: the kernels record nothing for
-    autograd, and forward-mode derivatives and saved-tensor hooks do not reach them there."""
-    if not (torch.is_inference_mode_enabled() and x.is_cuda and x.dim() == 2):
+    autograd, and forward-mode derivatives and saved-tensor hooks do not reach them there. Not under autocast, whose type
+    the products' results have."""
+    if not (torch.is_inference_mode_enabled() and x.is_cuda and x.dim() == 2) or torch.is_autocast_enabled():
         return False
     T, K = x.shape
     dev = x.get_device()

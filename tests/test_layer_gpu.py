@@ -267,3 +267,16 @@ def test_attention_results_of_other_forms(T):
     for bad in [attn.float(), attn[:, :64].contiguous(), torch.cat([attn, attn], 1), attn.cpu()] + bad_rows:
         with pytest.raises(RuntimeError):
             layer(bad)
+
+
+def test_autocast_keeps_the_torch_operations():
+    cfg = ModelConfig(vocab_size=64, hidden_size=128, intermediate_size=64, num_layers=1, num_q_heads=4, num_kv_heads=2,
+                      head_dim=32)
+    model = Qwen2Model(cfg, "cuda", torch.bfloat16, seed=1, max_positions=64, std=0.05)
+    x = torch.zeros(4, 128, device="cuda", dtype=torch.bfloat16)
+    rot = model.rotary.rows(torch.arange(4, device="cuda"), torch.bfloat16)
+    with torch.inference_mode():
+        assert hip_layer.supported(x, model.layers[0], rot, 8, 32)
+        with torch.autocast("cuda", torch.float16):
+            assert not hip_layer.supported(x, model.layers[0], rot, 8, 32)
+            assert not hip_layer.rows_ok(x, model.final_norm)

@@ -423,13 +423,27 @@ struct LinearPlan {
   int64_t counters;
 };
 
+// Tiles 64 x 64, 64 x 128 and 128 x 128 of a gated projection by the workgroups each makes: its time at K = 896 is close
+// to 6 + 4.1 c, 4 + 8 c and (17.5, 25, 13 c from three on) us, c the most workgroups a CU gets (in proportion at 1536),
+// measured at 33 to 1000 tokens on both model shapes. Against the smallest tile of at most 200 workgroups, which this
+// replaces: 0.5B 160 tokens 18.7 -> 13.1 us (228 workgroups of 64 x 128, not 152 of 128 x 128), 800 39.2 -> 35.6, 1.5B
+// 160 39.2 -> 32.3.
+static int gated_tile(int64_t g2, int64_t g3, int64_t g4) {
+  const auto per_cu = [](int64_t g) { return (double)((g + 255) / 256); };
+  const double t2 = 6 + 4.1 * per_cu(g2), t3 = 4 + 8 * per_cu(g3);
+  const double t4 = g4 <= 256 ? 17.5 : g4 <= 512 ? 25 : 13 * per_cu(g4);
+  return t4 <= t2 && t4 <= t3 ? 4 : t3 <= t2 ? 3 : 2;
+}
+
 // The smallest tile whose grid stays within a number of workgroups that depends on the epilogue: small tiles fill the
-// chip, large ones read less. Measured at 8 to 1024 tokens on both model shapes; the rule is within 8% of the best tile
-// in all but two of 56 cases (1.5B gate/up at 64 tokens 20.6 us here, 24.4 one tile smaller; QKV 0.5B at 544 tokens 9.6
-// with 612 small workgroups, 10.9 with 162). ROPE: 640 (K is short and the tiles' norm is their cost). SILU: 200 (every
-// workgroup reads its own 57 to 230 KB of W; from 32 x 64 on). RESIDUAL: 256, and a K from 4096 on is then split until
-// the grid has about 256 again, at most six ways (the merge: 896 x 4864 at 8 tokens 7.5 us with six, 8.0 with eight,
-// 11.5 with one). num_splits and shape of the caller come first (0: the rule).
+// chip, large ones read less. ROPE: 640 (K is short and the tiles' norm is their cost; QKV 0.5B at 544 tokens 9.6 with
+// 612 small workgroups, 10.9 with 162). SILU: 200 workgroups of 32 x 64, gated_tile above them. RESIDUAL: 256, and a K
+// from 4096 on is then split, at most six ways (896 x 4864 at 8 tokens 7.5 us with six, 8.0 with eight, 11.5 with one):
+// tiles of 32 x 32 until the grid has about 256 again, larger ones only as far as one workgroup a CU goes (896 x 4864 at
+// 300 tokens, 140 tiles, 14.7 us whole and 17.4 in halves; 800 tokens, 182 tiles, 21.7 and 25.7; 160 tokens, 140 tiles
+// of 32 x 32, 12.7 and 11.9). From 128 slices of K on, a grid too large to split takes the next larger tile in halves
+// (1536 x 8960: 160 tokens 23.2 -> 20.1 us, 300 29.2 -> 24.8; 896 x 4864 at 544 16.0 -> 17.7, not there).
+// num_splits and shape of the caller come first (0: the rule).
 static LinearPlan plan_linear(int epi, bool norm, int T, int tiles, int K, int want_splits, int want_shape) {
   LinearPlan p{};
   const int units = K >> 6;
@@ -443,15 +457,24 @@ static LinearPlan plan_linear(int epi, bool norm, int T, int tiles, int K, int w
   } else {
     const int most = epi == kEpiRope ? 640 : epi == kEpiSilu ? 200 : 256;
     p.shape = epi == kEpiSilu ? 1 : 0;
-    while (p.shape + 1 < kNumTiles && grid(p.shape) > most) ++p.shape;
+    if (epi != kEpiSilu)
+      while (p.shape + 1 < kNumTiles && grid(p.shape) > most) ++p.shape;
+    else if (grid(1) > most)
+      p.shape = gated_tile(grid(2), grid(3), grid(4));
+    // a long K in whole workgroups of one tile against two halves of the next larger one
+    if (epi == kEpiResidual && !norm && want_splits <= 0 && units >= 128 && p.shape < 2 &&
+        (p.shape == 0 ? grid(0) * 5 > 4 * 256 : 2 * grid(1) > 256) && 2 * grid(p.shape + 1) <= 256)
+      ++p.shape;
   }
   p.splits = 1;
   if (p.shape != kSkinny && epi == kEpiResidual && !norm) {
     const int64_t g = grid(p.shape);
     if (want_splits > 0)
       p.splits = want_splits;
-    else if (K >= 4096 && g * 5 <= 4 * 256)
+    else if (K >= 4096 && p.shape == 0 && g * 5 <= 4 * 256)
       p.splits = (int)std::min<int64_t>(6, (256 + g - 1) / g);
+    else if (K >= 4096 && p.shape > 0)
+      p.splits = (int)std::min<int64_t>(6, std::max<int64_t>(1, 256 / g));
     const int per = (units + p.splits - 1) / p.splits;
     p.splits = (units + per - 1) / per;
     if (p.splits > 1) {

@@ -467,7 +467,8 @@ int32_t sipa_kchan_write_rows(const sipa_kchan_write_params* p, void* stream);
  * strides of a multiple of 4. out must not overlap the inputs, except that it may be the residual itself.
  * A long K of the residual epilogue without norm may be shared by several workgroups (num_splits, 0: the library's
  * choice); the call then needs sipa_linear_scratch_bytes(p) bytes of scratch (any contents) and zero counters, int32,
- * one per tile: the counter region of a decode workspace serves (they are left at zero).
+ * one per tile, which it leaves at zero. Calls that may run at the same time (other streams, graphs replayed side by side)
+ * need counters of their own. clear, clear_count: int32 counters of a later call on the stream that this call sets to zero.
  */
 enum { SIPA_LINEAR_RESIDUAL = 0, SIPA_LINEAR_ROPE = 1, SIPA_LINEAR_SILU = 2 };
 
@@ -502,6 +503,8 @@ typedef struct sipa_linear_params {
   int64_t kv_stride_h, kv_stride_n, kv_stride_b;
   const int64_t* kv_blocks;
   const int64_t* kv_offsets;
+  void* clear; /* NULL, or int32 [clear_count] */
+  int32_t clear_count;
 } sipa_linear_params;
 
 int32_t sipa_fused_linear(const sipa_linear_params* p, void* stream);
@@ -513,8 +516,11 @@ int64_t sipa_linear_scratch_bytes(const sipa_linear_params* p);
 /*
  * A decoder layer after its attention, three launches: h = x + attn o_w^T; out = h + swiglu(rms_norm(h) gate_up_w^T)
  * down_w^T. x, attn with row strides, out [T, hidden] contiguous; matrices [out, in] contiguous; sizes and alignment as
- * for sipa_fused_linear. scratch: sipa_layer_out_scratch_bytes(p) bytes (any contents); counters as above.
+ * for sipa_fused_linear. scratch: sipa_layer_out_scratch_bytes(p) bytes; counters: int32 [SIPA_LAYER_COUNTERS]; both of
+ * any contents and the call's own, like every buffer that it writes.
  */
+enum { SIPA_LAYER_COUNTERS = 512 };
+
 typedef struct sipa_layer_out_params {
   int32_t struct_size; /* sizeof(sipa_layer_out_params) */
   int32_t num_tokens, hidden, attn_features, inter;

@@ -49,7 +49,21 @@ struct LinearArgs {
   int32_t splits;          // workgroups that share a tile's K (RESIDUAL)
   float* part;             // [tile][splits][tokens x rows of a tile] partial sums
   int32_t* counters;       // [tile] workgroups done, zero between calls
+  int32_t* clear;          // counters of a later launch, zeroed by this one's first workgroup
+  int32_t clear_n;
 };
+
+// A split launch needs its counters at zero. The projection launched before it on the stream clears them (clear), so that
+// they can lie in memory of the call's own: no launch is added, and calls share nothing.
+__device__ __forceinline__ void clear_counters(const LinearArgs& a) {
+  if (blockIdx.x + blockIdx.y + blockIdx.z != 0) return;
+  for (int i = threadIdx.x; i < a.clear_n; i += blockDim.x)
+    __hip_atomic_store(a.clear + i, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ void __launch_bounds__(256) clear_kernel(int32_t* p, int n) {
+  if ((int)threadIdx.x < n) p[threadIdx.x] = 0;
+}
 
 template <int EPI>
 __device__ __forceinline__ int linear_row(const LinearArgs& a, int tile, int r) {
@@ -117,6 +131,7 @@ __global__ void __launch_bounds__(64 * kSkinnyWaves) skinny_linear(const LinearA
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, r = lane & 15, q4 = lane >> 4;
   const int tile = blockIdx.x;
+  clear_counters(a);
   const int units = a.K >> 6;
   const uint16_t* const wrow = a.w + (int64_t)linear_row<EPI>(a, tile, r) * a.K + 16 * q4;
   const uint16_t* const xrow = a.x + (int64_t)min(r, a.T - 1) * a.x_st + 16 * q4;
@@ -227,6 +242,7 @@ __global__ void __launch_bounds__(256) tile_linear(const LinearArgs a) {
   const int tile0 = blockIdx.x * (2 * TN), t_base = blockIdx.y * BT;
   const int unit0 = blockIdx.z * a.units;
   const int n = min(a.units, (a.K >> 6) - unit0);
+  clear_counters(a);
 
   // this thread's chunk of rows (tid / 8) + 32 i
   const int row0 = threadIdx.x >> 3, ch = threadIdx.x & 7;
@@ -642,6 +658,8 @@ static int check_linear(const sipa_linear_params* p) {
              p->head_dim, p->rot_channels, N);
   SIPA_CHECK(p->num_splits <= 1 || (p->epilogue == SIPA_LINEAR_RESIDUAL && p->norm_weight == nullptr), SIPA_EINVAL,
              "linear: only the residual epilogue without norm splits K");
+  SIPA_CHECK(p->clear_count >= 0 && p->clear_count <= kMaxCounters && (p->clear_count == 0 || p->clear), SIPA_EINVAL,
+             "linear: %d counters to clear", p->clear_count);
   return SIPA_OK;
 }
 
@@ -696,6 +714,7 @@ extern "C" int32_t sipa_fused_linear(const sipa_linear_params* p, void* stream) 
   a.T = p->num_tokens, a.K = p->in_features, a.D = p->head_dim;
   a.tiles = p->out_features / 16, a.inter = p->out_features / 2;
   a.rot = p->epilogue == SIPA_LINEAR_ROPE ? p->rot_channels : 0;
+  a.clear = (int32_t*)p->clear, a.clear_n = p->clear_count;
   a.splits = plan.splits;
   const int units = a.K >> 6;
   a.units = (units + a.splits - 1) / a.splits;
@@ -739,7 +758,6 @@ static int layer_out_parts(const sipa_layer_out_params* p, sipa_linear_params (&
     q.num_tokens = p->num_tokens;
     q.scratch = base == nullptr ? nullptr : act + act_bytes;
     q.scratch_bytes = p->scratch_bytes - h_bytes - act_bytes;
-    q.counters = p->counters;
   }
   l[0].epilogue = SIPA_LINEAR_RESIDUAL, l[0].in_features = p->attn_features, l[0].out_features = p->hidden;
   l[0].x = p->attn, l[0].x_stride = p->attn_stride, l[0].weight = p->o_w, l[0].residual = p->x;
@@ -777,6 +795,17 @@ extern "C" int32_t sipa_layer_out(const sipa_layer_out_params* p, void* stream) 
              SIPA_EINVAL, "layer: null pointer");
   SIPA_CHECK(p->scratch != nullptr && p->scratch_bytes >= bytes && ((uintptr_t)p->scratch & 255) == 0, SIPA_EWORKSPACE,
              "layer: %lld bytes of 256-byte aligned scratch needed", (long long)bytes);
+  const int n0 = (int)plan_of(&l[0]).counters, n2 = (int)plan_of(&l[2]).counters;
+  SIPA_CHECK(n0 <= SIPA_LAYER_COUNTERS / 2 && n2 <= SIPA_LAYER_COUNTERS / 2, SIPA_EUNSUPPORTED,
+             "layer: %d and %d split tiles exceed the %d counters", n0, n2, SIPA_LAYER_COUNTERS);
+  int32_t* const counters = (int32_t*)p->counters;
+  l[0].counters = counters, l[2].counters = counters + SIPA_LAYER_COUNTERS / 2;
+  if (n0 > 0) {  // from 4096 attention features on: no projection of this call runs before it
+    clear_kernel<<<1, 256, 0, (hipStream_t)stream>>>(counters, n0);
+    const int r = launched("layer counters");
+    if (r != SIPA_OK) return r;
+  }
+  l[0].clear = l[2].counters, l[0].clear_count = n2;
   for (const auto& q : l) {
     const int r = sipa_fused_linear(&q, stream);
     if (r != SIPA_OK) return r;

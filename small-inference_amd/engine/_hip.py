@@ -91,8 +91,11 @@ class LinearParams(ctypes.Structure):
         ("residual", vp), ("res_stride", i64), ("out", vp), ("out_stride", i64), ("rot_cos", vp), ("rot_sin", vp),
         ("num_splits", i32), ("tile", i32), ("scratch", vp), ("scratch_bytes", i64), ("counters", vp),
         ("kv_heads", i32), ("k_pool", vp), ("v_pool", vp), ("kv_stride_h", i64), ("kv_stride_n", i64),
-        ("kv_stride_b", i64), ("kv_blocks", vp), ("kv_offsets", vp),
+        ("kv_stride_b", i64), ("kv_blocks", vp), ("kv_offsets", vp), ("clear", vp), ("clear_count", i32),
     ]
+
+
+LAYER_COUNTERS = 512  # SIPA_LAYER_COUNTERS
 
 
 class LayerOutParams(ctypes.Structure):

@@ -15,7 +15,6 @@ import torch
 import torch.nn.functional as F
 
 from . import _hip
-from .hip_decode import reserve_workspace
 
 RESIDUAL, ROPE, SILU = 0, 1, 2  # SIPA_LINEAR_*
 
@@ -85,25 +84,31 @@ def _linear_scratch(epilogue: int, norm: bool, T: int, K: int, N: int, head_dim:
 def fused_linear(x: torch.Tensor, weight: torch.Tensor, epilogue: int, *, norm_weight: torch.Tensor | None = None,
                  eps: float = 0.0, bias: torch.Tensor | None = None, residual: torch.Tensor | None = None,
                  rot: tuple[torch.Tensor, torch.Tensor] | None = None, head_dim: int = 0, rot_channels: int = 0,
-                 num_splits: int = 0, tile: int = 0, store: tuple | None = None) -> torch.Tensor:
+                 num_splits: int = 0, tile: int = 0, store: tuple | None = None,
+                 counters: torch.Tensor | None = None, clear: torch.Tensor | None = None) -> torch.Tensor:
     """epilogue(norm(x) W^T) in one launch (sipa_fused_linear): x [T, K], weight [N, K]; RESIDUAL adds bias and
     residual, ROPE adds bias and rotates the first rot_channels channels by rot = (cos, signed sin), SILU multiplies
     the second half of the channels by silu of the first. num_splits, tile: 0 for the library's choice. store (ROPE):
-    PagedKVCache.store_target's tuple; the K and V channels then go to the pools and are undefined in the result."""
+    PagedKVCache.store_target's tuple; the K and V channels then go to the pools and are undefined in the result. A K that
+    several workgroups share needs merge counters at zero: `counters`, int32, which an earlier launch was given as `clear`,
+    or new ones from a launch of their own (None)."""
     T, K = x.shape
     N = weight.shape[0]
     out = torch.empty(T, N // 2 if epilogue == SILU else N, device=x.device, dtype=torch.bfloat16)
     stream = _hip.stream_of(x)
     n = _linear_scratch(epilogue, norm_weight is not None, T, K, N, head_dim, num_splits, tile)
-    scratch = counters = None
+    scratch = None
     if n:
         scratch = torch.empty(n, device=x.device, dtype=torch.uint8)
-        counters = reserve_workspace(x.device, stream, 0).data_ptr()
+        if counters is None:  # one a tile, and a tile has 32 x 32 fp32 sums or more
+            counters = torch.zeros(n // 4096, device=x.device, dtype=torch.int32)
     p = _hip.LinearParams(ctypes.sizeof(_hip.LinearParams), epilogue, T, K, N, head_dim, rot_channels, eps,
                           x.data_ptr(), x.stride(0), weight.data_ptr(), _hip.ptr(norm_weight), _hip.ptr(bias),
                           _hip.ptr(residual), residual.stride(0) if residual is not None else 0, out.data_ptr(),
                           out.stride(0), *((rot[0].data_ptr(), rot[1].data_ptr()) if rot is not None else (None, None)),
-                          num_splits, tile, _hip.ptr(scratch), n, counters, *(store or ()))
+                          num_splits, tile, _hip.ptr(scratch), n, _hip.ptr(counters),
+                          *(store or (0, None, None, 0, 0, 0, None, None)), _hip.ptr(clear),
+                          clear.numel() if clear is not None else 0)
     _hip.check(_hip.lib().sipa_fused_linear(ctypes.byref(p), stream), "fused_linear")
     return out
 
@@ -165,16 +170,18 @@ def layer_out(x: torch.Tensor, attn: torch.Tensor, w, eps: float) -> torch.Tenso
         n, h = rms_norm(x, w.post_norm, eps, add=F.linear(attn, w.o_w))
         return h + F.linear(silu_mul(F.linear(n, w.gate_up_w)), w.down_w)
     if 4.0 * T * hidden * inter > MAX_GATED_FLOPS:
-        h = fused_linear(attn, w.o_w, RESIDUAL, residual=x)
+        counters = torch.empty(_hip.LAYER_COUNTERS, device=x.device, dtype=torch.int32)
+        h = fused_linear(attn, w.o_w, RESIDUAL, residual=x, clear=counters)
         act = silu_mul(F.linear(rms_norm(h, w.post_norm, eps), w.gate_up_w))
-        return fused_linear(act, w.down_w, RESIDUAL, residual=h)
+        return fused_linear(act, w.down_w, RESIDUAL, residual=h, counters=counters)
     out = torch.empty(T, hidden, device=x.device, dtype=torch.bfloat16)
-    stream = _hip.stream_of(x)
     nbytes = _layer_out_scratch(T, hidden, attn.shape[1], inter)
-    scratch = torch.empty(nbytes, device=x.device, dtype=torch.uint8)
+    # the sums and then the merge counters of split projections, in memory of this call's own: what a graph holds of them
+    # is its own too
+    scratch = torch.empty(nbytes + 4 * _hip.LAYER_COUNTERS, device=x.device, dtype=torch.uint8)
     p = _hip.LayerOutParams(ctypes.sizeof(_hip.LayerOutParams), T, hidden, attn.shape[1], inter, eps, x.data_ptr(),
                             x.stride(0), attn.data_ptr(), attn.stride(0), w.o_w.data_ptr(), w.post_norm.data_ptr(),
                             w.gate_up_w.data_ptr(), w.down_w.data_ptr(), out.data_ptr(), scratch.data_ptr(), nbytes,
-                            reserve_workspace(x.device, stream, 0).data_ptr())
-    _hip.check(_hip.lib().sipa_layer_out(ctypes.byref(p), stream), "layer_out")
+                            scratch.data_ptr() + nbytes)
+    _hip.check(_hip.lib().sipa_layer_out(ctypes.byref(p), _hip.stream_of(x)), "layer_out")
     return out

@@ -603,3 +603,42 @@ def test_plan_staging_equals_the_per_token_plan():
         assert book.slot_of == ref_slot_of and book.free == ref_free, step
         checked += len(meta.slots_cpu)
     assert checked > 3000 and next_id > 20
+
+
+@pytest.mark.parametrize("T,hidden,attn,inter", [(8, 896, 896, 4864), (128, 896, 896, 4864), (4, 64, 4096, 4096)])
+def test_layer_merge_counters_lie_in_the_calls_own_memory(monkeypatch, T, hidden, attn, inter):
+    """The counters of a layer's split projections are part of a buffer that the call allocates (which a captured graph then
+    owns), not of the stream's split workspace, which a later call may replace."""
+    import ctypes
+
+    from engine import _hip, hip_decode, hip_layer
+    from engine.model import Layer
+
+    real, seen, made = _hip.lib(), [], []
+
+    class Lib:
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+        def sipa_layer_out(self, p, stream):
+            seen.append(ctypes.cast(p, ctypes.POINTER(_hip.LayerOutParams)).contents)
+            return 0
+
+    empty = torch.empty
+
+    def recording(*size, **kw):
+        made.append(empty(*size, **kw))
+        return made[-1]
+
+    monkeypatch.setattr(_hip, "lib", lambda: Lib())
+    monkeypatch.setattr(_hip, "stream_of", lambda t: 0)
+    monkeypatch.setattr(torch, "empty", recording)
+    held = dict(hip_decode._workspaces)
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)  # noqa: E731
+    w = Layer(z(hidden), z(hidden, hidden), z(hidden), z(hidden, attn), z(hidden), z(2 * inter, hidden), z(hidden, inter))
+    hip_layer.layer_out(z(T, hidden), z(T, attn), w, 1e-6)
+    p, size = seen[0], 4 * _hip.LAYER_COUNTERS
+    assert any(t.data_ptr() <= p.counters and p.counters + size <= t.data_ptr() + t.numel() * t.element_size()
+               for t in made)
+    assert p.scratch + p.scratch_bytes <= p.counters or p.counters + size <= p.scratch
+    assert hip_decode._workspaces == held

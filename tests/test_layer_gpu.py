@@ -14,7 +14,7 @@ import torch.nn.functional as F
 from cases import fragmented_manager
 from engine import hip_layer
 from engine.config import ModelConfig
-from engine.model import Qwen2Model, rms_norm, rotate
+from engine.model import Layer, Qwen2Model, rms_norm, rotate
 from engine.paged_cache import PagedKVCache, build_metadata
 
 pytestmark = pytest.mark.gpu
@@ -280,3 +280,72 @@ def test_autocast_keeps_the_torch_operations():
         with torch.autocast("cuda", torch.float16):
             assert not hip_layer.supported(x, model.layers[0], rot, 8, 32)
             assert not hip_layer.rows_ok(x, model.final_norm)
+
+
+def layer_weights(g, hidden, attn, inter):
+    return Layer(None, None, None, randn(g, hidden, attn) * 0.05, 1 + 0.1 * randn(g, hidden), randn(g, 2 * inter, hidden) * 0.05,
+                 randn(g, hidden, inter) * 0.05)
+
+
+def layer_out64(x, attn, w):
+    h = x.double() + attn.double() @ w.o_w.double().t()
+    gate, up = (norm64(h, w.post_norm) @ w.gate_up_w.double().t()).chunk(2, -1)
+    return h + (F.silu(gate) * up) @ w.down_w.double().t()
+
+
+@pytest.mark.parametrize("T,hidden,attn,inter", [(8, 896, 896, 4864), (128, 896, 896, 4864), (512, 1536, 1536, 8960),
+                                                 (20, 128, 4096, 4096)])
+def test_captured_layers_own_their_merge_counters(T, hidden, attn, inter):
+    """Layers whose projections share K among workgroups, captured twice on a stream without a workspace: the second
+    graph is replayed before the first, the stream's workspace is made, replaced and overwritten in between, and the two
+    are replayed side by side on two streams. Every replay gives the eager result."""
+    from engine.hip_decode import reserve_workspace
+
+    g = torch.Generator(device="cuda").manual_seed(T)
+    w = layer_weights(g, hidden, attn, inter)
+    inputs = [(randn(g, T, hidden), randn(g, T, attn)) for _ in range(2)]
+    print(f"case captured layer T {T} {hidden} {attn} {inter}", flush=True)
+    s, other = torch.cuda.Stream(), torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        eager = [hip_layer.layer_out(x, a, w, EPS) for x, a in inputs]
+    torch.cuda.synchronize()
+    for (x, a), out in zip(inputs, eager):
+        # h, the activations and the sum are rounded to bf16, each 2^-9 at worst, beside the gated product's bound
+        assert rel(out, layer_out64(x, a, w)) < 2 * BOUND
+    torch.cuda.synchronize()
+    graphs = []
+    for x, a in inputs:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            outs = [hip_layer.layer_out(x, a, w, EPS) for _ in range(3)]
+        graphs.append((graph, outs))
+    torch.cuda.synchronize()
+
+    def check(i):
+        torch.cuda.synchronize()
+        for out in graphs[i][1]:
+            assert torch.equal(out, eager[i])
+            out.fill_(7)
+        torch.cuda.synchronize()
+
+    for i in (1, 0, 1):
+        graphs[i][0].replay()
+        check(i)
+    for nbytes in (1 << 20, 8 << 20, 24 << 20):
+        ws = reserve_workspace(torch.device("cuda"), s.cuda_stream, nbytes)
+        torch.cuda.synchronize()
+        junk = [torch.full((1 << 18,), 0x5a5a5a5a, device="cuda", dtype=torch.int32) for _ in range(8)]
+        graphs[0][0].replay()
+        check(0)
+        assert not ws.any()
+        del junk
+    if 4.0 * T * hidden * inter > hip_layer.MAX_GATED_FLOPS:
+        return  # a library product among them: torch gives the stream's graphs one library workspace
+    for _ in range(5):
+        with torch.cuda.stream(s):
+            graphs[0][0].replay()
+        with torch.cuda.stream(other):
+            graphs[1][0].replay()
+        check(0)
+        check(1)

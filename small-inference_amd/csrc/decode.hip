@@ -54,8 +54,9 @@ namespace sipa {
 constexpr int kHotArgBytes = 3 * 8 + 6 * 4;
 
 // NB: tiles in flight per wave (the register prefetch ring); PHL: P as a bf16 hi + lo pair (else one bf16 term).
-// BS: blocks of 16 << BS tokens, addressed as 16-token blocks (fetch_split_ids_flat). 24 x 3000 tokens of 32-token
-// blocks at head_dim 128: 94.4 us on the VALU kernel, which served every block size but 16; 17.3 here.
+// BS: blocks of 16 << BS tokens, addressed as 16-token blocks (fetch_split_ids_flat), with P in all its 24 bits as three
+// bf16 terms, as the VALU kernel held it, which served every block size but 16. 24 x 3000 tokens of 32-token blocks at
+// head_dim 128: 95.3 us there, 17.4 here (17.3 with the pair).
 template <int D, int NB, bool PHL, int BS>
 __global__ void __launch_bounds__(kThreads) decode_mfma_bf16(const int32_t* __restrict__ hbt,
                                                              const int32_t* __restrict__ hctx,
@@ -211,13 +212,27 @@ __global__ void __launch_bounds__(kThreads) decode_mfma_bf16(const int32_t* __re
       m_run = m_new;
     }
     bf16x8 pop, plo;
+    u32x4 p3[3];  // BS: the three terms of P
     float psum = 0.f;
+    if constexpr (BS > 0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float p = fast_exp2(fmaf(sc[i >> 2][i & 3], a.scale_log2, -m_run));
-      psum += p;
-      pop[i] = (__bf16)p;
-      if (PHL) plo[i] = (__bf16)(p - (float)pop[i]);  // the rounding residual, exact in fp32
+      for (int i = 0; i < 8; i += 2) {
+        const float pa = fast_exp2(fmaf(sc[i >> 2][i & 3], a.scale_log2, -m_run));
+        const float pb = fast_exp2(fmaf(sc[i >> 2][(i & 3) + 1], a.scale_log2, -m_run));
+        psum += pa;
+        psum += pb;
+        uint32_t t0, t1, t2;
+        split_bf16x3(pa, pb, t0, t1, t2);
+        p3[0][i >> 1] = t0, p3[1][i >> 1] = t1, p3[2][i >> 1] = t2;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float p = fast_exp2(fmaf(sc[i >> 2][i & 3], a.scale_log2, -m_run));
+        psum += p;
+        pop[i] = (__bf16)p;
+        if (PHL) plo[i] = (__bf16)(p - (float)pop[i]);  // the rounding residual, exact in fp32
+      }
     }
     l_run += psum;
 
@@ -225,6 +240,12 @@ __global__ void __launch_bounds__(kThreads) decode_mfma_bf16(const int32_t* __re
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       const bf16x8 vop = read_v_operand<bf16x8>(vw, tr_off, VP, 16 * dt);
+      if constexpr (BS > 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, __builtin_bit_cast(bf16x8, p3[k]), acc[dt], 0, 0, 0);
+        continue;
+      }
       acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop, acc[dt], 0, 0, 0);
       if (PHL) acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, plo, acc[dt], 0, 0, 0);
     }

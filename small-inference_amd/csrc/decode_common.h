@@ -384,6 +384,26 @@ __device__ __forceinline__ T8 read_v_operand(const uint16_t* tile, int tr_off, i
   return __builtin_bit_cast(T8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
+// Two values as three bf16 terms each, packed in pairs: hi + mid + lo is the fp32 value exactly (8 significant bits a
+// term), and no term of a value above 2^-95 is zero or has the other sign, so that an infinite factor gives the sum's
+// infinity and not inf * 0: a term is cut from the fp32 number just below what remains. Used where P is multiplied with
+// blocks of more than 16 tokens: the pair (hi, lo) of the 16-token kernels has 16 bits, and a lo of 0 against an infinite V
+// gives NaN.
+__device__ __forceinline__ void split_bf16x3(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  const auto below = [](float x) {  // inf: the largest finite bf16, inf remains
+    return __uint_as_float(__builtin_elementwise_sub_sat(__float_as_uint(x), 1u) & 0xffff0000u);
+  };
+  const auto pack = [](float x, float y) {
+    return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u);
+  };
+  const float ah = below(a), bh = below(b);
+  const float ar = a - ah, br = b - bh;
+  const float am = below(ar), bm = below(br);
+  hi = pack(ah, bh);
+  mid = pack(am, bm);
+  lo = pack(ar - am, br - bm);
+}
+
 template <int D>
 struct MfmaSmem {
   static constexpr int kVPitch = D + 8;                                // bf16 elements per LDS row of V

@@ -46,6 +46,16 @@ __device__ __forceinline__ f16x8 codes8_to_f16(uint32_t w0, uint32_t w1) {
   return f16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
+// 8 int8 codes -> 8 bf16 values, exact.
+__device__ __forceinline__ u32x4 codes8_to_bf16(uint32_t w0, uint32_t w1) {
+  const uint32_t w[2] = {w0, w1};
+  u32x4 out;
+#pragma unroll
+  for (int j = 0; j < 8; j += 2)
+    out[j >> 1] = pack_bf16x2((float)(int8_t)(w[j >> 2] >> (8 * (j & 3))), (float)(int8_t)(w[j >> 2] >> (8 * (j & 3) + 8)));
+  return out;
+}
+
 __device__ __forceinline__ float h2f(uint32_t bits16) { return f16_bits_to_f32(bits16 & 0xffffu); }
 
 template <int D>
@@ -73,7 +83,10 @@ constexpr int kWaveScaleBlocks = kScaleBlocks / kWaves;  // blocks of one wave's
 
 // MODE 1: per-token K scales; 2: per-(block, channel) K scales; 3: mode 2 with one channel scale per (head,
 // channel) for every block (a zero block stride), folded into the query once.
-// BS (mode 1): blocks of 16 << BS tokens, addressed as 16-token blocks with 16 token scales each.
+// BS (mode 1): blocks of 16 << BS tokens, addressed as 16-token blocks with 16 token scales each. Operands in bf16 there:
+// codes and the query exactly, P' in all its 24 bits as three terms, of any magnitude (no 2^vshift), as the VALU kernel
+// held them, which served every block size but 16. 64 x 4096 tokens of 32-token blocks at head_dim 128: 187 us
+// there, 30.8 here (28.4 over 16-token blocks, with fp16 operands and P' in 11 bits).
 template <int D, int MODE, int NB, int BS>
 __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs a) {
   constexpr int KS = D / 32;   // QK k-steps per block
@@ -82,6 +95,8 @@ __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs
   constexpr int VC = D / 64;   // 16-byte V chunks (16 codes) per lane per block
   constexpr int VP = MfmaSmem<D>::kVPitch;
   constexpr int CPR = D / 16;  // 16-code chunks per token row
+  constexpr bool kExact = BS > 0;
+  static_assert(!kExact || MODE == 1, "larger blocks: per-token scales only");
 
   __shared__ __align__(16) char smem[MfmaSmem<D>::kBytes];
   // mode 2: each wave's channel scales of two tiles (slot = tile index parity), [wave][slot][block][lane]
@@ -198,6 +213,7 @@ __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs
   float sl2 = a.scale_log2;
   float vshift = 0.f;  // p' = p 2^vshift (set once the wave's V scales are in)
   auto convert_query = [&]() {
+    if (kExact) return;
     float qf[KS][8];
     float qmax = 0.f;
 #pragma unroll
@@ -335,6 +351,12 @@ __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs
         const int row = c / CPR;
         u32x4 wv = tl.v[mt][i];
         if (partial && t0 + 16 * mt + row >= end) wv = u32x4{0, 0, 0, 0};
+        if constexpr (kExact) {
+          u32x4* dst = (u32x4*)(vw + (16 * mt + row) * VP + (c % CPR) * 16);
+          dst[0] = codes8_to_bf16(wv[0], wv[1]);
+          dst[1] = codes8_to_bf16(wv[2], wv[3]);
+          continue;
+        }
         const f16x8 lo = codes8_to_f16(wv[0], wv[1]);
         const f16x8 hi = codes8_to_f16(wv[2], wv[3]);
         _Float16* dst = vw + (16 * mt + row) * VP + (c % CPR) * 16;
@@ -361,6 +383,12 @@ __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs
 #pragma unroll
       for (int j = 0; j < KS; ++j) {
         const u32x4 kw = tl.k[mt][j >> 1];
+        if constexpr (kExact) {
+          const u32x4 kb = codes8_to_bf16(kw[2 * (j & 1)], kw[2 * (j & 1) + 1]);
+          sc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kb),
+                                                           __builtin_bit_cast(bf16x8, qraw[j]), sc[mt], 0, 0, 0);
+          continue;
+        }
         const f16x8 kop = codes8_to_f16(kw[2 * (j & 1)], kw[2 * (j & 1) + 1]);
         if (MODE == 1) {
           sc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop, qh[j], sc[mt], 0, 0, 0);
@@ -410,7 +438,8 @@ __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs
       m_run = m_new;
     }
     f16x8 pop;
-    float psum = 0.f;
+    u32x4 p3[3];  // kExact: the three terms of P'
+    float psum = 0.f, px[8];
     const uint2 vsc[2] = {token_scales(0, t0, 0), token_scales(0, t0, 1)};
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -418,13 +447,34 @@ __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs
       const float p = fast_exp2(fmaf(sc[mt][e], sl2, vshift - m_run));  // p 2^vshift
       psum += p;
       const uint32_t vsw = (e < 2) ? vsc[mt].x : vsc[mt].y;
-      pop[i] = (_Float16)(p * h2f(vsw >> (16 * (e & 1))));
+      px[i] = p * h2f(vsw >> (16 * (e & 1)));
+      pop[i] = (_Float16)px[i];
     }
     l_run += psum;
+    if constexpr (kExact) {
+      if (partial) {  // a token past the end may have any scale
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (t0 + 16 * (i >> 2) + 4 * q4 + (i & 3) >= end) px[i] = 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        uint32_t x0, x1, x2;
+        split_bf16x3(px[i] + 0.f, px[i + 1] + 0.f, x0, x1, x2);  // + 0: a zero of either sign is 0
+        p3[0][i >> 1] = x0, p3[1][i >> 1] = x1, p3[2][i >> 1] = x2;
+      }
+    }
 
     wave_sync();  // the wave's V tile is in LDS
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
+      if constexpr (kExact) {
+        const bf16x8 vb = read_v_operand<bf16x8>((const uint16_t*)vw, tr_off, VP, 16 * dt);
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb, __builtin_bit_cast(bf16x8, p3[k]), acc[dt], 0, 0, 0);
+        continue;
+      }
       const f16x8 vop = read_v_operand<f16x8>((const uint16_t*)vw, tr_off, VP, 16 * dt);
       acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop, pop, acc[dt], 0, 0, 0);
     }
@@ -450,7 +500,7 @@ __global__ void __launch_bounds__(kThreads, 2) decode_mfma_int8(const DecodeArgs
     uint32_t mb = 0;
 #pragma unroll
     for (int i = 0; i < kWaves; ++i) mb = max(mb, vmax_bits[i]);
-    vshift = shift_of(mb);
+    vshift = kExact ? 0.f : shift_of(mb);
   }
   if (piped) {
     // Tile k is in ring[k % NB]; after tile k, tile k + 1's channel scales (mode 2) go to LDS slot (k + 1) & 1.

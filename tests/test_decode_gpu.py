@@ -10,6 +10,8 @@ max-abs 8e-3 against the fp32 oracle (the north-star bound for unit-variance inp
 reference's), and the median relative error under 2^-8 (reference :89-94).
 """
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -381,9 +383,10 @@ def test_scores_trending_across_keys(direction, splits):
 @pytest.mark.parametrize("B", [32, 64])
 @pytest.mark.parametrize("path", ["single", "split3", "auto", "work list", "bad ids"])
 def test_larger_blocks_equal_their_16_token_parts(fmt, heads, B, path):
-    """Blocks of 32 and 64 tokens run the MFMA kernels as 16-token blocks: the same bits as the pool and tables
-    rewritten in 16-token blocks (token for token the same memory), at lengths around the edges of both block sizes;
-    ids outside the pool are clamped to it first."""
+    """Blocks of 32 and 64 tokens run the MFMA kernels as 16-token blocks: the results of the pool and tables rewritten
+    in 16-token blocks (token for token the same memory), at lengths around the edges of both block sizes; ids outside
+    the pool are clamped to it first. The 16-token kernels round each probability to 2^-17 (bf16 pools) or 2^-12 (INT8),
+    the others not at all, and each rounds its output to bf16, whose neighbours are up to 2^-7 of their size apart."""
     Hq, Hkv, D = HEADS[heads]
     lengths = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 96, 300, 1000, 2500]
     q, k, v, bt, ctx, _ = make_case(lengths, Hq, Hkv, D, B, torch.bfloat16, seed=B)
@@ -408,4 +411,109 @@ def test_larger_blocks_equal_their_16_token_parts(fmt, heads, B, path):
     out = paged_decode_attention(q, k, v, bt, ctx, D ** -0.5, max(lengths), quant=quant, **kw)
     ref = paged_decode_attention(q, k16, v16, ids.flatten(1).contiguous(), ctx, D ** -0.5, max(lengths), quant=quant16,
                                  **kw)
-    assert torch.equal(out, ref)
+    out, ref = out.float(), ref.float()
+    largest = 127 * float(vs.max()) if fmt == "int8" else float(v.abs().max())
+    assert ((out - ref).abs() <= 2.0 ** -12 * largest + 2.0 ** -7 * torch.maximum(out.abs(), ref.abs())).all()
+
+
+def cancelling_case(fmt, D, B, seed):
+    """64 sequences of three tokens whose weighted V rows nearly cancel: the first value is drawn, each later one is the
+    nearest that takes what is left to zero. (q, k, v, quant, bt, ctx, out in 64 bits, sum of |weighted V|)"""
+    S, G, n = 64, 4, 3
+    g = torch.Generator().manual_seed(seed)
+    q = torch.zeros(S, 2 * G, D, dtype=torch.bfloat16)
+    q[:, :, 0] = 8
+    bt = torch.arange(S, dtype=torch.int32)[:, None]
+    k = torch.zeros(2, S, B, D)
+    quant = None
+    vs = torch.ones(2, S, n, dtype=torch.float64)
+    if fmt == "int8":
+        k[:, :, :n, 0] = torch.randint(-127, 1, (2, S, n), generator=g).float()
+        ks = torch.full((2, S, B), 2.0 ** -8).half()
+        scales = torch.full((2, S, B), math.nan).half()  # past the context: anything
+        scales[:, :, 0] = (0.5 + 0.5 * torch.rand(2, S, generator=g)).half()
+        scales[:, :, 1], scales[:, :, 2] = 1, 2.0 ** -7
+        quant = QuantKV(1, ks.cuda(), scales.cuda())
+        vs = scales[:, :, :n].double()
+        score = 8 * k[:, :, :n, 0].double() * 2.0 ** -8
+    else:
+        k[:, :, :n, 0] = (-0.5 * torch.rand(2, S, n, generator=g)).bfloat16().float()
+        score = 8 * k[:, :, :n, 0].double()
+    scale = float(np.float32(D ** -0.5))
+    w = torch.softmax(score * scale, -1)[..., None]  # [2, S, n, 1]
+    v = torch.zeros(2, S, B, D, dtype=torch.float64)
+    left = 0.0
+    for t in range(n):
+        unit = w[:, :, t] * vs[:, :, t, None]
+        want = torch.randn(2, S, D, generator=g).double() * (50 if fmt == "int8" else 1) if t == 0 else -left / unit
+        v[:, :, t] = want.round().clamp(-127, 127) if fmt == "int8" else want.bfloat16().double()
+        left = left + unit * v[:, :, t]
+    size = (w * (v[:, :, :n] * vs[..., None]).abs()).sum(2)
+    dt = torch.int8 if fmt == "int8" else torch.bfloat16
+    ctx = torch.full((S,), n, dtype=torch.int32)
+    rows = lambda x: x.transpose(0, 1).repeat_interleave(G, 1)  # noqa: E731  [2, S, D] -> [S, 2 G, D]
+    return (q.cuda(), k.to(dt).cuda(), v.to(dt).cuda(), quant, bt.cuda(), ctx.cuda(), rows(left), rows(size))
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "int8"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B", [32, 64])
+def test_larger_blocks_hold_probabilities_in_fp32(fmt, D, B):
+    """Against 64 bits where the terms cancel, which shows the probabilities' own error: the exponential's ulp, its
+    argument's and the sums' roundings are under 2^-21 of the terms' size in fp32; a bf16 pair has 2^-17, an fp16 2^-12.
+    The output's bf16 rounding is at most 2^-8 of what is left."""
+    q, k, v, quant, bt, ctx, ref, size = cancelling_case(fmt, D, B, seed=B + D)
+    print(f"case cancelling {fmt} D {D} B {B}", flush=True)
+    out = paged_decode_attention(q, k, v, bt, ctx, D ** -0.5, 3, quant=quant).double().cpu()
+    assert ((out - ref).abs() <= 2.0 ** -20 * size + 2.0 ** -8 * ref.abs()).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B", [32, 64])
+def test_larger_blocks_int8_scales_of_any_ratio(D, B):
+    """A token with nearly all the weight and fp16's smallest V scale beside one with its largest scale, no weight and
+    codes of zero."""
+    q = torch.zeros(1, 2, D, device="cuda", dtype=torch.bfloat16)
+    q[..., 0] = 64
+    k, v = (torch.zeros(2, 1, B, D, device="cuda", dtype=torch.int8) for _ in range(2))
+    k[:, :, 1, 0] = -64  # 64 . 64 / sqrt(D) below the other
+    v[:, :, 0] = 100
+    ks, vs = torch.ones(2, 1, B, device="cuda").half(), torch.zeros(2, 1, B, device="cuda").half()
+    vs[:, :, 0], vs[:, :, 1] = 2.0 ** -24, 2.0 ** 15
+    bt, ctx = torch.zeros(1, 1, device="cuda", dtype=torch.int32), torch.full((1,), 2, device="cuda", dtype=torch.int32)
+    out = paged_decode_attention(q, k, v, bt, ctx, D ** -0.5, 2, quant=QuantKV(1, ks, vs))
+    assert (out.float() == torch.tensor(100 * 2.0 ** -24).bfloat16().float().item()).all()
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "int8"])
+@pytest.mark.parametrize("heads", list(HEADS))
+@pytest.mark.parametrize("B", [32, 64])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_larger_blocks_with_infinite_values(fmt, heads, B, splits):
+    """Infinite and NaN V (infinite and NaN V scales of INT8 pools) give what the fp32 kernel gives: infinities of
+    their sign, NaN where both signs or a NaN meet, everything else untouched."""
+    Hq, Hkv, D = HEADS[heads]
+    lengths = [1, 20, 33, 64, 100, 700]
+    q, k, v, bt, ctx, tables = make_case(lengths, Hq, Hkv, D, B, torch.bfloat16, seed=B)
+    quant = None
+    if fmt == "int8":
+        g = torch.Generator(device="cuda").manual_seed(B)
+        k, v = (torch.randint(-127, 128, k.shape, device="cuda", dtype=torch.int8, generator=g) for _ in range(2))
+        ks, vs = ((torch.rand(k.shape[:3], device="cuda", generator=g) / 256 + 1 / 512).half() for _ in range(2))
+        quant = QuantKV(1, ks, vs)
+        for s, t, x in ((1, 19, math.inf), (3, 40, math.inf), (3, 41, math.nan), (5, 650, math.inf)):
+            vs[0, tables[s][t // B], t % B] = x
+        v[0, tables[1][19 // B], 19 % B, 5] = 0  # 0 x inf
+    else:
+        for s, t, ch, x in ((0, 0, 3, math.inf), (1, 7, 0, math.inf), (1, 18, 1, -math.inf), (2, 32, 2, math.inf),
+                            (2, 3, 2, -math.inf), (4, 99, 4, math.nan), (5, 650, 9, math.inf), (5, 17, 10, -math.inf)):
+            v[1, tables[s][t // B], t % B, ch] = x
+    print(f"case infinite {fmt} {heads} B {B} splits {splits}", flush=True)
+    args = (q, k, v, bt, ctx, D ** -0.5, max(lengths))
+    out = paged_decode_attention(*args, num_splits=splits, quant=quant, impl="mfma").float()
+    ref = paged_decode_attention(*args, num_splits=splits, quant=quant, impl="valu").float()
+    assert ref.isinf().any() and ref.isnan().any()
+    assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
+    assert torch.equal(out[ref.isinf()], ref[ref.isinf()])
+    ok = ref.isfinite()
+    assert ((out - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e-6)[ok].all()  # a bf16 step; fp32 sums in another order

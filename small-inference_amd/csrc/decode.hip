@@ -640,8 +640,10 @@ static int launch_bf16(dim3 grid, const DecodeArgs& a, hipStream_t st) {
 
 template <bool PHL>
 static int launch_mfma(int D, int nb, int bs, dim3 grid, const DecodeArgs& a, hipStream_t st) {
-  if (bs == 1) return D == 64 ? launch_bf16<64, 2, PHL, 1>(grid, a, st) : launch_bf16<128, 2, PHL, 1>(grid, a, st);
-  if (bs == 2) return D == 64 ? launch_bf16<64, 2, PHL, 2>(grid, a, st) : launch_bf16<128, 2, PHL, 2>(grid, a, st);
+  if constexpr (PHL) {
+    if (bs == 1) return D == 64 ? launch_bf16<64, 2, PHL, 1>(grid, a, st) : launch_bf16<128, 2, PHL, 1>(grid, a, st);
+    if (bs == 2) return D == 64 ? launch_bf16<64, 2, PHL, 2>(grid, a, st) : launch_bf16<128, 2, PHL, 2>(grid, a, st);
+  }
   if (D == 64) {
     switch (nb) {
       case 1: return launch_bf16<64, 1, PHL>(grid, a, st);
@@ -1066,8 +1068,8 @@ static int decode_impl(const sipa_decode_params* p, void* stream, bool use_scrat
                SIPA_EUNSUPPORTED, "the VALU streaming kernels need a bf16 query, block 16, head_dim 64/128, a group "
                "of 6-8, a bf16 pool or an int8 per-token pool with fp16 scales, and 16-byte aligned rows");
   }
-  SIPA_CHECK(p->impl != SIPA_IMPL_MFMA_PBF16 || (mfma_ok && mode == SIPA_KV_PLAIN), SIPA_EUNSUPPORTED,
-             "the bf16-P MFMA variant needs a bf16 query and pool, block 16, 32 or 64, head_dim 64/128, 16-byte aligned rows");
+  SIPA_CHECK(p->impl != SIPA_IMPL_MFMA_PBF16 || (mfma_ok && mode == SIPA_KV_PLAIN && bs == 0), SIPA_EUNSUPPORTED,
+             "the bf16-P MFMA variant needs a bf16 query and pool, block 16, head_dim 64/128, 16-byte aligned rows");
   SIPA_CHECK(p->impl != SIPA_IMPL_MFMA || mfma_ok, SIPA_EUNSUPPORTED,
              "the MFMA kernels need a bf16 query, block 16 (32 or 64: not per channel), head_dim 64/128, 16-byte aligned rows and fp16 scales "
              "(or fp32 channel scales with a zero block stride)");

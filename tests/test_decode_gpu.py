@@ -517,3 +517,10 @@ def test_larger_blocks_with_infinite_values(fmt, heads, B, splits):
     assert torch.equal(out[ref.isinf()], ref[ref.isinf()])
     ok = ref.isfinite()
     assert ((out - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e-6)[ok].all()  # a bf16 step; fp32 sums in another order
+
+
+@pytest.mark.parametrize("B", [32, 64])
+def test_bf16_probability_variant_keeps_to_16_token_blocks(B):
+    q, k, v, bt, ctx, _ = make_case([40], 14, 2, 64, B, torch.bfloat16)
+    with pytest.raises(ValueError, match="block 16"):
+        paged_decode_attention(q, k, v, bt, ctx, 0.125, 40, impl="mfma_pbf16")

@@ -279,11 +279,11 @@ enum {
 
 int32_t sipa_prefill(const sipa_prefill_params* p, void* stream);
 
-/* Key splits for a prefill call (no counterpart in the reference, whose gather path has no grid): one under 512 keys
- * of context; about two workgroups per CU over the call's 8-column units from 4096 keys (from 2048 where not even two
+/* Key splits for a prefill call (no counterpart in the reference, whose gather path has no grid): one up to
+ * 448 keys of context (511 at head_dim 128); about two workgroups per CU over the call's 8-column units from 4096 keys (from 2048 where not even two
  * splits fit one workgroup per CU); between, at most one workgroup per CU and 8 splits. At least 256 keys per split
- * and at most 32 splits. query_tiles = sum over sequences of ceil(query_len / 16) (head_dim is part of the policy's
- * signature and does not change it today). cu_count <= 0 asks the current device. */
+ * and at most 32 splits. query_tiles = sum over sequences of ceil(query_len / 16). cu_count <= 0 asks the current
+ * device. */
 int32_t sipa_prefill_splits(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t query_tiles,
                             int32_t max_context, int32_t cu_count);
 

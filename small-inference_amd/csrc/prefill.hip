@@ -5,9 +5,10 @@
 // (query at position p sees keys 0 .. p, query head g uses KV head g / G, softmax in fp32, probabilities rounded
 // to the model dtype before P.V). This kernel computes the same rows in place from the pool.
 //
-// Work unit: (sequence s, KV head h, NC column tiles). The column tiles of a (sequence, KV head) are its (16 new tokens,
-// query head) pairs, heads fastest; unit j takes columns NC j .. NC j + NC - 1, so that every unit but a sequence's last
-// one fills its waves whatever the group size (whole 16-token steps of G = 6 or 7 heads left 4 or 2 of 16 waves idle).
+// Work unit: (sequence s, KV head h, `cols` column tiles). The column tiles of a (sequence, KV head) are its (16 new tokens,
+// query head) pairs, heads fastest; unit j takes columns cols j .. cols j + cols - 1. cols = NC fills every wave of every
+// unit but a sequence's last whatever the group size (whole 16-token steps of G = 6 or 7 heads leave 4 or 2 of 16 waves
+// idle); whole steps are taken where the launch puts no more workgroups on a CU with them (see sipa_prefill).
 // The unit's keys are positions [0, P0 + ntok) of the sequence, P0 the position of its first token and ntok the tokens
 // its columns span; they are cut into splits of `chunk` keys, one
 // workgroup each, so that a short chunk over a long context still fills the chip. The four waves of a workgroup
@@ -41,7 +42,10 @@ struct PrefillArgs {
   const int32_t* qlen;    // [S] new tokens per sequence
   void* out;
   int64_t o_st, o_sh;
-  int32_t S, G, qtiles;   // qtiles: units of the longest sequence, ceil(ceil(max new tokens / 16) G / NC)
+  int32_t S, G, qtiles;   // qtiles: units of the longest sequence, ceil(ceil(max new tokens / 16) G / cols)
+  int32_t cols;            // column tiles of a unit, at most NC
+  uint32_t inv_g;          // ceil(2^31 / G): c / G is the high word of 2 c inv_g for c < 2^28 (a division in the kernel's
+                           // prologue is some 20 instructions)
   int32_t npair;           // S * Hkv
   int32_t T, nb, max_ctx;  // rows of q / out, pool blocks, context clamp
   int32_t nsplit, chunk;   // key splits per unit, keys per split (a multiple of 64)
@@ -86,8 +90,8 @@ static inline PfShape prefill_shape(int layout) {
   }
 }
 
-// Units of a (sequence, KV head) with n new tokens.
-static inline int64_t prefill_units(int n, int G, int nc) { return ((n + 15) / 16 * (int64_t)G + nc - 1) / nc; }
+// Units of cols column tiles of a (sequence, KV head) with n new tokens.
+static inline int64_t prefill_units(int n, int G, int cols) { return ((n + 15) / 16 * (int64_t)G + cols - 1) / cols; }
 
 // Whole 16-token steps of G heads that fit NC column tiles: the unit of the split policy and of the workspace size (at
 // least as many units as prefill_units gives).
@@ -203,9 +207,12 @@ __global__ void __launch_bounds__(64 * NC / CW * KH) prefill_mfma_bf16(const Pre
   const int s = pair % a.S, h = pair / a.S;
   const int G = a.G;
   const int n = a.qlen[s];
-  const int c_base = NC * j;                              // the unit's first column
-  const int tok0 = 16 * (c_base / G);                     // its first token,
-  const int span = 16 * ((c_base + NC - 1) / G + 1) - tok0;  // and the tokens its columns span
+  auto step_of = [&](int c) { return (int)__umulhi(2u * (uint32_t)c, a.inv_g); };  // c / G: the column's 16-token step
+  const int c_base = a.cols * j;                                  // the unit's first column
+  const int tok0 = 16 * step_of(c_base);                          // its first token,
+  // and the tokens its columns span. (Columns past a unit of whole steps, cols < NC, belong to tokens past the span and so
+  // have none.)
+  const int span = 16 * (step_of(c_base + a.cols - 1) + 1) - tok0;
   if (tok0 >= n) return;
   const int row0 = a.qstart[s] + tok0;
   const int ctx = min(a.ctx[s], a.max_ctx);
@@ -244,8 +251,9 @@ __global__ void __launch_bounds__(64 * NC / CW * KH) prefill_mfma_bf16(const Pre
 #pragma unroll
   for (int ci = 0; ci < CW; ++ci) {
     const int c = c_base + wcol + CWV * ci;
-    cg[ci] = c % G;
-    ctok[ci] = 16 * (c / G) - tok0;
+    const int step = step_of(c);
+    cg[ci] = c - step * G;
+    ctok[ci] = 16 * step - tok0;
     cvalid[ci] = ctok[ci] < ntok;
     const bool valid = cvalid[ci] && ctok[ci] + r < ntok;
     const uint16_t* qrow = (const uint16_t*)a.q + (int64_t)(row0 + min(ctok[ci] + r, ntok - 1)) * a.q_st +
@@ -629,7 +637,7 @@ __global__ void __launch_bounds__(64 * NC / CW * KH) prefill_mfma_bf16(const Pre
       constexpr int TPR = PT / kSlots, CPT = D / TPR, CB = CPT < 32 ? CPT : 32, KB = 4;  // threads per row
       const int slot = threadIdx.x / TPR, part = threadIdx.x % TPR;
       const int c = c_base + (slot >> 4), rr = slot & 15;
-      const int g = c % G, tok = 16 * (c / G) - tok0 + rr;
+      const int g = c % G, tok = 16 * (c / G) - tok0 + rr;  // divisions: with step_of the merge takes 130 registers, not 122
       if (tok < ntok) {
         uint16_t* orow = (uint16_t*)a.out + (int64_t)(row0 + tok) * a.o_st + (int64_t)(h * G + g) * a.o_sh;
         for (int c0 = CPT * part; c0 < CPT * (part + 1); c0 += CB) {
@@ -730,7 +738,9 @@ static int prefill_chunk(int max_context, int splits) {
 }
 
 // Split count policy, over `tiles` 16-token query tiles of all sequences and the longest context:
-//  - under 512 keys: one split (two of 256 or less cost their merge: 448 keys 18.2 against 19.0 us, 343 11.6 / 12.2).
+//  - up to 448 keys, 511 at head_dim 128: one split (two cost their merge, us with one and two: head_dim 64, four 100-token
+//    chunks, 440 keys 9.7 / 10.3, 460 10.4 / 10.3, INT8 10.9 / 11.1 and 11.9 / 11.2; head_dim 128 440 keys 14.1 / 15.5, 500
+//    15.3 / 15.6, INT8 chunks up to 280 at 503 19.5 / 22.5, 100 at 500 18.9 / 17.6).
 //  - from 4096 keys, or from 2048 where not even two whole splits a unit fit one workgroup per CU: about two workgroups
 //    per CU over units of whole 16-token steps (512 tokens at 8K 28.6 us with 8 splits, two chunks a workgroup, 30.8
 //    with 4; 241 tokens at 6.8K at head_dim 128 35.7 with 16, 41.5 with 8).
@@ -739,12 +749,12 @@ static int prefill_chunk(int max_context, int splits) {
 //    with three, 16.2 with five; 22 at 2.4K 11.9 with 8, 12.6 with 10; 298 at 3.8K (format B) 34.7 with 8, 64.6 with 12.
 // At least 256 keys a split and at most 32 splits in any case. (Graph replays of 73 shapes, this rule's time over the
 // best of all layouts and split counts: 1.02 in the geometric mean, 1.13 with two workgroups per CU throughout.)
-static int prefill_splits_host(int Hkv, int G, int64_t tiles, int max_context, int cu_count) {
+static int prefill_splits_host(int Hkv, int G, int D, int64_t tiles, int max_context, int cu_count) {
   if (tiles <= 0 || max_context <= 0) return 1;
   const int64_t cu = std::max(cu_count, 1);
   const int64_t fit = cu / std::max<int64_t>(1, Hkv * ((tiles * G + 7) / 8));  // splits at one workgroup per CU
   int64_t want;
-  if (max_context < 512) {
+  if (max_context < (D == 128 ? 512 : 449)) {
     want = 1;
   } else if (max_context >= 4096 || (fit < 2 && max_context >= 2048)) {
     const int tt = prefill_subtiles(G, 8);
@@ -777,7 +787,7 @@ extern "C" int32_t sipa_prefill_splits(int32_t num_q_heads, int32_t num_kv_heads
                                        int64_t query_tiles, int32_t max_context, int32_t cu_count) {
   if (num_kv_heads <= 0 || num_q_heads < num_kv_heads) return 1;
   if (cu_count <= 0) cu_count = sipa_device_cu_count(-1);
-  return prefill_splits_host(num_kv_heads, num_q_heads / num_kv_heads, query_tiles, max_context, cu_count);
+  return prefill_splits_host(num_kv_heads, num_q_heads / num_kv_heads, head_dim, query_tiles, max_context, cu_count);
 }
 
 extern "C" int64_t sipa_prefill_workspace_bytes(int32_t num_seqs, int32_t num_q_heads, int32_t num_kv_heads,
@@ -863,7 +873,7 @@ extern "C" int32_t sipa_prefill(const sipa_prefill_params* p, void* stream) {
   const int cus = sipa_device_cu_count(-1);
   int splits = p->num_splits;
   if (splits <= 0)
-    splits = prefill_splits_host(Hkv, G, (int64_t)S * ((p->max_query_len + 15) / 16), p->max_context, cus);
+    splits = prefill_splits_host(Hkv, G, D, (int64_t)S * ((p->max_query_len + 15) / 16), p->max_context, cus);
   const int chunk = prefill_chunk(p->max_context, splits);
   const int nchunk = (p->max_context + chunk - 1) / chunk;  // key chunks per unit
   // split launches: whole groups of 8 units, one XCD each (the kernel's workgroup-to-unit mapping); a
@@ -908,7 +918,14 @@ extern "C" int32_t sipa_prefill(const sipa_prefill_params* p, void* stream) {
              SIPA_EUNSUPPORTED, "format B pools take SIPA_PREFILL_W4X2 or _W8X1 (16-wave workgroups cannot hold "
              "their registers)");
   const PfShape shape = prefill_shape(layout);
-  const int64_t qtiles64 = prefill_units(p->max_query_len, G, shape.nc);
+  // Whole 16-token steps where they fit one workgroup per CU: the same time limit on fewer columns (1.5B 5 x 36 tokens at 73
+  // keys 8.2 us packed, 7.6 whole, 3 x 136 at 430 15.4 / 14.1, 6 x 21 at 164 9.6 / 8.5). Packed units above: fewer
+  // workgroups to go round (INT8 chunks up to 461 tokens at 4.4K 63.1 packed, 75.8 whole, four 2048-token prompts 44.8 /
+  // 45.5).
+  const int whole = prefill_subtiles(G, shape.nc) * G;
+  const int64_t whole_units = (int64_t)S * Hkv * prefill_units(p->max_query_len, G, whole);
+  const int cols = grid_of(whole_units, shape.kh) <= cus ? whole : shape.nc;
+  const int64_t qtiles64 = prefill_units(p->max_query_len, G, cols);
   const int64_t units = (int64_t)S * Hkv * qtiles64;
   SIPA_CHECK(units <= 0x7fffffff, SIPA_EINVAL, "%lld units exceed the grid limit", (long long)units);
   const int qtiles = (int)qtiles64;
@@ -946,6 +963,8 @@ extern "C" int32_t sipa_prefill(const sipa_prefill_params* p, void* stream) {
   a.S = S;
   a.G = G;
   a.qtiles = qtiles;
+  a.cols = cols;
+  a.inv_g = (uint32_t)(((1ll << 31) + G - 1) / G);
   a.npair = S * Hkv;
   a.T = p->num_tokens;
   a.nb = p->num_blocks;

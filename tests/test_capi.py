@@ -374,9 +374,10 @@ def test_layer_out_refuses_bad_arguments():
 
 
 @pytest.mark.parametrize("Hq,D,tiles,ctx,want", [
-    (14, 64, 4, 511, 1), (14, 64, 4, 512, 2), (14, 64, 8, 1003, 4), (14, 64, 38, 1128, 3), (14, 64, 150, 1530, 1),
+    (14, 64, 4, 448, 1), (14, 64, 4, 449, 2), (14, 64, 200, 460, 1), (12, 128, 4, 511, 1), (12, 128, 4, 512, 2),
+    (14, 64, 4, 512, 2), (14, 64, 8, 1003, 4), (14, 64, 38, 1128, 3), (14, 64, 150, 1530, 1),
     (12, 128, 19, 3765, 8), (12, 128, 84, 1711, 2), (14, 64, 86, 3012, 3), (14, 64, 4, 4095, 8), (14, 64, 4, 4096, 16)])
 def test_prefill_split_policy_between_short_and_long_contexts(Hq, D, tiles, ctx, want):
-    """One workgroup per CU and at most 8 splits between 512 and 4096 keys; two workgroups per CU from 4096, or from 2048
+    """One workgroup per CU and at most 8 splits from 449 (head_dim 128: 512) to 4096 keys; two workgroups per CU from 4096, or from 2048
     where one split a unit already fills more than half the CUs."""
     assert _hip.lib().sipa_prefill_splits(Hq, 2, D, tiles, ctx, 256) == want

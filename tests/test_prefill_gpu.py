@@ -506,3 +506,28 @@ def test_units_packed_across_token_steps(Hq, Hkv, D, layout, splits):
     rows = np.concatenate([np.arange(s, s + n) for s, n in zip(starts, qlen)])
     assert_bf16_close(got[rows], ref[rows], f"packed {layout}")
     assert (got[np.setdiff1d(np.arange(T), rows)] == SENTINEL).all()
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(10, 2, 64), (12, 2, 128), (14, 2, 64), (24, 8, 128)])
+@pytest.mark.parametrize("layout", ["w4x2", "w8x1", "w16x1", "w16h2"])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_packed_units_equal_whole_steps(Hq, Hkv, D, layout, splits):
+    """Launches of more than one workgroup per CU pack their units' columns, smaller ones take whole 16-token steps: thirty
+    sequences together against each of them alone (the test above has such calls against the oracle). One split: the same
+    bits. Several: a token's unit may reach into a split that its other unit does not, and its own output then passes
+    through that merge's fp16 (2^-11 of a split's mean of V rows) before its rounding to bf16."""
+    ctx, qlen = [17, 33, 100, 700, 900] * 6, [17, 33, 47, 129, 16] * 6
+    q, k, v, bt, c, st, ln, tables, starts, T = make_prefill(ctx, qlen, Hq, Hkv, D, seed=Hq, gap=2)
+    assert len(ctx) * Hkv * -(-129 // 16) > 256
+    print(f"case units {Hq}/{Hkv}/{D} {layout} splits {splits}", flush=True)
+    kw = dict(num_splits=splits, wg_layout=layout)
+    out = paged_prefill_attention(q, k, v, bt, c, st, ln, D ** -0.5, max(ctx), max(qlen), out=torch.full_like(q, SENTINEL),
+                                  **kw)
+    alone = torch.full_like(q, SENTINEL)
+    for i in range(30):
+        row = slice(i, i + 1)
+        paged_prefill_attention(q, k, v, bt[row], c[row], st[row], ln[row], D ** -0.5, max(ctx), max(qlen), out=alone, **kw)
+    if splits == 1:
+        assert torch.equal(out, alone)
+    out, alone = out.float(), alone.float()
+    assert ((out - alone).abs() <= 2.0 ** -11 * v.abs().max() + 2.0 ** -7 * torch.maximum(out.abs(), alone.abs())).all()

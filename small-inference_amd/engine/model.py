@@ -90,8 +90,10 @@ class Qwen2Model:
             if T > hip_layer.MAX_TOKENS:
                 qkv = hip_layer.layer_qkv_large(x, w, cfg.rms_norm_eps, rot, Hq + Hkv, d)
             else:
-                target = getattr(cache, "store_target", None)  # caches that take K and V straight from the projection
-                store = target(i, x, Hkv, d) if target is not None else None
+                # caches that take K and V straight from the projection; asked of the class, so that an object which
+                # passes other names on to a cache but has a write of its own keeps it
+                target = getattr(type(cache), "store_target", None)
+                store = target(cache, i, x, Hkv, d) if target is not None else None
                 qkv = hip_layer.layer_qkv(x, w, cfg.rms_norm_eps, rot, Hq + Hkv, d, store)
             qkv = qkv.view(T, Hq + 2 * Hkv, d)
             if store is None:

@@ -253,20 +253,23 @@ class PagedKVCache:
         self.v[layer][:, m.slot_blocks, m.slot_offsets] = v.transpose(0, 1)
 
     def store_target(self, layer: int, x: torch.Tensor, heads: int, head_dim: int) -> tuple | None:
-        """Where write(layer, k, v) would store the bf16 rows projected from x [T, hidden], for a projection kernel that stores them itself
-        (the kv fields of sipa_linear_params: heads, pools, strides, slots): it saves the write's launch and one pass
-        over K and V. None where write() has to be called: another pool dtype or device, rows that are not the
-        forward's, a cache that writes in a way of its own (another write method, in a subclass, the class or the object)."""
-        m, k, v = self.meta, self.k, self.v
-        if type(self).write is not _STORE or "write" in self.__dict__ or m is None or not k.is_cuda or \
-                k.get_device() != x.get_device() or v.get_device() != x.get_device() or k.dtype is not torch.bfloat16 or v.dtype is not torch.bfloat16 or not k.is_contiguous() or \
-                not v.is_contiguous() or v.shape != k.shape or k.dim() != 5 or k.shape[1] != heads or \
-                k.shape[4] != head_dim:
+        """Where write(layer, k, v) would store the bf16 rows projected from x [T, hidden], for a projection kernel that stores
+        them itself (the kv fields of sipa_linear_params: heads, pools, strides, slots): it saves the write's launch and
+        one pass over K and V. None where write() has to be called: another pool dtype or device, rows that are not the
+        forward's, a cache that writes in a way of its own (another write method, in a subclass, the class or the
+        object)."""
+        m, k, v, dev = self.meta, self.k, self.v, x.get_device()
+        write = self.write
+        if getattr(write, "__func__", None) is not _STORE or write.__self__ is not self or m is None or not k.is_cuda:
+            return None
+        for t in (k, v):
+            if t.get_device() != dev or t.dtype is not torch.bfloat16 or not t.is_contiguous():
+                return None
+        if v.shape != k.shape or k.dim() != 5 or k.shape[1] != heads or k.shape[4] != head_dim:
             return None
         blocks, offsets = m.slot_blocks, m.slot_offsets
         for t in (blocks, offsets):
-            if t.dtype is not torch.int64 or t.numel() != x.shape[0] or not t.is_contiguous() or \
-                    t.get_device() != x.get_device():
+            if t.dtype is not torch.int64 or t.numel() != x.shape[0] or not t.is_contiguous() or t.get_device() != dev:
                 return None
         _, sh, sn, sb, _ = k.stride()
         return (heads, layer_ptr(k, layer), layer_ptr(v, layer), sh, sn, sb, blocks.data_ptr(), offsets.data_ptr())

@@ -231,6 +231,51 @@ def test_caches_that_write_their_own_way_are_asked_to():
         assert cache.store_target(0, x, 2, 64) is None
 
 
+def test_a_wrapped_cache_keeps_its_write():
+    """An object that passes names on to a cache, and a subclass whose write is found by __getattribute__, see every write
+    of a layer."""
+    cfg = ModelConfig(vocab_size=64, hidden_size=128, intermediate_size=64, num_layers=1, num_q_heads=4, num_kv_heads=2,
+                      head_dim=32)
+    model = Qwen2Model(cfg, "cuda", torch.bfloat16, seed=1, max_positions=64, std=0.05)
+    m = fragmented_manager(16, 16, torch.Generator().manual_seed(4))
+    m.allocate(0, 5)
+    meta = build_metadata(m, [(0, 0, 5)], "cuda")
+    seen = []
+
+    class Wrapper:
+        def __init__(self, cache):
+            self.cache = cache
+
+        def __getattr__(self, name):
+            return getattr(self.cache, name)
+
+        def write(self, layer, k, v):
+            seen.append((k.clone(), v.clone()))
+            self.cache.write(layer, k, v)
+
+    class Watched(PagedKVCache):
+        def __getattribute__(self, name):
+            found = super().__getattribute__(name)
+            if name != "write":
+                return found
+            return lambda layer, k, v: (seen.append((k.clone(), v.clone())), found(layer, k, v))
+
+    x = randn(torch.Generator(device="cuda").manual_seed(2), 5, 128)
+    rot = model.rotary.rows(meta.positions, torch.bfloat16)
+    results = []
+    for make in (PagedKVCache, lambda *a, **kw: Wrapper(PagedKVCache(*a, **kw)), Watched):
+        cache = make(cfg, m.num_blocks, 16, "cuda", torch.bfloat16, attn_backend="hip")
+        cache.begin(5, meta)
+        seen.clear()
+        with torch.inference_mode():
+            results.append(model.layer_forward(0, x, meta.positions, cache, rot))
+        assert len(seen) == (make is not PagedKVCache)
+        for k, v in seen:
+            assert torch.equal(cache.k[0][:, meta.slot_blocks, meta.slot_offsets], k.transpose(0, 1))
+            assert torch.equal(cache.v[0][:, meta.slot_blocks, meta.slot_offsets], v.transpose(0, 1))
+    assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
+
+
 @pytest.mark.parametrize("T", [1, 3, 40])
 def test_attention_results_of_other_forms(T):
     """What a cache's attend returns is read by the kernels only in the form that they take: other strides and offsets

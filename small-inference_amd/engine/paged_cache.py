@@ -167,6 +167,13 @@ def _run(seqs: list[int]) -> slice | None:
     return slice(seqs[0], seqs[-1] + 1) if seqs[-1] - seqs[0] + 1 == len(seqs) else None
 
 
+def _kernel_rows(q: torch.Tensor) -> bool:
+    """Whether the decode kernels take q's rows [S, H, d] as they lie: channels next to each other, 16-byte aligned heads."""
+    st, sh, sd = q.stride()
+    size = q.element_size()
+    return sd == 1 and st * size % 16 == 0 and sh * size % 16 == 0 and q.data_ptr() % 16 == 0
+
+
 class PagedKVCache:
     def __init__(self, cfg: ModelConfig, num_blocks: int, block_size: int, device: str | torch.device,
                  dtype: torch.dtype, attn_backend: str = "gather"):
@@ -328,6 +335,8 @@ class PagedKVCache:
         in_place = type(rows) is slice
         out = None if rows is None else torch.empty(T, Hq * d, device=q.device, dtype=q.dtype)
         q_dec = q if rows is None else q[rows]
+        if in_place and not _kernel_rows(q_dec):  # as the gather would lay them out
+            q_dec = q_dec.clone(memory_format=torch.contiguous_format)
         dec_out = out[rows].view(-1, Hq, d) if in_place else None
         if self._plan is None or self._plan_scale != scale:  # first layer of the forward: validate once
             # The host-side lengths let a ragged batch run from a work list (built once, used by every layer).

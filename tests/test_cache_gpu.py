@@ -197,3 +197,33 @@ def test_rows_in_any_order_match_the_gather_backend(fmt, order):
         b = results[1][key]
         # other split counts, another order of fp32 sums: a bf16 step of outputs below 4
         assert (a.float() - b.float()).abs().max() <= 2.0 ** -6, key
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("form", ["channels apart", "offset", "odd rows"])
+def test_decode_rows_of_any_layout_in_a_mixed_forward(form, dtype):
+    """Decode rows that stand together in a forward with a chunk, in a q whose channels, rows or first element lie as no
+    kernel takes them: the result of a contiguous q (the chunk attends over gathered keys: blocks of 32 tokens)."""
+    cfg = ModelConfig(vocab_size=64, hidden_size=896, intermediate_size=64, num_layers=1, num_q_heads=14, num_kv_heads=2,
+                      head_dim=64)
+    m = fragmented_manager(32, 32, torch.Generator().manual_seed(1))
+    for s, n in enumerate((40, 70, 9)):
+        m.allocate(s, n)
+    cache = PagedKVCache(cfg, m.num_blocks, 32, "cuda", dtype, attn_backend="hip")
+    g = torch.Generator(device="cuda").manual_seed(2)
+    for pool in (cache.k, cache.v):
+        pool.copy_(torch.randn(pool.shape, device="cuda", generator=g))
+    meta = build_metadata(m, [(0, 39, 1), (1, 69, 1), (2, 4, 5)], "cuda")
+    q = torch.randn(7, 14, 64, device="cuda", generator=g).to(dtype)
+    cache.begin(7, meta)
+    ref = cache.attend(0, q, meta.positions, 0.125)
+    if form == "channels apart":
+        other = torch.empty(7, 64, 14, device="cuda", dtype=dtype).transpose(1, 2)
+    elif form == "offset":
+        other = torch.empty(7 * 14 * 64 + 1, device="cuda", dtype=dtype)[1:].view(7, 14, 64)
+    else:
+        other = torch.empty(7, 14 * 64 + 3, device="cuda", dtype=dtype)[:, :14 * 64].view(7, 14, 64)
+    other.copy_(q)
+    cache.begin(7, meta)
+    print(f"case layout {form} {dtype}", flush=True)
+    assert torch.equal(cache.attend(0, other, meta.positions, 0.125), ref)

@@ -13,6 +13,7 @@ import functools
 
 import torch
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from . import _hip
 
@@ -35,11 +36,27 @@ def _ok(t, device: int, *shape: int) -> bool:
         t.is_contiguous() and t.data_ptr() % 16 == 0
 
 
+# looked up once: a layer asks them all for every call
+_inference, _autocast, _compiling = torch.is_inference_mode_enabled, torch.is_autocast_enabled, torch.compiler.is_compiling
+_tracing, _transform = torch._C._get_tracing_state, torch._C._functorch.peek_interpreter_stack
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+
+
+def _plain() -> bool:
+    """Whether torch operations would just run: under torch.inference_mode (the kernels record nothing for autograd, and
+    saved-tensor hooks do not reach them there), not under autocast, whose type the products' results have, and with
+    nobody between who is to see each operation: vmap, grad or jvp, tracing or compilation, a dispatch mode, or a function
+    mode other than the default device's."""
+    if not _inference() or _autocast() or _compiling() or _tracing() is not None or _transform() is not None or \
+            _dispatch_modes():
+        return False
+    n = _function_modes()
+    return n == 0 or all(type(torch._C._get_function_stack_at(i)) is DeviceContext for i in range(n))
+
+
 def rows_ok(x: torch.Tensor, norm_weight: torch.Tensor) -> bool:
-    """Whether rms_norm can run on rows x [T, K]. Only under torch.inference_mode: the kernels record nothing for
-    autograd, and forward-mode derivatives and saved-tensor hooks do not reach them there. Not under autocast, whose type
-    the products' results have."""
-    if not (torch.is_inference_mode_enabled() and x.is_cuda and x.dim() == 2) or torch.is_autocast_enabled():
+    """Whether rms_norm can run on rows x [T, K], and stand for the torch operations."""
+    if not (x.is_cuda and x.dim() == 2 and _plain()):
         return False
     T, K = x.shape
     dev = x.get_device()

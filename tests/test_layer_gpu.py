@@ -394,3 +394,56 @@ def test_captured_layers_own_their_merge_counters(T, hidden, attn, inter):
             graphs[1][0].replay()
         check(0)
         check(1)
+
+
+def test_transforms_and_modes_keep_the_torch_operations():
+    """vmap over a layer, and modes that are to see each of its operations, under inference_mode: what the torch operations
+    give; the default device's own mode changes nothing."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    cfg = ModelConfig(vocab_size=64, hidden_size=128, intermediate_size=64, num_layers=1, num_q_heads=4, num_kv_heads=2,
+                      head_dim=32)
+    model = Qwen2Model(cfg, "cuda", torch.bfloat16, seed=1, max_positions=64, std=0.05)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    xs, pos = randn(g, 3, 4, 128), torch.arange(4, device="cuda")
+    rot = model.rotary.rows(pos, torch.bfloat16)
+
+    class Values:  # each query head returns its group's values
+        def write(self, layer, k, v):
+            self.v = v
+
+        def attend(self, layer, q, positions, scale):
+            return self.v.repeat_interleave(2, 1).reshape(q.shape[0], -1)
+
+    def layer(x):
+        return model.layer_forward(0, x, pos, Values(), rot)
+
+    linears = []
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            linears.append(func is F.linear)
+            return func(*args, **(kwargs or {}))
+
+    class Operations(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            linears.append(func in (torch.ops.aten.mm.default, torch.ops.aten.addmm.default, torch.ops.aten.linear.default))
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad():
+        ref = [layer(x) for x in xs]
+    with torch.inference_mode():
+        assert hip_layer.supported(xs[0], model.layers[0], rot, 8, 32)
+        with torch.device("cuda"):
+            assert hip_layer.supported(xs[0], model.layers[0], rot, 8, 32)
+        out = torch.func.vmap(layer)(xs)
+        for mode in (Functions, Operations):
+            linears.clear()
+            with mode():
+                seen = layer(xs[0])
+            assert sum(linears) == 4 and torch.equal(seen, ref[0])
+        traced = torch.jit.trace(layer, (xs[0],), check_trace=False)(xs[1])
+    assert torch.equal(traced, ref[1])
+    for a, b in zip(out, ref):
+        assert rel(a, b.double()) < 2.0 ** -6

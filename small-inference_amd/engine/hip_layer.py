@@ -72,6 +72,8 @@ def supported(x: torch.Tensor, w, rot, heads: int, head_dim: int) -> bool:
     T, hidden = x.shape
     dev, width, inter, attn = x.get_device(), heads * head_dim, w.down_w.shape[-1], w.o_w.shape[-1]
     cos, sin = rot
+    if max(width, inter, attn) > 1 << 20 or T * max(width, inter) >= 1 << 34:  # the library's limits
+        return False
     return (head_dim % 16 == 0 and hidden % 64 == 0 and inter % 64 == 0 and attn % 64 == 0 and
             _ok(w.qkv_w, dev, width, hidden) and _ok(w.qkv_b, dev, width) and _ok(w.o_w, dev, hidden, attn) and
             _ok(w.post_norm, dev, hidden) and _ok(w.gate_up_w, dev, 2 * inter, hidden) and

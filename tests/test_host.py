@@ -642,3 +642,20 @@ def test_layer_merge_counters_lie_in_the_calls_own_memory(monkeypatch, T, hidden
                for t in made)
     assert p.scratch + p.scratch_bytes <= p.counters or p.counters + size <= p.scratch
     assert hip_decode._workspaces == held
+
+
+def test_layer_sizes_past_the_librarys_limits_keep_the_torch_operations(monkeypatch):
+    """A layer whose sizes the library refuses is not given to it (meta tensors: only shapes and strides are asked for)."""
+    from engine import hip_layer
+    from engine.model import Layer
+
+    monkeypatch.setattr(hip_layer, "rows_ok", lambda x, w: True)
+    monkeypatch.setattr(hip_layer, "_ok", lambda t, device, *shape: tuple(t.shape) == shape)
+
+    def supported(T, inter):
+        z = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device="meta")  # noqa: E731
+        w = Layer(z(64), z(192, 64), z(192), z(64, 64), z(64), z(2 * inter, 64), z(64, inter))
+        return hip_layer.supported(z(T, 64), w, (z(T, 1, 64), z(T, 1, 64)), 3, 64)
+
+    assert supported(1 << 20, 16384 - 64) and supported(4, 1 << 20)
+    assert not supported(1 << 20, 16384) and not supported(4, (1 << 20) + 64)

@@ -77,8 +77,8 @@ __device__ __forceinline__ int linear_row(const LinearArgs& a, int tile, int r) 
 }
 
 // Where channel c of token t is stored. K and V straight to the pools: a separate store launch took 2.5 to 3.8 us a layer
-// (kernel and the gap before it) for a few KB; without it a replayed 24-layer step of 8 sequences takes 889 us, 950 with it,
-// and 24 layers over 544 mixed tokens 2230 us, 2306 with it.
+// (kernel and the gap before it) for a few KB; without it a replayed 24-layer step of 8 sequences went from 950 to 889 us,
+// and 24 layers over 544 mixed tokens from 2306 to 2230.
 template <int EPI>
 __device__ __forceinline__ uint16_t* out_at(const LinearArgs& a, int t, int c) {
   if (EPI == kEpiRope && a.kv_heads > 0 && c >= a.kv0) {
@@ -119,8 +119,8 @@ __device__ __forceinline__ u32x4 scale_channels(u32x4 x, u32x4 w, float& ss) {
 // flight together, and their sums meet in LDS.
 //
 // Measured in a graph, weights from memory, 8 tokens, against tile_linear's smallest tile and the GEMM library's product
-// alone (us): norm + QKV 1152 x 896 + bias + rotary 4.9, 6.1, 5.6; 2048 x 1536 6.1, 8.0, 7.2; 896 x 896 + residual 4.1,
-// 4.4, 5.6. An empty launch there is about 2.
+// alone (us): norm + QKV 1152 x 896 + bias + rotary 5.1, 6.2, 5.7; 2048 x 1536 6.3, 8.3, 7.2; 896 x 896 + residual 4.1,
+// 4.2, 5.5. An empty launch there is about 2.
 constexpr int kSkinnyWaves = 8;
 
 template <int EPI, bool NORM, int U>
@@ -225,9 +225,9 @@ __global__ void __launch_bounds__(64 * kSkinnyWaves) skinny_linear(const LinearA
 // six share it and the last one to arrive adds their sums in split order.
 //
 // Measured in a graph, weights from memory, against the GEMM library's product alone (us; the library needs a norm, 2.9,
-// a rotary, 2.1, a SwiGLU, 2.2 to 6, or a residual launch, 2, besides): 64 tokens: QKV 1152 x 896 6.3 (7.9), o 896 x 896
-// 4.5 (7.8), gate/up 9728 x 896 9.4 (11.8), down 896 x 4864 8.4 (13.7); 544 tokens: 9.6 (8.3), 5.6 (7.9), 25.3 (17.0),
-// 16.7 (15.9).
+// a rotary, 2.1, a SwiGLU, 2.2 to 6, or a residual launch, 2, besides): 64 tokens: QKV 1152 x 896 6.4 (8.0), o 896 x 896
+// 4.4 (7.9), gate/up 9728 x 896 10.0 (11.9), down 896 x 4864 8.4 (13.6); 544 tokens: 9.6 (8.4), 5.5 (7.9), 26.3 (17.7),
+// 15 to 16 (16.5).
 template <int EPI, bool NORM, int TT, int TN, int NR>
 __global__ void __launch_bounds__(256) tile_linear(const LinearArgs a) {
   static_assert(NR % 2 == 0, "a ring slot always meets the same LDS buffer");
@@ -441,26 +441,25 @@ struct LinearPlan {
 
 // Tiles 64 x 64, 64 x 128 and 128 x 128 of a gated projection by the workgroups each makes: its time at K = 896 is close
 // to 6 + 4.1 c, 4 + 8 c and (17.5, 25, 13 c from three on) us, c the most workgroups a CU gets (in proportion at 1536),
-// measured at 33 to 1000 tokens on both model shapes. Against the smallest tile of at most 200 workgroups, which this
-// replaces: 0.5B 160 tokens 18.7 -> 13.1 us (228 workgroups of 64 x 128, not 152 of 128 x 128), 800 39.2 -> 35.6, 1.5B
-// 160 39.2 -> 32.3.
-static int gated_tile(int64_t g2, int64_t g3, int64_t g4) {
-  const auto per_cu = [](int64_t g) { return (double)((g + 255) / 256); };
+// measured at 33 to 1000 tokens on both model shapes. Against 128 x 128 throughout: 0.5B 160 tokens 18.0 -> 13.4 us, 800
+// 37.1 -> 33.5, 1.5B 160 36.8 -> 32.5.
+static int gated_tile(int64_t g2, int64_t g3, int64_t g4, int cus) {
+  const auto per_cu = [&](int64_t g) { return (double)((g + cus - 1) / cus); };
   const double t2 = 6 + 4.1 * per_cu(g2), t3 = 4 + 8 * per_cu(g3);
-  const double t4 = g4 <= 256 ? 17.5 : g4 <= 512 ? 25 : 13 * per_cu(g4);
+  const double t4 = g4 <= cus ? 17.5 : g4 <= 2 * cus ? 25 : 13 * per_cu(g4);
   return t4 <= t2 && t4 <= t3 ? 4 : t3 <= t2 ? 3 : 2;
 }
 
-// The smallest tile whose grid stays within a number of workgroups that depends on the epilogue: small tiles fill the
-// chip, large ones read less. ROPE: 640 (K is short and the tiles' norm is their cost; QKV 0.5B at 544 tokens 9.6 with
-// 612 small workgroups, 10.9 with 162). SILU: 200 workgroups of 32 x 64, gated_tile above them. RESIDUAL: 256, and a K
-// from 4096 on is then split, at most six ways (896 x 4864 at 8 tokens 7.5 us with six, 8.0 with eight, 11.5 with one):
-// tiles of 32 x 32 until the grid has about 256 again, larger ones only as far as one workgroup a CU goes (896 x 4864 at
-// 300 tokens, 140 tiles, 14.7 us whole and 17.4 in halves; 800 tokens, 182 tiles, 21.7 and 25.7; 160 tokens, 140 tiles
-// of 32 x 32, 12.7 and 11.9). From 128 slices of K on, a grid too large to split takes the next larger tile in halves
-// (1536 x 8960: 160 tokens 23.2 -> 20.1 us, 300 29.2 -> 24.8; 896 x 4864 at 544 16.0 -> 17.7, not there).
-// num_splits and shape of the caller come first (0: the rule).
-static LinearPlan plan_linear(int epi, bool norm, int T, int tiles, int K, int want_splits, int want_shape) {
+// The smallest tile whose grid stays within a number of workgroups that depends on the epilogue (given for 256 CUs): small
+// tiles fill the chip, large ones read less. ROPE: 640 (K is short and the tiles' norm is their cost; QKV 0.5B at 544
+// tokens 9.4 us with 612 workgroups, 10.8 with 162). SILU: 200 workgroups of 32 x 64, gated_tile above them. RESIDUAL: 256,
+// and a K from 4096 on is then split, at most six ways (896 x 4864 at 8 tokens 7.7 us with six, 8.2 with eight, 10.6 with
+// one): tiles of 32 x 32 until the grid has about 256 again, larger ones only as far as one workgroup a CU goes (896 x
+// 4864, whole and in halves: 300 tokens, 140 tiles, 14.3 and 17.6; 800 tokens, 182 tiles, 21.2 and 25.6). From 96 slices of
+// K on, a grid too large to split takes the next larger tile in halves (us without and with: 1536 x 8960 160 tokens 23.4
+// and 20.0, 300 28.9 and 25.0; 1536 x 6144, 96 slices, 17.2 and 15.3, 21.4 and 19.1; 896 x 4864, 76 slices, 544 tokens 14.7
+// and 17.0: not there). num_splits and shape of the caller come first (0: the rule).
+static LinearPlan plan_linear(int epi, bool norm, int T, int tiles, int K, int want_splits, int want_shape, int cus) {
   LinearPlan p{};
   const int units = K >> 6;
   auto grid = [&](int s) {
@@ -468,18 +467,18 @@ static LinearPlan plan_linear(int epi, bool norm, int T, int tiles, int K, int w
   };
   if (want_shape > 0) {
     p.shape = want_shape - 1;
-  } else if (T <= 16 && units <= 24 && tiles <= 256 && want_splits <= 1) {
+  } else if (T <= 16 && units <= 24 && tiles <= cus && want_splits <= 1) {
     p.shape = kSkinny;
   } else {
-    const int most = epi == kEpiRope ? 640 : epi == kEpiSilu ? 200 : 256;
+    const int most = epi == kEpiRope ? 5 * cus / 2 : epi == kEpiSilu ? 25 * cus / 32 : cus;
     p.shape = epi == kEpiSilu ? 1 : 0;
     if (epi != kEpiSilu)
       while (p.shape + 1 < kNumTiles && grid(p.shape) > most) ++p.shape;
     else if (grid(1) > most)
-      p.shape = gated_tile(grid(2), grid(3), grid(4));
+      p.shape = gated_tile(grid(2), grid(3), grid(4), cus);
     // a long K in whole workgroups of one tile against two halves of the next larger one
-    if (epi == kEpiResidual && !norm && want_splits <= 0 && units >= 128 && p.shape < 2 &&
-        (p.shape == 0 ? grid(0) * 5 > 4 * 256 : 2 * grid(1) > 256) && 2 * grid(p.shape + 1) <= 256)
+    if (epi == kEpiResidual && !norm && want_splits <= 0 && units >= 96 && p.shape < 2 &&
+        (p.shape == 0 ? grid(0) * 5 > 4 * cus : 2 * grid(1) > cus) && 2 * grid(p.shape + 1) <= cus)
       ++p.shape;
   }
   p.splits = 1;
@@ -487,10 +486,10 @@ static LinearPlan plan_linear(int epi, bool norm, int T, int tiles, int K, int w
     const int64_t g = grid(p.shape);
     if (want_splits > 0)
       p.splits = want_splits;
-    else if (K >= 4096 && p.shape == 0 && g * 5 <= 4 * 256)
-      p.splits = (int)std::min<int64_t>(6, (256 + g - 1) / g);
+    else if (K >= 4096 && p.shape == 0 && g * 5 <= 4 * cus)
+      p.splits = (int)std::min<int64_t>(6, (cus + g - 1) / g);
     else if (K >= 4096 && p.shape > 0)
-      p.splits = (int)std::min<int64_t>(6, std::max<int64_t>(1, 256 / g));
+      p.splits = (int)std::min<int64_t>(6, std::max<int64_t>(1, cus / g));
     const int per = (units + p.splits - 1) / p.splits;
     p.splits = (units + per - 1) / per;
     if (p.splits > 1) {
@@ -665,8 +664,9 @@ static int check_linear(const sipa_linear_params* p) {
 
 static LinearPlan plan_of(const sipa_linear_params* p) {
   const int tiles = p->out_features / 16;  // SILU: 8 gate and 8 up rows each
+  const int cus = sipa_device_cu_count(-1);
   return plan_linear(p->epilogue, p->norm_weight != nullptr, p->num_tokens, tiles, p->in_features, p->num_splits,
-                     p->tile);
+                     p->tile, cus > 0 ? cus : 256);
 }
 
 extern "C" int64_t sipa_linear_scratch_bytes(const sipa_linear_params* p) {

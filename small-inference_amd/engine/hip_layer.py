@@ -23,9 +23,10 @@ RESIDUAL, ROPE, SILU = 0, 1, 2  # SIPA_LINEAR_*
 # operations around it. A 0.5B layer's projections and what they fuse (us, fused against library): 64 tokens 29 / 54,
 # 256 41 / 59, 544 57 / 64, 1024 81 / 84.
 MAX_TOKENS = 1024
-# The gated projection goes to the library above this many operations, where its large tiles are better: 0.5B at 1024
-# tokens (17.9 GFLOP) 37.9 us against 27.3 + norm and SwiGLU (10), 1.5B at 256 (14.1) 40.6 / 39, at 544 (30) 61.8 / 47.
-MAX_GATED_FLOPS = 18e9
+# The gated projection goes to the library above this many operations, where its large tiles are better. A whole layer (us,
+# fused against library): 0.5B at 768 tokens (13.4 GFLOP) 81 / 87, 832 (14.5) 88 / 92, 896 (15.6) 94 / 87, 960 96 / 97, 1024
+# (17.9) 97 / 96; 1.5B at 224 (12.3) 90 / 88, 256 (14.1) 95 / 93, 288 (15.9) 97 / 92, 320 101 / 97, 448 (24.7) 141 / 121.
+MAX_GATED_FLOPS = 15e9
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)

@@ -154,3 +154,40 @@ def test_runner_rejects_what_it_cannot_capture():
     with pytest.raises(ValueError):  # more rows than max_batch
         runner.step([0, 1, 2], torch.tensor([1, 2, 3], device="cuda"))
     runner.close()
+
+
+def test_steps_whose_decode_is_not_split():
+    """96 rows of short contexts decode in one split, so that the captured step has no split workspace, while its layers
+    share the K of their down projections among workgroups: replays equal eager steps also after the capture stream's
+    workspace was replaced and its old memory overwritten."""
+    from engine.hip_decode import grid_splits, reserve_workspace
+
+    cfg = ModelConfig(vocab_size=512, hidden_size=896, intermediate_size=4864, num_layers=3, num_q_heads=14, num_kv_heads=2,
+                      head_dim=64)
+    assert grid_splits(96, 2, 512) == 1
+    g = torch.Generator().manual_seed(3)
+    m = fragmented_manager(1024, 16, g)
+    for s in range(96):
+        m.allocate(s, 20 + s)
+    model = Qwen2Model(cfg, "cuda", torch.bfloat16, seed=3, max_positions=1024)
+    cache = PagedKVCache(cfg, m.num_blocks, 16, "cuda", torch.bfloat16, attn_backend="hip")
+    for pool in (cache.k, cache.v):
+        pool.copy_(torch.randn(pool.shape, generator=g))
+    runner = DecodeGraphRunner(model, cache, m, max_batch=96, max_context=512, buckets=[96])
+    ids = torch.randint(0, 512, (96,), generator=g).cuda()
+    runner.capture(96)
+    assert runner._graphs[96][2] is None  # no workspace among the decode's parameters
+    for i, nbytes in enumerate((0, 4 << 20, 16 << 20)):
+        for s in range(96):
+            m.append_slot(s)
+        reserve_workspace(torch.device("cuda"), runner._stream.cuda_stream, nbytes)
+        runner._workspace = None
+        torch.cuda.synchronize()
+        junk = [torch.full((1 << 18,), 0x5a5a5a5a, device="cuda", dtype=torch.int32) for _ in range(8)]
+        print(f"case unsplit step {i}", flush=True)
+        got = runner.step(list(range(96)), ids).clone()
+        torch.cuda.synchronize()
+        want = runner.step(list(range(96)), ids, graph=False)
+        assert torch.equal(got, want)
+        del junk
+    runner.close()

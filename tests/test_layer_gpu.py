@@ -114,6 +114,53 @@ def test_every_tile_shape(tile, T):
         assert rel(out, ref) < BOUND
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("T", [1, 16, 33, 129])
+def test_epilogues_with_and_without_norm(tile, T):
+    """The forms that a Qwen2 layer does not use: a residual after a normed product, rotary and gated ones without norm."""
+    if tile == 6 and T > 16:
+        return
+    g = torch.Generator(device="cuda").manual_seed(T)
+    K, d, heads, inter = 320, 48, 5, 120
+    x, nw, res, b = randn(g, T, K), 1 + 0.1 * randn(g, K), randn(g, T, heads * d), randn(g, heads * d)
+    w, gu = randn(g, heads * d, K) * 0.05, randn(g, 2 * inter, K) * 0.05
+    rot = randn(g, T, 1, d), randn(g, T, 1, d)
+    print(f"case forms tile {tile} T {T}", flush=True)
+    out = hip_layer.fused_linear(x, w, hip_layer.RESIDUAL, norm_weight=nw, eps=EPS, bias=b, residual=res, tile=tile)
+    assert rel(out, norm64(x, nw) @ w.double().t() + b.double() + res.double()) < BOUND
+    y = (x.double() @ w.double().t() + b.double()).view(T, heads, d)
+    out = hip_layer.fused_linear(x, w, hip_layer.ROPE, bias=b, rot=rot, head_dim=d, rot_channels=3 * d, tile=tile)
+    assert rel(out, torch.cat([rotate64(y[:, :3], *rot), y[:, 3:]], 1).view(T, -1)) < BOUND
+    out = hip_layer.fused_linear(x, gu, hip_layer.SILU, tile=tile)
+    y = x.double() @ gu.double().t()
+    assert rel(out, F.silu(y[:, :inter]) * y[:, inter:]) < BOUND
+
+
+@pytest.mark.parametrize("hidden,inter,Hq,d", [(896, 4864, 14, 64), (1536, 8960, 12, 128)])
+@pytest.mark.parametrize("T", [400, 544, 700, 1000, 1024])
+def test_projections_of_larger_batches(T, hidden, inter, Hq, d):
+    """Both model shapes' four projections at the tiles and splits that the library takes itself."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    heads = Hq + 4
+    x, nw, b = randn(g, T, hidden), 1 + 0.1 * randn(g, hidden), randn(g, heads * d)
+    rot = randn(g, T, 1, d), randn(g, T, 1, d)
+    print(f"case larger T {T} {hidden}", flush=True)
+    xn = norm64(x, nw)
+    w = randn(g, heads * d, hidden) * 0.05
+    out = hip_layer.fused_linear(x, w, hip_layer.ROPE, norm_weight=nw, eps=EPS, bias=b, rot=rot, head_dim=d,
+                                 rot_channels=(Hq + 2) * d)
+    y = (xn @ w.double().t() + b.double()).view(T, heads, d)
+    assert rel(out, torch.cat([rotate64(y[:, :Hq + 2], *rot), y[:, Hq + 2:]], 1).view(T, -1)) < BOUND
+    w = randn(g, 2 * inter, hidden) * 0.05
+    y = xn @ w.double().t()
+    assert rel(hip_layer.fused_linear(x, w, hip_layer.SILU, norm_weight=nw, eps=EPS),
+               F.silu(y[:, :inter]) * y[:, inter:]) < BOUND
+    for K in (hidden, inter):
+        a, w, res = randn(g, T, K), randn(g, hidden, K) * 0.05, randn(g, T, hidden)
+        out = hip_layer.fused_linear(a, w, hip_layer.RESIDUAL, residual=res)
+        assert rel(out, a.double() @ w.double().t() + res.double()) < BOUND
+
+
 @pytest.mark.parametrize("K", [8, 896, 1024, 1032, 1536, 2056, 8192])
 @pytest.mark.parametrize("T", [1, 4, 5, 300])
 def test_rms_norm_rows(T, K):
@@ -147,11 +194,43 @@ def test_rope_and_silu_rows(T, heads, extra, d):
 def test_layer_on_kernels_matches_torch_operations(T):
     """layer_forward under inference_mode (the kernels) against the same call outside it (the torch operations), and
     what the layer wrote into the cache."""
-    cfg = ModelConfig(vocab_size=64, hidden_size=896, intermediate_size=4864, num_layers=1, num_q_heads=14,
-                      num_kv_heads=2, head_dim=64)
+    for a, b in zip(*run_layer_both_ways(T, 896, 4864, 14, 64)[0]):
+        # the torch side rounds up to 16 times along a chain of operations (norm 2, projection, rotary 3, attention,
+        # projection, sum, norm 2, projection, gate 2, projection, sum), at most 2^-9 of the value each and independent:
+        # sqrt(16) 2^-9 = 2^-7 a side, 2^-6 between two sides
+        assert rel(a, b.double()) < 2.0 ** -6
+
+
+@pytest.mark.parametrize("hidden,inter,Hq,d", [(896, 4864, 14, 64), (1536, 8960, 12, 128)])
+@pytest.mark.parametrize("T", ["below", "above", 1024, 1025])
+def test_layer_on_either_side_of_the_gated_limit(T, hidden, inter, Hq, d):
+    """The last batch whose gated projection is fused, the first whose goes to the library between fused projections, the
+    last and first batch around MAX_TOKENS, against 64 bits: no further from it than the torch operations, whose roundings
+    are a superset of the kernels' (2% for the draw of the others)."""
+    most = int(hip_layer.MAX_GATED_FLOPS / (4.0 * hidden * inter))
+    assert most < 1024
+    T = {"below": most, "above": most + 1}.get(T, T)
+    (kernels, torch_ops), (x, w, rot) = run_layer_both_ways(T, hidden, inter, Hq, d)
+    qkv = (norm64(x, w.input_norm) @ w.qkv_w.double().t() + w.qkv_b.double()).view(T, Hq + 4, d)
+    qk, v = rotate64(qkv[:, :Hq + 2], *rot), qkv[:, Hq + 2:]
+    k, v = (t.transpose(0, 1).repeat_interleave(Hq // 2, 0) for t in (qk[:, Hq:], v))
+    score = torch.bmm(qk[:, :Hq].transpose(0, 1), k.transpose(1, 2).contiguous()) * d ** -0.5
+    score.masked_fill_(torch.ones(T, T, device="cuda", dtype=torch.bool).triu(1), -torch.inf)
+    attn = torch.bmm(torch.softmax(score, -1), v.contiguous()).transpose(0, 1).reshape(T, Hq * d)
+    ref = layer_out64(x, attn, w)
+    assert rel(kernels[0], ref) <= 1.02 * rel(torch_ops[0], ref) < 2.0 ** -5
+    for a, b in zip(kernels[1:], torch_ops[1:]):  # K (rounded four times less) and V in the pools
+        assert rel(a, b.double()) < 2.0 ** -7
+
+
+def run_layer_both_ways(T, hidden, inter, Hq, d):
+    """([hidden states and pools on the kernels, the same on torch operations], (x, weights, rotary rows))"""
+    cfg = ModelConfig(vocab_size=64, hidden_size=hidden, intermediate_size=inter, num_layers=1, num_q_heads=Hq,
+                      num_kv_heads=2, head_dim=d)
     model = Qwen2Model(cfg, "cuda", torch.bfloat16, seed=1, max_positions=2048, std=0.05)
     g = torch.Generator(device="cuda").manual_seed(2)
-    x = randn(g, T, 896)
+    x = randn(g, T, hidden)
+    print(f"case layer T {T} {hidden}", flush=True)
     results = []
     for fused in (True, False):
         m = fragmented_manager(128, 16, torch.Generator().manual_seed(3))
@@ -163,13 +242,9 @@ def test_layer_on_kernels_matches_torch_operations(T):
         cache.begin(T, meta)
         rot = model.rotary.rows(meta.positions, torch.bfloat16)
         with torch.inference_mode() if fused else torch.no_grad():
-            assert hip_layer.supported(x, model.layers[0], rot, 18, 64) == fused
+            assert hip_layer.supported(x, model.layers[0], rot, Hq + 4, d) == fused
             results.append((model.layer_forward(0, x, meta.positions, cache, rot), cache.k, cache.v))
-    for a, b in zip(*results):
-        # the torch side rounds up to 16 times along a chain of operations (norm 2, projection, rotary 3, attention,
-        # projection, sum, norm 2, projection, gate 2, projection, sum), at most 2^-9 of the value each and independent:
-        # sqrt(16) 2^-9 = 2^-7 a side, 2^-6 between two sides
-        assert rel(a, b.double()) < 2.0 ** -6
+    return results, (x, model.layers[0], rot)
 
 
 def test_rotate_reference_matches_the_model():

@@ -218,3 +218,8 @@ def layer_ptr(pools: torch.Tensor, layer: int) -> int:
     if not -n <= layer < n:
         raise IndexError(f"layer {layer} of {n}")
     return pools.data_ptr() + (layer + n if layer < 0 else layer) * pools.stride(0) * pools.element_size()
+
+
+def layers_contiguous(pools: torch.Tensor) -> bool:
+    """Whether every pools[layer] is contiguous (the layers themselves may lie apart, as K and V side by side do)."""
+    return pools.shape[0] > 0 and pools[0].is_contiguous()

@@ -322,7 +322,8 @@ class DecodePlan:
         """The decode over layer `layer` of pools [L, Hkv, N, B, D] (quant: scales and staging with a leading layer
         dimension too): the plan called with pools[layer] and the like, without making those views."""
         for pools in (k_pools, v_pools):
-            if pools.shape[1:] != self.pool_shape or pools.dtype != self.pool_dtype or not pools.is_contiguous():
+            if pools.shape[1:] != self.pool_shape or pools.dtype != self.pool_dtype or \
+                    not (pools.is_contiguous() or _hip.layers_contiguous(pools)):
                 raise ValueError("the pools do not match the plan")
         self._bind_q(q)
         p = self.params

@@ -153,6 +153,19 @@ def store_tokens(x: torch.Tensor, blocks: torch.Tensor, offsets: torch.Tensor, p
     _hip.check(rc, "store_tokens")
 
 
+def _kv_rows(k: torch.Tensor, v: torch.Tensor, blocks: torch.Tensor, offsets: torch.Tensor, k_pools: torch.Tensor,
+             v_pools: torch.Tensor, need_all: bool) -> None:
+    """Checks that store_layer and quantize_store_layer share: K and V rows [T, H, D], their slots (for every row, or for
+    the first ones), and pools [L, H, N, B, D]."""
+    rows, shape, n = k.shape, k_pools.shape, blocks.numel()
+    if v.shape != rows or v.dtype != k.dtype or k.stride(-1) != 1 or v.stride(-1) != 1:
+        raise ValueError("k and v must match in shape and dtype, last dim contiguous")
+    if offsets.numel() != n or n > rows[0] or need_all and n < rows[0]:
+        raise ValueError(f"{n} blocks and {offsets.numel()} offsets for {rows[0]} rows")
+    if len(shape) != 5 or shape[1] != rows[1] or shape[4] != rows[2] or v_pools.shape != shape:
+        raise ValueError(f"pools {tuple(shape)} and {tuple(v_pools.shape)} must both be [L, H={rows[1]}, N, B, D={rows[2]}]")
+
+
 def store_layer(layer: int, k: torch.Tensor, v: torch.Tensor, blocks: torch.Tensor, offsets: torch.Tensor,
                 k_pools: torch.Tensor, v_pools: torch.Tensor) -> None:
     """store_tokens(k, blocks, offsets, k_pools[layer], x2=v, pool2=v_pools[layer]) for pools [L, H, N, B, D], without
@@ -160,19 +173,15 @@ def store_layer(layer: int, k: torch.Tensor, v: torch.Tensor, blocks: torch.Tens
     n = blocks.numel()
     if n == 0:
         return
-    T, H, D = k.shape
-    _require(v.shape == k.shape and v.dtype == k.dtype and k.stride(-1) == 1 and v.stride(-1) == 1,
-             "k and v must match in shape and dtype, last dim contiguous")
-    _require(offsets.numel() == n and n <= T, lambda: f"{n} blocks but {offsets.numel()} offsets and {T} rows")
-    shape, strides = k_pools.shape, k_pools.stride()
-    _require(len(shape) == 5 and shape[1] == H and shape[4] == D and strides[4] == 1 and v_pools.shape == shape and
-             v_pools.stride() == strides and v_pools.dtype == k_pools.dtype,
-             lambda: f"pools {tuple(shape)} and {tuple(v_pools.shape)} must both be [L, H={H}, N, B, D={D}]")
+    strides = k_pools.stride()
+    _kv_rows(k, v, blocks, offsets, k_pools, v_pools, False)
+    _require(strides[4] == 1 and v_pools.stride()[1:] == strides[1:] and v_pools.dtype == k_pools.dtype,
+             "the pools must match in strides and dtype, last dim contiguous")
     _hip.require_gpu(k, v, blocks, offsets, k_pools, v_pools)
     blocks, offsets = _i64(blocks), _i64(offsets)
     (kt, kh, _), (vt, vh, _) = k.stride(), v.stride()
     rc = _hip.lib().sipa_store_tokens(
-        k.data_ptr(), v.data_ptr(), _hip.dtype_code(k.dtype), kt, kh, vt, vh, None, n, H, D, blocks.data_ptr(),
+        k.data_ptr(), v.data_ptr(), _hip.dtype_code(k.dtype), kt, kh, vt, vh, None, n, *k.shape[1:], blocks.data_ptr(),
         offsets.data_ptr(), _hip.layer_ptr(k_pools, layer), _hip.layer_ptr(v_pools, layer),
         _hip.dtype_code(k_pools.dtype), strides[1], strides[2], strides[3], _hip.stream_of(k))
     if rc:
@@ -187,18 +196,16 @@ def quantize_store_layer(layer: int, k: torch.Tensor, v: torch.Tensor, blocks: t
     T, H, D = k.shape
     if T == 0:
         return
-    _require(v.shape == k.shape and v.dtype == k.dtype and k.stride(-1) == 1 and v.stride(-1) == 1,
-             "k and v must match in shape and dtype, last dim contiguous")
-    _require(blocks.numel() == T and offsets.numel() == T, lambda: f"{T} tokens need {T} blocks and offsets")
+    _kv_rows(k, v, blocks, offsets, k_pools, v_pools, True)
     shape = k_pools.shape
-    _require(len(shape) == 5 and shape[1] == H and shape[4] == D and v_pools.shape == shape,
-             lambda: f"pools {tuple(shape)} and {tuple(v_pools.shape)} must both be [L, H={H}, N, B, D={D}]")
-    _require(k_scales.shape == shape[:4] and v_scales.shape == shape[:4],
-             lambda: f"scales must be [L, H, N, B] = {tuple(shape[:4])}")
-    _require(k_pools.dtype == torch.int8 and v_pools.dtype == torch.int8 and k_scales.dtype == torch.float16 and
-             v_scales.dtype == torch.float16, "pools must be int8 and scales fp16")
-    _require(k_pools.is_contiguous() and v_pools.is_contiguous() and k_scales.is_contiguous() and
-             v_scales.is_contiguous(), "the pools must be contiguous")
+    if k_scales.shape != shape[:4] or v_scales.shape != shape[:4]:
+        raise ValueError(f"scales must be [L, H, N, B] = {tuple(shape[:4])}")
+    if k_pools.dtype is not torch.int8 or v_pools.dtype is not torch.int8 or \
+            k_scales.dtype is not torch.float16 or v_scales.dtype is not torch.float16:
+        raise ValueError("pools must be int8 and scales fp16")
+    for t in (k_pools, v_pools, k_scales, v_scales):
+        if not (t.is_contiguous() or _hip.layers_contiguous(t)):
+            raise ValueError("the pools must be contiguous")
     _hip.require_gpu(k, v, blocks, offsets, k_pools, v_pools, k_scales, v_scales)
     blocks, offsets = _i64(blocks), _i64(offsets)
     (kt, kh, _), (vt, vh, _) = k.stride(), v.stride()

@@ -15,6 +15,7 @@ import torch
 
 from cases import assert_decode_close, fragmented_manager
 from engine.config import ModelConfig
+from engine.model import Qwen2Model
 from engine.paged_cache import PagedKVCache, build_metadata
 from engine.quant_cache import QuantPagedKVCache
 from oracle import paged_ref
@@ -227,3 +228,37 @@ def test_decode_rows_of_any_layout_in_a_mixed_forward(form, dtype):
     cache.begin(7, meta)
     print(f"case layout {form} {dtype}", flush=True)
     assert torch.equal(cache.attend(0, other, meta.positions, 0.125), ref)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "int8", "int8-kchannel"])
+def test_layers_of_a_pool_may_lie_apart(fmt):
+    """K and V of a layer side by side (each layer contiguous, the stack of them not): every layer is written and read as
+    in pools of their own, by a layer's call and by write and attend."""
+    cfg = ModelConfig(vocab_size=64, hidden_size=896, intermediate_size=256, num_layers=3, num_q_heads=14, num_kv_heads=2,
+                      head_dim=64)
+    model = Qwen2Model(cfg, "cuda", torch.bfloat16, seed=1, max_positions=256)
+    outs = []
+    for apart in (False, True):
+        m = fragmented_manager(64, 16, torch.Generator().manual_seed(1))
+        for s, n in enumerate((40, 70, 9, 100)):
+            m.allocate(s, n)
+        if fmt == "bf16":
+            cache = PagedKVCache(cfg, 64, 16, "cuda", torch.bfloat16, attn_backend="hip")
+        else:
+            cache = QuantPagedKVCache(cfg, 64, 16, "cuda", torch.bfloat16, "hip", fmt, m, n_stage=32)
+        names = ["k", "v"] + (["k_scale", "v_scale"] if fmt == "int8" else [])
+        for i, name in enumerate(names):
+            pool = getattr(cache, name)
+            pool.zero_()
+            if apart:
+                wide = torch.zeros(pool.shape[0], 2, *pool.shape[1:], device="cuda", dtype=pool.dtype)
+                setattr(cache, name, wide[:, i % 2])
+                assert not getattr(cache, name).is_contiguous()
+        batches = [[(0, 0, 39), (1, 0, 69), (2, 0, 4), (3, 0, 99)], [(0, 39, 1), (1, 69, 1), (2, 4, 5), (3, 99, 1)]]
+        for batch in batches:
+            meta = build_metadata(m, batch, "cuda")
+            ids = torch.arange(meta.num_tokens, device="cuda") % 64
+            outs.append(model.forward(ids, meta.positions, cache, meta, last_only=False))
+        outs.append(cache.k.clone())
+    for a, b in zip(outs[:3], outs[3:]):
+        assert torch.equal(a, b)

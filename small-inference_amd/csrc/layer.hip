@@ -664,9 +664,13 @@ static int check_linear(const sipa_linear_params* p) {
 
 static LinearPlan plan_of(const sipa_linear_params* p) {
   const int tiles = p->out_features / 16;  // SILU: 8 gate and 8 up rows each
-  const int cus = sipa_device_cu_count(-1);
+  // of the first device asked for (a process's GPUs are alike; a layer's call plans eight times); 256 without one
+  static const int cus = [] {
+    const int n = sipa_device_cu_count(-1);
+    return n > 0 ? n : 256;
+  }();
   return plan_linear(p->epilogue, p->norm_weight != nullptr, p->num_tokens, tiles, p->in_features, p->num_splits,
-                     p->tile, cus > 0 ? cus : 256);
+                     p->tile, cus);
 }
 
 extern "C" int64_t sipa_linear_scratch_bytes(const sipa_linear_params* p) {

@@ -32,14 +32,18 @@ MAX_GATED_FLOPS = 15e9
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
-def _ok(t, device: int, *shape: int) -> bool:
-    return type(t) in _PLAIN and t.dtype is torch.bfloat16 and t.get_device() == device and t.shape == shape and \
-        t.is_contiguous() and t.data_ptr() % 16 == 0
+def _ok(device: int, *wanted: tuple[torch.Tensor, tuple[int, ...]]) -> bool:
+    """Whether every (tensor, shape) is a contiguous bf16 tensor of that shape on the device, 16-byte aligned."""
+    for t, shape in wanted:
+        if type(t) not in _PLAIN or t.dtype is not torch.bfloat16 or t.get_device() != device or t.shape != shape or \
+                not t.is_contiguous() or t.data_ptr() % 16:
+            return False
+    return True
 
 
 # looked up once: a layer asks them all for every call
 _inference, _autocast, _compiling = torch.is_inference_mode_enabled, torch.is_autocast_enabled, torch.compiler.is_compiling
-_tracing, _transform = torch._C._get_tracing_state, torch._C._functorch.peek_interpreter_stack
+_tracing, _transform = torch._C._is_tracing, torch._C._functorch.peek_interpreter_stack
 _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
 
 
@@ -48,7 +52,7 @@ def _plain() -> bool:
     saved-tensor hooks do not reach them there), not under autocast, whose type the products' results have, and with
     nobody between who is to see each operation: vmap, grad or jvp, tracing or compilation, a dispatch mode, or a function
     mode other than the default device's."""
-    if not _inference() or _autocast() or _compiling() or _tracing() is not None or _transform() is not None or \
+    if not _inference() or _autocast() or _compiling() or _tracing() or _transform() is not None or \
             _dispatch_modes():
         return False
     n = _function_modes()
@@ -60,8 +64,7 @@ def rows_ok(x: torch.Tensor, norm_weight: torch.Tensor) -> bool:
     if not (x.is_cuda and x.dim() == 2 and _plain()):
         return False
     T, K = x.shape
-    dev = x.get_device()
-    return K % 8 == 0 and K <= 8192 and _ok(x, dev, T, K) and _ok(norm_weight, dev, K)
+    return K % 8 == 0 and K <= 8192 and _ok(x.get_device(), (x, (T, K)), (norm_weight, (K,)))
 
 
 def supported(x: torch.Tensor, w, rot, heads: int, head_dim: int) -> bool:
@@ -76,9 +79,9 @@ def supported(x: torch.Tensor, w, rot, heads: int, head_dim: int) -> bool:
     if max(width, inter, attn) > 1 << 20 or T * max(width, inter) >= 1 << 34:  # the library's limits
         return False
     return (head_dim % 16 == 0 and hidden % 64 == 0 and inter % 64 == 0 and attn % 64 == 0 and
-            _ok(w.qkv_w, dev, width, hidden) and _ok(w.qkv_b, dev, width) and _ok(w.o_w, dev, hidden, attn) and
-            _ok(w.post_norm, dev, hidden) and _ok(w.gate_up_w, dev, 2 * inter, hidden) and
-            _ok(w.down_w, dev, hidden, inter) and _ok(cos, dev, T, 1, head_dim) and _ok(sin, dev, T, 1, head_dim))
+            _ok(dev, (w.qkv_w, (width, hidden)), (w.qkv_b, (width,)), (w.o_w, (hidden, attn)), (w.post_norm, (hidden,)),
+                (w.gate_up_w, (2 * inter, hidden)), (w.down_w, (hidden, inter)), (cos, (T, 1, head_dim)),
+                (sin, (T, 1, head_dim))))
 
 
 def attention_ok(attn: torch.Tensor, x: torch.Tensor, w) -> bool:
@@ -126,9 +129,9 @@ def fused_linear(x: torch.Tensor, weight: torch.Tensor, epilogue: int, *, norm_w
                           x.data_ptr(), x.stride(0), weight.data_ptr(), _hip.ptr(norm_weight), _hip.ptr(bias),
                           _hip.ptr(residual), residual.stride(0) if residual is not None else 0, out.data_ptr(),
                           out.stride(0), *((rot[0].data_ptr(), rot[1].data_ptr()) if rot is not None else (None, None)),
-                          num_splits, tile, _hip.ptr(scratch), n, _hip.ptr(counters),
-                          *(store or (0, None, None, 0, 0, 0, None, None)), _hip.ptr(clear),
-                          clear.numel() if clear is not None else 0)
+                          num_splits, tile, _hip.ptr(scratch), n, _hip.ptr(counters), *(store or ()))
+    if clear is not None:
+        p.clear, p.clear_count = clear.data_ptr(), clear.numel()
     _hip.check(_hip.lib().sipa_fused_linear(ctypes.byref(p), stream), "fused_linear")
     return out
 

@@ -650,7 +650,7 @@ def test_layer_sizes_past_the_librarys_limits_keep_the_torch_operations(monkeypa
     from engine.model import Layer
 
     monkeypatch.setattr(hip_layer, "rows_ok", lambda x, w: True)
-    monkeypatch.setattr(hip_layer, "_ok", lambda t, device, *shape: tuple(t.shape) == shape)
+    monkeypatch.setattr(hip_layer, "_ok", lambda device, *wanted: all(tuple(t.shape) == shape for t, shape in wanted))
 
     def supported(T, inter):
         z = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device="meta")  # noqa: E731

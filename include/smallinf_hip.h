@@ -301,7 +301,8 @@ int64_t sipa_prefill_workspace_bytes(int32_t num_seqs, int32_t num_q_heads, int3
  * work starts first and consecutive workgroups spread over the XCDs. Pieces are at least 512 tokens (a small
  * batch's long sequence is not cut into more merges than its streaming saves), or 256 when max_piece <= 4096:
  * the INT8 kernels, two workgroups per CU, do better with the shorter pieces. max_piece aside, the longest sequence
- * is cut into 32 pieces at most.
+ * is cut into 32 pieces at most, or for max_piece > 4096 into as many as keep each within one and a half times a CU's
+ * share of all tokens.
  * context_lens_host [num_seqs] (each >= 1) are the lengths the decode call will read. Writes at most capacity
  * items (8 int32 each) to items_out and the largest split count of a pair to *max_splits; returns the number of
  * items, or a negative SIPA_E* code (items_out may be NULL to ask for the count).

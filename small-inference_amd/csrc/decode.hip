@@ -763,9 +763,14 @@ extern "C" int32_t sipa_build_work_list(const int32_t* ctx, int32_t S, int32_t H
   // their 4096-token cap (their small batches: 10.5 us at 256 against 12.1 at 512).
   int64_t min_piece = (max_piece > 0 && max_piece <= kMaxInt8Split) ? kMinChunk : kLatencyChunk;
   // and at most kMaxPairPieces pieces of the longest sequence, two rounds of its merge (14 INT8 sequences of up to 16384
-  // tokens: 52 pieces of 320 30.4 us, 32 of 512 21.4)
+  // tokens: 52 pieces of 320 30.4 us, 32 of 512 21.4), but over bf16 pools no piece beyond one and a half times a CU's share
+  // of the tokens, so that one long sequence among short ones does not leave CUs idle (32 pieces, and with that limit:
+  // 65536 tokens and 7 x 500 21.1 and 16.4 us, 1.5B 35.4 and 24.3; 131072 and 7 x 500 36.4 and 24.1, 63.1 and 36.3; 24000 and
+  // 20 x 2000 12.5 and 12.1. At 1.25 the last took 14.0. INT8, 16384 and 7 x 500: 10.8 and 12.4, not there).
   const int longest = S > 0 ? *std::max_element(ctx, ctx + S) : 0;
-  min_piece = std::min(cap, std::max<int64_t>(min_piece, ceil_div(longest, kMaxPairPieces)));
+  int64_t fewest = ceil_div(longest, kMaxPairPieces);
+  if (min_piece == kLatencyChunk) fewest = std::min(fewest, 3 * total / (2 * (int64_t)cu_count));
+  min_piece = std::min(cap, std::max(min_piece, fewest));
   piece = std::max(piece, min_piece);
   piece = std::min<int64_t>((piece + kChunkAlign - 1) / kChunkAlign * kChunkAlign, cap / kChunkAlign * kChunkAlign);
   struct Item {

@@ -76,7 +76,7 @@ def build_work_list(context_lens: list[int], num_kv_heads: int, cu_count: int | 
     """Work list for a ragged batch from host-side context lengths: ([n, 8] int32 items, largest split count of
     a pair). Each (sequence, KV head) pair is cut into near-equal pieces of about sum(ctx) * Hkv /
     (cu_count * items_per_cu) tokens (at most max_piece; 0: 32768; max_piece aside, at most 32 a
-    pair); items are ordered longest first. Three items
+    pair, or over bf16 pools as many as keep each within 1.5 times a CU's share); items are ordered longest first. Three items
     per CU measured best on MI355X (C3 ragged 256: 30.4 -> 29.4 us against two; 512 x U[1024, 16384]: 390 -> 382 us;
     four to six were no better)."""
     cu = device_cu_count() if cu_count is None else cu_count

@@ -172,6 +172,15 @@ def test_work_list_caps_the_pieces_of_a_pair(longest):
     assert len(first) == maxs and sum(i[5] - i[4] for i in first) == longest
 
 
+@pytest.mark.parametrize("lens", [[65536] + [500] * 7, [131072] + [500] * 7, [100_000] + [1000] * 100, [30000, 2]])
+def test_work_list_spreads_a_long_sequence_over_the_cus(lens):
+    """bf16 pools: no piece longer than one and a half times a CU's share of all tokens (rounded up to 64), however many
+    pieces that makes of one sequence; 512 tokens at least."""
+    items, _ = work_list(lens, 2, max_piece=0)
+    share = 3 * sum(lens) * 2 // (2 * 256)
+    assert max(i[5] - i[4] for i in items) <= max(512, -(-share // 64) * 64)
+
+
 def test_work_list_piece_size_and_errors():
     """Pieces are about total / (cu * items_per_cu) tokens, at least 256; bad lengths and short buffers fail."""
     items, maxs = work_list([8192] * 32, 2, cu=256, per_cu=2)  # 524288 token-heads / 512 -> 1024-token pieces

@@ -256,11 +256,12 @@ typedef struct sipa_prefill_params {
      them through memory (agent-coherent loads). Both give the same bits. */
   int32_t merge_path;
   /* Workgroup layout (ABI 6), a SIPA_PREFILL_* value. A column tile is a query head and 16 of a unit's tokens.
-     SIPA_PREFILL_AUTO lets the library choose from g8, the grid of 8-column workgroups: SIPA_PREFILL_W8X1 for
-     g8 <= CUs; for a chunk at least its own length into its context, SIPA_PREFILL_W16H2 over bf16 pools with 8
-     or more key splits of at most 1024 keys, else SIPA_PREFILL_W16X1 with one split or splits of at least 1024
-     keys, else W8X1; for fresh prompts W8X1 up to 3 workgroups per CU, then W16X1, except SIPA_PREFILL_W4X2
-     beyond 4 per CU at head_dim 64. Format B pools (SIPA_KV_INT8_KCHAN) take W4X2 (W4X2 or W8X1 when forced). W4X2 and
+     SIPA_PREFILL_AUTO lets the library choose from g8, the grid of 8-column workgroups: for g8 <= CUs
+     SIPA_PREFILL_W8X1, or SIPA_PREFILL_W16H2 past 16 key splits; for a chunk at least its own length into its context,
+     W16H2 with 8 or more key splits of at most 1024 keys (bf16 pools, or head_dim 128), else SIPA_PREFILL_W16X1 with
+     one split or splits of at least 1024 keys, else W8X1; for fresh prompts W8X1 up to 3 workgroups per CU, then W16X1.
+     Format B pools (SIPA_KV_INT8_KCHAN) take W8X1 up to 1.5 workgroups per CU and SIPA_PREFILL_W4X2 above (and no
+     other layout when forced); over the other pools W4X2 runs only when asked for. W4X2 and
      W8X1 give the same bits; W16X1 too with one split (with several, a row may go through the split merge's
      fp16 partials in one layout and not in the other); W16H2 combines key splits in its own order. Every
      layout meets the same error bound. With W16H2, num_splits counts key chunks, two to a workgroup. */
@@ -279,11 +280,11 @@ enum {
 
 int32_t sipa_prefill(const sipa_prefill_params* p, void* stream);
 
-/* Key splits for a prefill call (no counterpart in the reference, whose gather path has no grid): one up to
- * 448 keys of context (511 at head_dim 128); about two workgroups per CU over the call's 8-column units from 4096 keys (from 2048 where not even two
- * splits fit one workgroup per CU); between, at most one workgroup per CU and 8 splits. At least 256 keys per split
- * and at most 32 splits. query_tiles = sum over sequences of ceil(query_len / 16). cu_count <= 0 asks the current
- * device. */
+/* Key splits for a prefill call (no counterpart in the reference, whose gather path has no grid): one up to 448 keys of
+ * context (511 at head_dim 128); about two workgroups per CU over the call's 8-column units from 4096 keys (from 2048
+ * where not even two splits fit one workgroup per CU); between, at most one workgroup per CU and 8 splits. At least 256
+ * keys per split and at most 32 splits. query_tiles = sum over sequences of ceil(query_len / 16). cu_count <= 0 asks the
+ * current device. */
 int32_t sipa_prefill_splits(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t query_tiles,
                             int32_t max_context, int32_t cu_count);
 

@@ -8,8 +8,9 @@ several CUs) and, for small batches, not so short that the merge's round trips o
 (the library's sipa_choose_splits_for). A split past a sequence's end does no work; the last split workgroup of a
 (sequence, KV head) to finish merges the partials (combine="fused"), or a second kernel does (combine="kernel").
 
-Kernels: bf16 queries with 16-token blocks and head_dim 64/128 run the MFMA kernels (bf16 pools, and both INT8
-formats with fp16 or constant scales); everything else (fp32 models, other block sizes or head dims) runs the
+Kernels: bf16 queries with head_dim 64/128 run the MFMA kernels over blocks of 16 tokens (bf16 pools, and both INT8
+formats with fp16 or constant scales) and of 32 or 64 (bf16 pools and the per-token INT8 format, with fp32 probabilities
+and their sums as the VALU kernel forms them); everything else (fp32 models, other block sizes or head dims) runs the
 VALU kernel. impl="valu" / "mfma" forces one.
 """
 

@@ -346,6 +346,7 @@ def bad_linear(**over):
     (dict(epilogue=1, rot_channels=1024, kv_heads=2), _hip.EINVAL),  # no pools
     (dict(epilogue=1, rot_channels=1024, kv_heads=2, k_pool=4096, v_pool=4096, kv_blocks=4096, kv_offsets=4096,
           kv_stride_b=66), _hip.EUNSUPPORTED),
+    (dict(clear_count=4), _hip.EINVAL), (dict(clear=4096, clear_count=-1), _hip.EINVAL),
     (dict(num_tokens=-1), _hip.EINVAL)])
 def test_fused_linear_refuses_bad_arguments(over, code):
     assert _hip.lib().sipa_fused_linear(ctypes.byref(bad_linear(**over)), None) == code

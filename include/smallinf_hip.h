@@ -258,8 +258,9 @@ typedef struct sipa_prefill_params {
   /* Workgroup layout (ABI 6), a SIPA_PREFILL_* value. A column tile is a query head and 16 of a unit's tokens.
      SIPA_PREFILL_AUTO lets the library choose from g8, the grid of 8-column workgroups: for g8 <= CUs
      SIPA_PREFILL_W8X1, or SIPA_PREFILL_W16H2 past 16 key splits; for a chunk at least its own length into its context,
-     W16H2 with 8 or more key splits of at most 1024 keys (bf16 pools, or head_dim 128), else SIPA_PREFILL_W16X1 with
-     one split or splits of at least 1024 keys, else W8X1; for fresh prompts W8X1 up to 3 workgroups per CU, then W16X1.
+     W16H2 with 8 or more key splits of at most 1024 keys (bf16 pools, or head_dim 128; there also with 6 or 7 where its
+     grid is at most the CUs), else SIPA_PREFILL_W16X1 with one split or splits of at least 1024 keys, else W8X1; for
+     fresh prompts W8X1 up to 3 workgroups per CU, then W16X1.
      Format B pools (SIPA_KV_INT8_KCHAN) take W8X1 up to 1.5 workgroups per CU and SIPA_PREFILL_W4X2 above (and no
      other layout when forced); over the other pools W4X2 runs only when asked for. W4X2 and
      W8X1 give the same bits; W16X1 too with one split (with several, a row may go through the split merge's

@@ -891,7 +891,10 @@ extern "C" int32_t sipa_prefill(const sipa_prefill_params* p, void* stream) {
   //    . 8 or more key chunks of at most 1024 keys, bf16 pools or head_dim 128: 16 waves over 8 column tiles and two
   //      consecutive key chunks, combined in the workgroup, so that half as many splits store partials and merge: 512
   //      new tokens at 8K 30.8 (best of the others) -> 28.6, at head_dim 128 241 at 6.8K over INT8 41.5 -> 35.7. (INT8 at
-  //      head_dim 64 keeps W16X1: each half dequantizes its own tiles, 512 at 8K 32.4 -> 34.8.)
+  //      head_dim 64 keeps W16X1: each half dequantizes its own tiles, 512 at 8K 32.4 -> 34.8.) At head_dim 128 also 6
+  //      and 7 chunks where its halved grid fits one workgroup per CU: 71 shapes, 0.70 to 0.96 of W8X1's time (two
+  //      178-token chunks at 4.0K 37.3 -> 30.0, INT8 373 at 3.0K 40.9 -> 29.4). Not 5 (six chunks up to 88 at 1.5K 27.1
+  //      on W8X1, 32.4) and not more workgroups (six up to 137 at 4.1K, 352, 44.1 on W8X1, 55.9).
   //    . otherwise, with one chunk or chunks of at least 1024 keys: 16-wave workgroups of 16 column tiles, one per
   //      CU at a time. Two co-resident 8-column workgroups do not share a CU evenly (the later-dispatched ran ~30%
   //      longer and finished alone), and 16 column tiles share each K/V tile load: two 677-token chunks at 3K 29.2 ->
@@ -909,9 +912,11 @@ extern "C" int32_t sipa_prefill(const sipa_prefill_params* p, void* stream) {
     if (mode == SIPA_KV_INT8_KCHAN) layout = 2 * g8 <= 3LL * cus ? SIPA_PREFILL_W8X1 : SIPA_PREFILL_W4X2;
     else if (g8 <= cus) layout = nchunk > 16 ? SIPA_PREFILL_W16H2 : SIPA_PREFILL_W8X1;
     else if (balanced)
-      layout = (mode == SIPA_KV_PLAIN || D == 128) && nchunk >= 8 && chunk <= 1024 ? SIPA_PREFILL_W16H2
-               : nchunk == 1 || chunk >= 1024                                    ? SIPA_PREFILL_W16X1
-                                                                                 : SIPA_PREFILL_W8X1;
+      layout = chunk <= 1024 && (nchunk >= 8 ? mode == SIPA_KV_PLAIN || D == 128
+                                             : D == 128 && nchunk >= 6 && grid_of(units8, 2) <= cus)
+                   ? SIPA_PREFILL_W16H2
+               : nchunk == 1 || chunk >= 1024 ? SIPA_PREFILL_W16X1
+                                              : SIPA_PREFILL_W8X1;
     else layout = g8 <= 3LL * cus ? SIPA_PREFILL_W8X1 : SIPA_PREFILL_W16X1;
   }
   SIPA_CHECK(mode != SIPA_KV_INT8_KCHAN || layout == SIPA_PREFILL_W4X2 || layout == SIPA_PREFILL_W8X1,

@@ -487,6 +487,39 @@ def test_wave_layouts_agree(shape, pool, splits):
                 run(lay)
 
 
+@pytest.mark.parametrize("pool", ["bf16", "int8"])
+@pytest.mark.parametrize("n,new,ctx,splits,layout", [(4, 107, 3198, 6, "w16h2"), (2, 183, 3768, 7, "w16h2"),
+                                                     (3, 171, 1644, 5, "w8x1"), (6, 137, 4103, 7, "w8x1")])
+def test_few_key_chunks_take_two_a_workgroup(pool, n, new, ctx, splits, layout):
+    """At head_dim 128 and 256 CUs, calls of more than one 8-column workgroup per CU: 6 and 7 key chunks whose grid of two
+    chunks a workgroup fits the CUs run the two-chunk layout; 5 chunks, and 7 whose halved grid does not fit, do not.
+    Each is its forced layout's bits, the other layout's within the rounding of the output and of the fp16 partials,
+    and over bf16 pools the oracle's."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes are chosen for 256 CUs")
+    Hq, Hkv, D = SHAPES["1.5B"]
+    ctxs, qlen = [ctx] * n, [new] * n
+    print(f"case few key chunks {n} x {new} at {ctx} {pool}", flush=True)
+    q, k, v, bt, c, st, ln, tables, starts, T = make_prefill(ctxs, qlen, Hq, Hkv, D, seed=ctx)
+    quant = None
+    if pool != "bf16":
+        g = torch.Generator(device="cuda").manual_seed(7)
+        quant, k, v, _, _ = int8_pools(k, v, pool, ctxs, tables, g)
+    run = lambda lay: paged_prefill_attention(q, k, v, bt, c, st, ln, D ** -0.5, ctx, new,  # noqa: E731
+                                              num_splits=splits, quant=quant, wg_layout=lay)
+    got, forced = run("auto"), {lay: run(lay) for lay in ("w8x1", "w16h2")}
+    torch.cuda.synchronize()
+    assert not torch.equal(forced["w8x1"], forced["w16h2"])  # or the next line could not tell them apart
+    assert torch.equal(got, forced[layout])
+    a, b = forced["w8x1"].float(), forced["w16h2"].float()
+    assert ((a - b).abs() <= 2 ** -7 * torch.maximum(a.abs(), b.abs()) + 2 ** -9).all()
+    if quant is None:
+        ref32 = paged_ref.prefill(as_np32(q), as_np32(k), as_np32(v), tables, ctxs, starts, qlen, D ** -0.5,
+                                  dtype=np.float32)
+        rows = np.concatenate([np.arange(s, s + m) for s, m in zip(starts, qlen)])
+        assert_bf16_close(got.double().cpu().numpy()[rows], ref32[rows], "few key chunks")
+
+
 @pytest.mark.parametrize("Hq,Hkv,D", [(10, 2, 64), (12, 2, 64), (14, 2, 128), (24, 8, 128), (5, 1, 64)])
 @pytest.mark.parametrize("layout", ["w4x2", "w8x1", "w16x1", "w16h2"])
 @pytest.mark.parametrize("splits", [1, 3])
